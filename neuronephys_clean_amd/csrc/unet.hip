@@ -699,8 +699,14 @@ __global__ __launch_bounds__(256) void k_wgrad(WgArgs a) {
             }
         }
         __syncthreads();
-        if (tid < COUT)
-            for (int v = 0; v < 256; ++v) bsum += bf2f(s_g[tid * kWgRows + v]);
+        // bias: every thread adds COUT of its channel's 256 voxels (16 or 32
+        // threads alone held the tile's other waves at the next barrier:
+        // 172 -> 153 us for 16 -> 16 at 8 x 64^3)
+#pragma unroll 4
+        for (int v = 0; v < COUT; v += 2) {
+            const uint32_t p = *(const uint32_t*)&s_g[(tid % COUT) * kWgRows + (tid / COUT) * COUT + v];
+            bsum += bf2f(p & 0xffffu) + bf2f(p >> 16);
+        }
         for (int ch = 0; ch < 8; ++ch) {  // 32 voxels: rows 2ch, 2ch+1 of the 16 (y,z) rows
             const int rr = 2 * ch + (g >> 1), xs0 = 8 * (g & 1);
             const int ry = rr & 3, rz = rr >> 2;
@@ -732,23 +738,58 @@ __global__ __launch_bounds__(256) void k_wgrad(WgArgs a) {
             for (int q = 0; q < 4; ++q)
                 a.part[((size_t)blockIdx.x * COUT + 16 * mt + 4 * g + q) * KP + 16 * nt + xl] = acc[j][mt][q];
     }
-    if (tid < COUT) a.bpart[blockIdx.x * COUT + tid] = bsum;
+    __syncthreads();
+    float* sb = reinterpret_cast<float*>(s_g);  // the tile's gradients are read
+    sb[tid] = bsum;
+    __syncthreads();
+    if (tid < COUT) {
+        float t = 0.f;
+#pragma unroll
+        for (int q = 0; q < 256 / COUT; ++q) t += sb[q * COUT + tid];
+        a.bpart[blockIdx.x * COUT + tid] = t;
+    }
 }
 
-// dW[co][k] (k < 27 CIN) and db[co]: partials added in workgroup order
-__global__ void k_wgrad_reduce(const float* __restrict__ part, const float* __restrict__ bpart, int nwg,
-                               int cout, int kp, int kreal, float* __restrict__ dw, float* __restrict__ db) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < cout * kreal) {
-        const int co = i / kreal, k = i - co * kreal;
-        float s = 0.f;
-        for (int w = 0; w < nwg; ++w) s += part[((size_t)w * cout + co) * kp + k];
-        dw[i] = s;
-    } else if (i < cout * kreal + cout) {
-        const int co = i - cout * kreal;
-        float s = 0.f;
-        for (int w = 0; w < nwg; ++w) s += bpart[w * cout + co];
-        db[co] = s;
+// dW[co][k] (k < 27 CIN) and db[co] from the workgroups' partials: a block
+// takes 64 consecutive columns of the [co][kp] partial rows (the blocks past
+// them: the bias), wave s of 16 adds rows s, s + 16, ... of its column - four
+// loads in flight - and the 16 sums are added in order, so the order is fixed.
+// Bound by reading the partials once (512 x 27.6 KB for 16 -> 16: 14 MB);
+// one thread per column, its loads one after the other, took 125 us (231 for
+// 32 -> 32), this takes 5.4.
+constexpr int kWrSlices = 16;
+__global__ __launch_bounds__(1024) void k_wgrad_reduce(const float* __restrict__ part, const float* __restrict__ bpart,
+                                                       int nwg, int cout, int kp, int kreal, float* __restrict__ dw,
+                                                       float* __restrict__ db) {
+    __shared__ float sh[kWrSlices][64];
+    const int cols = cout * kp, nblk = (cols + 63) / 64;
+    const bool bias = (int)blockIdx.x >= nblk;
+    const float* __restrict__ src = bias ? bpart : part;
+    const int width = bias ? cout : cols;
+    const int lane = threadIdx.x & 63, slice = threadIdx.x >> 6;
+    const int col = (bias ? 0 : (int)blockIdx.x * 64) + lane;
+    float s = 0.f;
+    if (col < width) {
+        int w = slice;
+        for (; w + 3 * kWrSlices < nwg; w += 4 * kWrSlices) {
+            const float v0 = src[(size_t)w * width + col], v1 = src[(size_t)(w + kWrSlices) * width + col],
+                        v2 = src[(size_t)(w + 2 * kWrSlices) * width + col],
+                        v3 = src[(size_t)(w + 3 * kWrSlices) * width + col];
+            s = (((s + v0) + v1) + v2) + v3;
+        }
+        for (; w < nwg; w += kWrSlices) s += src[(size_t)w * width + col];
+    }
+    sh[slice][lane] = s;
+    __syncthreads();
+    if (slice || col >= width) return;
+    float t = sh[0][lane];
+#pragma unroll
+    for (int q = 1; q < kWrSlices; ++q) t += sh[q][lane];
+    if (bias) {
+        db[col] = t;
+    } else {
+        const int co = col / kp, k = col - co * kp;
+        if (k < kreal) dw[(size_t)co * kreal + k] = t;
     }
 }
 
@@ -1135,18 +1176,21 @@ __global__ __launch_bounds__(256) void k_head_bwd(const float* __restrict__ dzv,
         part[blockIdx.x * 17 + q] = ((sh[0][q] + sh[1][q]) + sh[2][q]) + sh[3][q];
     }
 }
-// head gradients (dhw[16], dhb) into grad[], the loss into loss[0]
-__global__ void k_head_fin(const double* __restrict__ part, const double* __restrict__ lpart, int nblk,
-                           float* __restrict__ ghead, double* loss, int batch) {
-    const int q = threadIdx.x;
-    if (q < 17) {
+// head gradients (dhw[16], dhb) into grad[], the loss into loss[0]: a
+// wavefront per quantity, lanes over the partials, one butterfly: 6.5 us
+// (latency) where one thread's serial sum of 512 doubles took 153
+__global__ __launch_bounds__(1024) void k_head_fin(const double* __restrict__ part, const double* __restrict__ lpart,
+                                                   int nblk, float* __restrict__ ghead, double* loss, int batch) {
+    const int lane = threadIdx.x & 63;
+    for (int q = threadIdx.x >> 6; q < 18; q += 16) {
         double s = 0;
-        for (int i = 0; i < nblk; ++i) s += part[i * 17 + q];
-        ghead[q] = (float)s;
-    } else if (q == 17) {
-        double s = 0;
-        for (int i = 0; i < nblk; ++i) s += lpart[i];
-        *loss = s / batch;
+        for (int i = lane; i < nblk; i += 64) s += q < 17 ? part[i * 17 + q] : lpart[i];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        if (lane == 0) {
+            if (q < 17) ghead[q] = (float)s;
+            else *loss = s / batch;
+        }
     }
 }
 
@@ -1309,9 +1353,8 @@ nnx_status launch_wgrad(nnx_ctx* c, WgArgs a, float* dw, float* db) {
     a.part = (float*)part;
     a.bpart = (float*)bpart;
     k_wgrad<CIN, COUT><<<nwg, 256, 0, c->stream>>>(a);
-    const int tot = COUT * 27 * CIN + COUT;
-    k_wgrad_reduce<<<ceil_div(tot, 256), 256, 0, c->stream>>>(a.part, a.bpart, nwg, COUT, kpad(CIN), 27 * CIN,
-                                                                 dw, db);
+    k_wgrad_reduce<<<ceil_div(COUT * kpad(CIN), 64) + 1, 64 * kWrSlices, 0, c->stream>>>(
+        a.part, a.bpart, nwg, COUT, kpad(CIN), 27 * CIN, dw, db);
     NNX_LAUNCHED(c);
     return NNX_OK;
 }
@@ -1643,7 +1686,7 @@ nnx_status nnx_unet_train_step(nnx_ctx* c, nnx_unet* u, int nx, int ny, int nz, 
         dzn = (float*)dzcp;
     }
     k_head_bwd<<<kHeadBlocks, 256, 0, c->stream>>>(dzn, n0, A.d0, u->p + P.head_off, G0, A.part);
-    k_head_fin<<<1, 64, 0, c->stream>>>(A.part, (const double*)lpart, kHeadBlocks, u->grad + P.head_off,
+    k_head_fin<<<1, 1024, 0, c->stream>>>(A.part, (const double*)lpart, kHeadBlocks, u->grad + P.head_off,
                                         (double*)lossp, batch);
     NNX_LAUNCHED(c);
     const int nx1 = mx / 2, ny1 = my / 2, nz1 = mz / 2, nx2 = mx / 4, ny2 = my / 4, nz2 = mz / 4;
