@@ -13,6 +13,7 @@ namespace nnx {
 struct GridK {
     int32_t nx, ny, nz, kind;  // kind: 0 const 7-pt, 1 variable 7-pt, 2 27-pt
     int32_t block;             // kind 0: Dirichlet faces every `block` voxels (0: none)
+    int32_t nxr;               // voxels of a row that belong to the grid (< nx: padded rows)
     float c, diag, a0, w;      // fp32 constants (cast once on the host)
     double cd, diagd, a0d, wd; // fp64 constants
     const float *kx, *ky, *kz;
@@ -25,6 +26,7 @@ inline GridK make_grid(const nnx_grid* g) {
     k.nz = g->nz;
     k.kind = g->stencil == NNX_STENCIL_27 ? 2 : (g->kx ? 1 : 0);
     k.block = g->block;
+    k.nxr = g->nx;
     k.cd = g->c;
     k.diagd = 1.0 + 6.0 * g->c;
     k.a0d = 1.0 + 0.5 * g->decay_dt;

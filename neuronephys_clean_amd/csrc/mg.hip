@@ -279,7 +279,7 @@ nnx_status mg_setup(nnx_ctx* c, const GridK& g0, int nu, int smoother, int gamma
         if ((f.nx & 1) || (f.ny & 1) || (f.nz & 1) || std::min(f.nx, std::min(f.ny, f.nz)) < 8) break;
         GridK& g = m->g[l + 1];
         g = f;
-        g.nx = f.nx / 2, g.ny = f.ny / 2, g.nz = f.nz / 2;
+        g.nx = g.nxr = f.nx / 2, g.ny = f.ny / 2, g.nz = f.nz / 2;
         const int64_t nfx = (int64_t)(g.nx + 1) * g.ny * g.nz, nfy = (int64_t)g.nx * (g.ny + 1) * g.nz,
                       nfz = (int64_t)g.nx * g.ny * (g.nz + 1);
         char name[32];

@@ -226,12 +226,12 @@ __global__ __launch_bounds__(256) void k_cg_status(CgDev d) {
 }
 
 // Constant 7-point stencil, 2.5D LDS tiling with four voxels per thread.
-// A block of 64 TY threads owns a 256 (x) x TY (y) tile (TY 16, or 8 and 4
-// where that measured faster) and marches kZ4 planes in z; thread (lx, ly)
-// holds x = 4lx .. 4lx+3 of row ly as a float4.  Each
-// plane (plus its one-voxel halo in x and y) goes into a double-buffered LDS
-// tile; the column's z neighbours stay in registers; the next plane's loads
-// are issued before the plane's barrier (a barrier drains outstanding loads,
+// A block of 64 TY threads owns a tile of 4 LX (x) x 64 TY / LX (y) voxels
+// (256 x TY for LX 64; TY 16, or 8 and 4 where that measured faster) and
+// marches kZ4 planes in z (DYN: zdyn of them); thread (lx, ly) holds x = 4lx ..
+// 4lx+3 of row ly as a float4.  tile_shape has the choice.  Each plane (plus
+// its one-voxel halo in x and y) goes into a double-buffered LDS tile; the
+// column's z neighbours stay in registers; the next plane's loads are issued before the plane's barrier (a barrier drains outstanding loads,
 // so 16-byte loads per thread are what keeps enough bytes in flight).
 // Requires nx % 4 == 0 (16-byte aligned rows).
 //   MODE 0: y = A src (summation order of the CPU restatement); dst = y.
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(256) void k_cg_status(CgDev d) {
 constexpr int kTX4 = 256, kTY4 = 16, kZ4 = 16, kT4 = 64 * kTY4, kRow4 = kTX4 + 8;
 // prefetch forms and tile heights the solver launches (measured at 256^3):
 // the apply and the variable-coefficient first half take the deferred form;
-// the constant-coefficient iteration stays at PF 2 (the deferred form for
+// the constant-coefficient iteration on 1024-thread tiles stays at PF 2 (the deferred form for
 // its second half or for both halves: 98.1-98.5 us per iteration against
 // 96.3-96.6), its first half on 16-row tiles and its second half on 4-row
 // tiles, four 256-thread workgroups per CU (94.4-94.5 us per iteration
@@ -276,14 +276,18 @@ __device__ __forceinline__ int xcd_tile(int b, int round, int nb) {
     const int t = nb % 8 == 0 ? (b % 8) * (nb / 8) + b / 8 : b;
     return t + round * nb;
 }
-template <int MODE, int PF, bool VAR = false, int TY = kTY4, bool BLK = false>
+template <int MODE, int PF, bool VAR = false, int TY = kTY4, bool BLK = false, int LX = 64, bool DYN = false>
 __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k, const float* __restrict__ src,
                                                     const float* __restrict__ pold, float* __restrict__ pnew,
-                                                    float* __restrict__ dst, int xzero) {
+                                                    float* __restrict__ dst, int xzero, int zdyn) {
+    constexpr int R = 64 * TY / LX;            // rows of the tile
+    constexpr int kTXs = 4 * LX, kRowS = kTXs + 8;  // its width, and the LDS row
+    const int kZs = DYN ? zdyn : kZ4;          // planes it marches (DYN: even)
+    static_assert(!DYN || PF == 3, "the deferred form for a march of any length");
     static_assert(MODE == 0 || MODE == 2 || MODE == 3, "mode");
     static_assert(PF == 1 || PF == 2 || PF == 3, "prefetch form");
     static_assert(!VAR || MODE == 2, "variable coefficients: the first half only (k_cg_rupd is the second)");
-    __shared__ float t[2][TY + 2][kRow4];
+    __shared__ float t[2][R + 2][kRowS];
     float beta = 0.0f, di = 1.0f, alpha = 0.0f;
     // the scalars in one round of loads: the done flag, r.z and alpha of
     // the previous iteration (stored by block 0 of its launches) and the
@@ -330,16 +334,16 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
     const bool read_x = upd_x && !(xzero && k == 1);
     const bool use_pold = MODE == 2 && k > 0;
     const int nx = g.nx, ny = g.ny, nz = g.nz;
-    const int tx = (nx + kTX4 - 1) / kTX4, ty = (ny + TY - 1) / TY, tz = (nz + kZ4 - 1) / kZ4;
+    const int tx = (nx + kTXs - 1) / kTXs, ty = (ny + R - 1) / R, tz = (nz + kZs - 1) / kZs;
     const int ntiles = tx * ty * tz;
     const int64_t sxy = (int64_t)nx * ny;
-    const int tt = threadIdx.x, lx = tt & 63, ly = tt >> 6;
-    // halo roles: 0..63 row y=-1, 64..127 row y=TY (float4 each), the next
-    // TY threads column x=-1, the TY after them column x=kTX4 (one voxel each)
-    const bool hrow = tt < 128, hcol = tt >= 128 && tt < 128 + 2 * TY;
-    const int hy = tt < 64 ? -1 : tt < 128 ? TY : (tt < 128 + TY ? tt - 128 : tt - 128 - TY);
-    const int hl = tt < 64 ? tt : tt - 64;
-    const int hslot = tt < 128 + TY ? 3 : 4 + kTX4;
+    const int tt = threadIdx.x, lx = tt & (LX - 1), ly = tt / LX;
+    // halo roles: the first LX threads row y=-1, the next LX row y=R (float4
+    // each), the next R column x=-1, the R after them column x=kTXs (one voxel each)
+    const bool hrow = tt < 2 * LX, hcol = tt >= 2 * LX && tt < 2 * LX + 2 * R;
+    const int hy = tt < LX ? -1 : tt < 2 * LX ? R : (tt < 2 * LX + R ? tt - 2 * LX : tt - 2 * LX - R);
+    const int hl = tt < LX ? tt : tt - LX;
+    const int hslot = tt < 2 * LX + R ? 3 : 4 + kTXs;
     const float cdiag = g.diag, cc = g.c;
     const int blk = BLK ? g.block : 0;  // BLK: a block lattice (no coupling across block faces)
     const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -351,13 +355,13 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
         const int tile = xcd_tile(blockIdx.x, round, nb);
         if (tile >= ntiles) break;
         const int bx = tile % tx, by = (tile / tx) % ty, bz = tile / (tx * ty);
-        const int x0 = bx * kTX4, k0 = bz * kZ4, kend = min(k0 + kZ4, nz);
-        const int j = by * TY + ly;
+        const int x0 = bx * kTXs, k0 = bz * kZs, kend = min(k0 + kZs, nz);
+        const int j = by * R + ly;
         const int xo = x0 + 4 * lx;
         const bool own = xo < nx && j < ny;
-        const int gj = by * TY + hy;
+        const int gj = by * R + hy;
         const bool hr_ok = hrow && gj >= 0 && gj < ny && x0 + 4 * hl < nx;
-        const int hx = tt < 128 + TY ? x0 - 1 : x0 + kTX4;
+        const int hx = tt < 2 * LX + R ? x0 - 1 : x0 + kTXs;
         const bool hc_ok = hcol && gj < ny && hx >= 0 && hx < nx;
         const int64_t ocol = xo + (int64_t)nx * j;
         const int64_t rcol = x0 + 4 * hl + (int64_t)nx * gj;
@@ -619,6 +623,10 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
                     }
                 }
                 if (MODE == 3) {
+                    // (padded rows: the operator at a pad voxel is left out)
+                    if (xo + 1 >= g.nxr) o.y = 0.0f;
+                    if (xo + 2 >= g.nxr) o.z = 0.0f;
+                    if (xo + 3 >= g.nxr) o.w = 0.0f;
                     float4 ro;
                     ro.x = xrc.x - alpha * o.x;
                     ro.y = xrc.y - alpha * o.y;
@@ -646,8 +654,13 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
         // a full tile's march has a compile-time trip count, so it unrolls
         // and the next plane's loads overlap the current one (a fifth of the
         // bandwidth otherwise)
-        if (kend - k0 == kZ4) {
-            if (PF == 3) {
+        if (kend - k0 == kZs) {
+            if (DYN) {
+                for (int q = 0; q < kZs; q += 2) {
+                    plane(k0 + q);
+                    plane(k0 + q + 1);
+                }
+            } else if (PF == 3) {
                 // the deferred form carries its loads across planes itself;
                 // unrolling further only adds registers
 #pragma unroll 2
@@ -1039,8 +1052,24 @@ static nnx_status check_grid(nnx_ctx* c, const nnx_grid* g) {
     return NNX_OK;
 }
 
+// Shape of the tiled iteration: lx = 0, the 256-wide tiles of 16 planes;
+// otherwise 256-thread tiles of 4 lx voxels by 256 / lx rows by zd planes.
+struct CgShape {
+    int lx, zd;
+};
+#define NNX_BY_LX(lx_, ...)                                         \
+    do {                                                            \
+        switch (lx_) {                                              \
+            case 8: { constexpr int LX = 8; __VA_ARGS__; } break;   \
+            case 16: { constexpr int LX = 16; __VA_ARGS__; } break; \
+            case 32: { constexpr int LX = 32; __VA_ARGS__; } break; \
+            default: { constexpr int LX = 64; __VA_ARGS__; } break; \
+        }                                                           \
+    } while (0)
+
 struct CgHost {
     CgDev d;
+    CgShape sh;          // of the tiled iteration
     float *pa, *pb;      // p ping-pong
     double* tr_part;     // true-residual partials
     double* out2;
@@ -1161,24 +1190,39 @@ static void cg_iter_launch(nnx_ctx* c, const GridK& gk, CgHost& h, int k, float*
     const int64_t n = (int64_t)gk.nx * gk.ny * gk.nz;
     float* pold = (k & 1) ? h.pb : h.pa;
     float* pnew = (k & 1) ? h.pa : h.pb;
+    const CgShape& sh = h.sh;
     if (fast == kFastVar) {
-        k_stencil7x4<2, kPFv, true, kTYv><<<nb4, 64 * kTYv, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero);
+        if (sh.lx == 0)
+            k_stencil7x4<2, kPFv, true, kTYv>
+                <<<nb4, 64 * kTYv, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, 0);
+        else
+            NNX_BY_LX(sh.lx, k_stencil7x4<2, 3, true, 4, false, LX, true>
+                      <<<nb4, 256, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, sh.zd));
         k_cg_rupd<<<kRedBlocks, 256, 0, c->stream>>>(n, h.d, k);
         return;
     }
     if (fast && gk.block) {
-        k_stencil7x4<2, kPFc, false, kTYc, true><<<nb4, 64 * kTYc, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x,
-                                                                                xzero);
+        k_stencil7x4<2, kPFc, false, kTYc, true>
+            <<<nb4, 64 * kTYc, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, 0);
         k_stencil7x4<3, kPFc, false, kTYc3, true>
-            <<<std::min(stencil4_blocks(gk, kTYc3), kRedBlocks), 64 * kTYc3, 0, c->stream>>>(gk, h.d, k, pnew, nullptr,
-                                                                                          nullptr, nullptr, 0);
+            <<<std::min(stencil4_blocks(gk, kTYc3), kRedBlocks), 64 * kTYc3, 0, c->stream>>>(
+                gk, h.d, k, pnew, nullptr, nullptr, nullptr, 0, 0);
+        return;
+    }
+    if (fast && sh.lx) {
+        NNX_BY_LX(sh.lx, k_stencil7x4<2, 3, false, 4, false, LX, true>
+                  <<<nb4, 256, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, sh.zd));
+        NNX_BY_LX(sh.lx, k_stencil7x4<3, 3, false, 4, false, LX, true>
+                  <<<std::min(nb4, kRedBlocks), 256, 0, c->stream>>>(gk, h.d, k, pnew, nullptr, nullptr, nullptr, 0,
+                                                                     sh.zd));
         return;
     }
     if (fast) {
-        k_stencil7x4<2, kPFc, false, kTYc><<<nb4, 64 * kTYc, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero);
+        k_stencil7x4<2, kPFc, false, kTYc>
+            <<<nb4, 64 * kTYc, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, 0);
         k_stencil7x4<3, kPFc, false, kTYc3>
-            <<<std::min(stencil4_blocks(gk, kTYc3), kRedBlocks), 64 * kTYc3, 0, c->stream>>>(gk, h.d, k, pnew, nullptr,
-                                                                                          nullptr, nullptr, 0);
+            <<<std::min(stencil4_blocks(gk, kTYc3), kRedBlocks), 64 * kTYc3, 0, c->stream>>>(
+                gk, h.d, k, pnew, nullptr, nullptr, nullptr, 0, 0);
         return;
     }
     k_cg_dir<<<kRedBlocks, 256, 0, c->stream>>>(n, h.d, k, pold, pnew);
@@ -1196,8 +1240,49 @@ static int cg_fast(const GridK& gk, const float* x) {
     if (gk.kind == 1 && (uintptr_t)gk.ky % 16 == 0 && (uintptr_t)gk.kz % 16 == 0) return kFastVar;
     return 0;
 }
+// Shape of a tiled launch on the grid.  The lanes of a row (8, 16, 32 or 64,
+// four voxels each): tiles per row x (lanes + 12), the idle lanes of the last
+// tile against the two halo columns of each (nx 152: 64 lanes 25.4 us per CG
+// iteration, 32 28.4, 16 27.3, 8 31.7; nx 100: 22.6, 20.4, 23.5, 20.2).  The
+// planes: a tile waits about a memory latency per plane, so few planes until
+// the chip is full - 2 up to 400 tiles of 4 planes, 4 up to 1024, 16 beyond
+// (32^3: 12.4 us with 2 planes, 14.9 with 4, 28 with 16; 128^3: 21.6, 20.9,
+// 35.3; 200^3: -, 67.0, 57.1).  The 16-row tiles of 1024 threads (lx = 0) where
+// they are one workgroup on (nearly) every CU (256^3: 93.5 against 100 us; but
+// 256 x 256 x 192 71.3 against 67.3, 512 x 512 x 128 218 against 208, and 39-60
+// us on the grids up to 128^3 above).  Variable coefficients: 2 planes up to
+// 128 tiles, 4 up to 640, 8 up to 2560 (64^3: 13.5, 15.8, 20.9 us; 128^3: 28.9,
+// 26.7, 26.8; 200^3 with 8, 16: 99.8, 108), then 16 where a row has idle lanes
+// in 64 (288 x 288 x 200: 204 against 246 us) and the 8-row tiles elsewhere.
+static CgShape tile_shape(const GridK& g, bool var) {
+    CgShape sh{64, 16};
+    const int64_t nx4 = ceil_div(g.nx, 4);
+    int64_t best = INT64_MAX;
+    for (int lx = 64; lx >= 8; lx /= 2) {
+        const int64_t cost = ceil_div(nx4, lx) * (lx + 12);
+        if (cost < best) best = cost, sh.lx = lx;
+    }
+    const int64_t t4 = ceil_div(nx4, sh.lx) * ceil_div(g.ny, 256 / sh.lx) * ceil_div(g.nz, 4);
+    if (var) {
+        sh.zd = t4 <= 128 ? 2 : t4 <= 640 ? 4 : t4 <= 2560 ? 8 : 16;
+        if (sh.lx == 64 && t4 > 2560) sh.lx = 0;
+        return sh;
+    }
+    sh.zd = t4 <= 400 ? 2 : t4 <= 1024 ? 4 : 16;
+    const int64_t t16 = ceil_div(g.nx, kTX4) * ceil_div(g.ny, kTY4) * ceil_div(g.nz, kZ4);
+    if (sh.lx == 64 && t16 > 200 && t16 <= 256) sh.lx = 0;
+    return sh;
+}
+// (a block lattice keeps the 256-wide tiles: its grids are laid side by side)
+static CgShape cg_shape(const GridK& gk, int fast) {
+    return fast && !gk.block ? tile_shape(gk, fast == kFastVar) : CgShape{0, 0};
+}
 // blocks of the first-half launch of a tiled iteration
-static int fast_blocks(const GridK& gk, int fast) { return stencil4_blocks(gk, fast == kFastVar ? kTYv : kTYc); }
+static int fast_blocks(const GridK& g, int fast, const CgShape& sh) {
+    if (!sh.lx) return stencil4_blocks(g, fast == kFastVar ? kTYv : kTYc);
+    const int64_t nt = ceil_div(g.nx, 4 * sh.lx) * ceil_div(g.ny, 256 / sh.lx) * ceil_div(g.nz, sh.zd);
+    return (int)std::min<int64_t>(nt, 2048);
+}
 
 // the pending x update of the fast path (nothing otherwise)
 static void cg_finish_launch(nnx_ctx* c, const GridK& gk, CgHost& h, float* x, int xzero = 0,
@@ -1218,7 +1303,8 @@ static nnx_status cg_run(nnx_ctx* c, const GridK& gk, CgHost& h, const float* b,
     const int vec = ((uintptr_t)x % 16) == 0;
     // 7-point grids with 16-byte rows: the LDS float4 kernels
     const int fast = cg_fast(gk, x);
-    const int nb4 = fast_blocks(gk, fast);
+    h.sh = cg_shape(gk, fast);
+    const int nb4 = fast_blocks(gk, fast, h.sh);
     h.d.npq = fast ? nb4 : kRedBlocks;
     int32_t fl[FL_N];
     double sc[SC_N];
@@ -1284,7 +1370,8 @@ static void cg_enqueue_fixed(nnx_ctx* c, const GridK& gk, CgHost& h, const float
     k_cg_init_fin<<<1, 256, 0, c->stream>>>(h.d, tol, 0, maxit);
     const int vec = ((uintptr_t)x % 16) == 0;
     const int fast = cg_fast(gk, x);
-    const int nb4 = fast_blocks(gk, fast);
+    h.sh = cg_shape(gk, fast);
+    const int nb4 = fast_blocks(gk, fast, h.sh);
     h.d.npq = fast ? nb4 : kRedBlocks;
     for (int k = 0; k < maxit; ++k) cg_iter_launch(c, gk, h, k, x, vec, fast, nb4);
     cg_finish_launch(c, gk, h, x);
@@ -1641,10 +1728,14 @@ nnx_status nnx_stencil_apply(nnx_ctx* c, const nnx_grid* g, const float* x, floa
         CgDev none{};
         if (gk.block)
             k_stencil7x4<0, kPFa, false, kTYa, true>
-                <<<stencil4_blocks(gk, kTYa), 64 * kTYa, 0, c->stream>>>(gk, none, 0, x, nullptr, nullptr, y, 0);
+                <<<stencil4_blocks(gk, kTYa), 64 * kTYa, 0, c->stream>>>(gk, none, 0, x, nullptr, nullptr, y, 0, 0);
+        else if (const CgShape sh = tile_shape(gk, false); sh.lx && sh.zd <= 4)
+            NNX_BY_LX(sh.lx, k_stencil7x4<0, 3, false, 4, false, LX, true>
+                      <<<fast_blocks(gk, kFastConst, sh), 256, 0, c->stream>>>(gk, none, 0, x, nullptr, nullptr, y, 0,
+                                                                                sh.zd));
         else
             k_stencil7x4<0, kPFa, false, kTYa>
-                <<<stencil4_blocks(gk, kTYa), 64 * kTYa, 0, c->stream>>>(gk, none, 0, x, nullptr, nullptr, y, 0);
+                <<<stencil4_blocks(gk, kTYa), 64 * kTYa, 0, c->stream>>>(gk, none, 0, x, nullptr, nullptr, y, 0, 0);
     } else {
         k_apply<float, float><<<grid3(gk), 256, 0, c->stream>>>(gk, x, y);
     }
@@ -1809,7 +1900,8 @@ nnx_status para_launch(nnx_ctx* c, const ParaIo& io) {
     // without storing it and its last update goes straight into the field
     const int fast = cg_fast(gk, ph.xin);
     const bool tiled = fast == kFastConst && (uintptr_t)q.conc % 16 == 0;
-    const int nb4 = fast_blocks(gk, fast), nbr = std::min(stencil4_blocks(gk), kRedBlocks);
+    h.sh = cg_shape(gk, fast);
+    const int nb4 = fast_blocks(gk, fast, h.sh), nbr = std::min(stencil4_blocks(gk), kRedBlocks);
     h.d.npq = fast ? nb4 : kRedBlocks;
     k_para_rhs<<<kRedBlocks, 256, 0, c->stream>>>(nv, q.conc, io.voxel_counts, q.release, ph.b, ph.pbb, ph.pfl);
     for (int o = 0; o < max_outer; ++o) {

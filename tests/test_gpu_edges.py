@@ -47,3 +47,48 @@ def test_count_coupling_splits(ctx, n, nnz):
             bits, out = DA.from_numpy(ctx, words), DA.from_numpy(ctx, np.full(n, np.nan, T))
             ctx.call("nnx_couple", C.byref(g), _lib.COUPLE_COUNT, DT[T], bits.ptr, None, None, None, out.ptr)
             assert np.array_equal(out.numpy(), (cum[off[1:]] - cum[off[:-1]]).astype(T))
+
+
+def _operator(ctx, nx, ny, nz, var, seed=6):
+    """Device grid, oracle grid and the arrays to keep: constant c = 1.3, or
+    random face coefficients."""
+    import oracle
+    if not var:
+        return _lib.Grid(nx, ny, nz, 7, 1.3, 0.0, None, None, None), oracle.grid(nx, ny, nz, 7, 1.3), []
+    rng = np.random.default_rng(seed)
+    k = [rng.uniform(0.1, 5, s).astype(np.float32)
+         for s in ((nz, ny, nx + 1), (nz, ny + 1, nx), (nz + 1, ny, nx))]
+    d = [DA.from_numpy(ctx, a) for a in k]
+    return _lib.Grid(nx, ny, nz, 7, 0.0, 0.0, *(a.ptr for a in d)), oracle.grid(nx, ny, nz, 7, 0.0, 0.0, *k), d
+
+
+# rows of 8, 16, 32 and 64 lanes with remainders in x, y and z; 2, 4 and 16
+# planes a tile (variable coefficients: 2, 4, 8 and 16)
+SHAPES = [(4, 3, 2), (20, 33, 7), (60, 50, 41), (100, 131, 22), (128, 130, 66), (152, 90, 97), (200, 120, 151)]
+
+
+@pytest.mark.parametrize("dims,var", [(d, v) for d in SHAPES for v in (False, True)] + [((276, 200, 190), True)])
+def test_tiled_solve_shapes(ctx, dims, var):
+    """The apply bit for bit; three CG iterations from zero against the
+    oracle's (its sums taken in another order: alpha and beta are fp32 roundings
+    of FP64 sums, each within 2^-23 of the oracle's, and the vectors' own
+    roundings add a few 2^-24 an iteration: 1e-5 of the largest value); a
+    refined solve to 1e-9 by its FP64 residual with the oracle's operator."""
+    import oracle
+    nx, ny, nz = dims
+    say("tiles", dims, "var" if var else "const")
+    g, og, keep = _operator(ctx, nx, ny, nz, var)
+    n = nx * ny * nz
+    b = np.random.default_rng(n).standard_normal(n).astype(np.float32)
+    db, dx = DA.from_numpy(ctx, b), DA.zeros(ctx, n, np.float32)
+    ctx.call("nnx_stencil_apply", C.byref(g), db.ptr, dx.ptr)
+    assert np.array_equal(dx.numpy(), oracle.apply(og, b))
+    o = _lib.CgOpts(rtol=0.0, maxit=3, precond=_lib.PRECOND_JACOBI, check_every=1)
+    assert ctx._l.nnx_cg_solve(ctx.h, C.byref(g), db.ptr, dx.ptr, C.byref(o), None) == 4  # NNX_ERR_NOCONV
+    ref = oracle.cg(og, b, 0.0, maxit=3)[0]
+    assert np.abs(dx.numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
+    b64, x64 = DA.from_numpy(ctx, b.astype(np.float64)), DA.zeros(ctx, n, np.float64)
+    o = _lib.CgOpts(rtol=1e-9, maxit=500, precond=_lib.PRECOND_JACOBI, check_every=4)
+    ctx.call("nnx_cg_solve_refine", C.byref(g), b64.ptr, x64.ptr, C.byref(o), 1e-6, 10, None)
+    res = b.astype(np.float64) - oracle.apply(og, x64.numpy())
+    assert np.linalg.norm(res) <= 1.001e-9 * np.linalg.norm(b.astype(np.float64))
