@@ -170,15 +170,18 @@ nnx_status check_hebbian_plan(nnx_ctx* c, const nnx_step_plan* p);
 // partials (kCgPartDoubles).
 struct CgMem {
     float *r, *pa, *pb, *q, *dinv;
+    float* xp;  // the iterate in padded rows (null: the caller's x is used)
     double* sc;
     int32_t* fl;
     double* part;
 };
 constexpr size_t kCgPartDoubles = (size_t)1024 * 16;
-// bytes of a working set for grid g (256-byte aligned pieces) and its
-// layout inside `base` (256-byte aligned, cg_mem_bytes long)
-size_t cg_mem_bytes(const nnx_grid* g, int precond);
-CgMem cg_mem_carve(void* base, const nnx_grid* g, int precond);
+// bytes of a working set for a solve of g into x (256-byte aligned pieces)
+// and its layout inside `base` (256-byte aligned, cg_mem_bytes long)
+size_t cg_mem_bytes(const nnx_grid* g, int precond, const float* x);
+CgMem cg_mem_carve(void* base, const nnx_grid* g, int precond, const float* x);
+// the fixed array of nnx_cg_solve_async_noalloc
+constexpr size_t kNoallocBytes = (size_t)48 << 20;
 // argument checks and the launches of nnx_cg_solve_async on a working set
 nnx_status cg_async_check(nnx_ctx* c, const nnx_grid* g, const float* b, const float* x, const nnx_cg_opts* o,
                           const double* d_result);

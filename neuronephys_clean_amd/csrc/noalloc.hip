@@ -17,7 +17,7 @@
 
 // 48 MiB: a 128^3 grid with variable coefficients and Jacobi needs 40 MiB
 // plus 132 KiB (five n-vectors and the reduction partials)
-constexpr size_t kNoallocBytes = (size_t)48 << 20;
+using nnx::kNoallocBytes;
 static __device__ __align__(256) unsigned char scratch[kNoallocBytes];
 
 namespace {
@@ -49,7 +49,7 @@ extern "C" nnx_status nnx_cg_solve_async_noalloc(nnx_ctx* c, const nnx_grid* g, 
                                                  const nnx_cg_opts* o, double* d_result) {
     if (!c) return NNX_ERR_ARG;
     NNX_TRY(nnx::cg_async_check(c, g, b, x, o, d_result));
-    const size_t need = nnx::cg_mem_bytes(g, o->precond);
+    const size_t need = nnx::cg_mem_bytes(g, o->precond, x);
     if (need > kNoallocBytes)
         return nnx::fail(c, NNX_ERR_ARG,
                          "nnx_cg_solve_async_noalloc: a %dx%dx%d grid needs %zu bytes of working memory, "
@@ -64,5 +64,5 @@ extern "C" nnx_status nnx_cg_solve_async_noalloc(nnx_ctx* c, const nnx_grid* g, 
     if (!base)
         return nnx::fail(c, NNX_ERR_STATE, "no working memory on device %d: the address lookup %s", c->device,
                          err != hipSuccess ? hipGetErrorString(err) : "did not run");
-    return nnx::cg_async_launch(c, g, b, x, o, d_result, nnx::cg_mem_carve(base, g, o->precond));
+    return nnx::cg_async_launch(c, g, b, x, o, d_result, nnx::cg_mem_carve(base, g, o->precond, x));
 }

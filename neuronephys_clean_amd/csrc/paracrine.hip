@@ -255,6 +255,7 @@ __global__ __launch_bounds__(256) void k_cg_status(CgDev d) {
 // still waited for in the step that issues it.  3, the deferred form: the
 // raw values are loaded two planes ahead at clamped addresses, with no
 // arithmetic and no condition at the load, and finished one step later.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // 16 bytes at a 4-byte address
 constexpr int kTX4 = 256, kTY4 = 16, kZ4 = 16, kT4 = 64 * kTY4, kRow4 = kTX4 + 8;
 // prefetch forms and tile heights the solver launches (measured at 256^3):
 // the apply and the variable-coefficient first half take the deferred form;
@@ -276,7 +277,8 @@ __device__ __forceinline__ int xcd_tile(int b, int round, int nb) {
     const int t = nb % 8 == 0 ? (b % 8) * (nb / 8) + b / 8 : b;
     return t + round * nb;
 }
-template <int MODE, int PF, bool VAR = false, int TY = kTY4, bool BLK = false, int LX = 64, bool DYN = false>
+template <int MODE, int PF, bool VAR = false, int TY = kTY4, bool BLK = false, int LX = 64, bool DYN = false,
+          bool RAG = false>
 __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k, const float* __restrict__ src,
                                                     const float* __restrict__ pold, float* __restrict__ pnew,
                                                     float* __restrict__ dst, int xzero, int zdyn) {
@@ -475,8 +477,31 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
         // the z face below a plane is the one above the plane before it
         float nkx[5] = {0, 0, 0, 0, 0};
         float4 nkym = z4, nkyp = z4, nkzp = z4, ckzm = z4;
+        // RAG: rows of nxr voxels at any alignment - 16-byte loads from 4-byte
+        // addresses; the group past the array's end (the last row's, whose
+        // last pad voxels are none of the grid) is loaded at the last 4
+        // entries and shifted
+        auto ldu = [&](const float* f, int64_t e, int64_t tot) -> float4 {
+            const int64_t ec = e < tot - 4 ? e : tot - 4;
+            const f4u v = *reinterpret_cast<const f4u*>(f + ec);
+            const int sh = (int)(e - ec);
+            return make_float4(sh == 0 ? v.x : sh == 1 ? v.y : sh == 2 ? v.z : v.w,
+                               sh == 0 ? v.y : sh == 1 ? v.z : v.w, sh == 0 ? v.z : v.w, v.w);
+        };
         auto ld_faces = [&](int kz) {
             const bool ok = own && kz < nz;
+            if (RAG) {
+                const int nr = g.nxr;
+                const int64_t ex = ok ? xo + (int64_t)(nr + 1) * (j + (int64_t)ny * kz) : 0;
+#pragma unroll
+                for (int q = 0; q < 5; ++q) nkx[q] = g.kx[ex + (ok && q > nr - xo ? nr - xo : q)];
+                const int64_t tky = (int64_t)nr * (ny + 1) * nz, tkz = (int64_t)nr * ny * (nz + 1);
+                const int64_t fy = ok ? xo + (int64_t)nr * (j + (int64_t)(ny + 1) * kz) : 0;
+                nkym = ldu(g.ky, fy, tky);
+                nkyp = ldu(g.ky, fy + (ok ? nr : 0), tky);
+                nkzp = ldu(g.kz, ok ? xo + (int64_t)nr * (j + (int64_t)ny * (kz + 1)) : 0, tkz);
+                return;
+            }
             const int64_t ex = ok ? xo + (int64_t)(nx + 1) * (j + (int64_t)ny * kz) : 0;
 #pragma unroll
             for (int q = 0; q < 5; ++q) nkx[q] = g.kx[ex + q];
@@ -506,7 +531,11 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
             ld_own(rok_o, ocol + sxy * (k0 + 1), rwo);
             ld_row(rok_r, rcol + sxy * (k0 + 1), rwr);
             ld_col(rok_c, ccol + sxy * (k0 + 1), rwc);
-            if (VAR) {
+            if (VAR && RAG) {
+                ckzm = ldu(g.kz, own ? xo + (int64_t)g.nxr * (j + (int64_t)ny * k0) : 0,
+                           (int64_t)g.nxr * ny * (nz + 1));
+                ld_faces(k0);
+            } else if (VAR) {
                 ckzm = *reinterpret_cast<const float4*>(g.kz + (own ? ocol + sxy * k0 : 0));
                 ld_faces(k0);
             }
@@ -604,6 +633,12 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
                     }
                     o = make_float4(ov[0], ov[1], ov[2], ov[3]);
                 }
+                if (MODE == 3 || VAR) {
+                    // (padded rows: the operator at a pad voxel is left out)
+                    if (xo + 1 >= g.nxr) o.y = 0.0f;
+                    if (xo + 2 >= g.nxr) o.z = 0.0f;
+                    if (xo + 3 >= g.nxr) o.w = 0.0f;
+                }
                 const int64_t id = ocol + sxy * kz;
                 if (MODE == 0) *reinterpret_cast<float4*>(dst + id) = o;
                 if (MODE == 2) {
@@ -623,10 +658,6 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
                     }
                 }
                 if (MODE == 3) {
-                    // (padded rows: the operator at a pad voxel is left out)
-                    if (xo + 1 >= g.nxr) o.y = 0.0f;
-                    if (xo + 2 >= g.nxr) o.z = 0.0f;
-                    if (xo + 3 >= g.nxr) o.w = 0.0f;
                     float4 ro;
                     ro.x = xrc.x - alpha * o.x;
                     ro.y = xrc.y - alpha * o.y;
@@ -1004,6 +1035,52 @@ __global__ void k_dinv(GridK g, float* dinv) {
         dinv[i] = dinv_at(g, i);
 }
 
+// ---- the same on working vectors in rows of px >= nx voxels, zero beyond nx ----
+__global__ __launch_bounds__(256) void k_dinv_pad(GridK g, int px, float* __restrict__ dinv) {
+    for_rows(px, g.ny, g.nz, [&](int i, int j, int k, int64_t id) {
+        dinv[id] = i < g.nx ? dinv_at(g, i + (int64_t)g.nx * (j + (int64_t)g.ny * k)) : 0.0f;
+    });
+}
+// k_cg_init with the iterate copied into xp
+__global__ __launch_bounds__(256) void k_cg_init_pad(GridK g, int px, CgDev d, const float* __restrict__ b,
+                                                     const float* __restrict__ x, int use_x0,
+                                                     float* __restrict__ p0, float* __restrict__ xp) {
+    double vb[1] = {0}, vu[2] = {0, 0};
+    for_rows(px, g.ny, g.nz, [&](int i, int j, int k, int64_t id) {
+        float ri = 0.0f, xi = 0.0f;
+        if (i < g.nx) {
+            const int64_t e = i + (int64_t)g.nx * (j + (int64_t)g.ny * k);
+            ri = b[e];
+            vb[0] += (double)ri * ri;
+            if (use_x0) {
+                xi = x[e];
+                ri = ri - apply_at<float, float>(x, g, i, j, k);
+            }
+        }
+        d.r[id] = ri;
+        p0[id] = 0.0f;
+        xp[id] = xi;
+        vu[0] += (double)ri * (ri * dv(d, id));
+        vu[1] += (double)ri * ri;
+    });
+    put_partial<1>(vb, d.pb);
+    put_partial<2>(vu, d.pu0);
+}
+// x = xp + the deferred alpha_k p_k of the last executed iteration (without
+// one: x = xp, or nothing unless `always`)
+__global__ __launch_bounds__(256) void k_cg_finish_pad(GridK g, CgDev d, const float* __restrict__ pa,
+                                                       const float* __restrict__ pb, const float* __restrict__ xp,
+                                                       float* __restrict__ x, int always) {
+    const bool pend = d.fl[FL_XPEND] != 0;
+    if (!pend && !always) return;
+    const int k = d.fl[FL_ITERS] - 1;
+    const float alpha = pend ? (float)d.sc[SC_ALK + (k & 1)] : 0.0f;
+    const float* __restrict__ p = (k & 1) ? pa : pb;
+    for_rows(g.nx, g.ny, g.nz, [&](int i, int j, int kk, int64_t id) {
+        if (i < g.nxr) x[i + (int64_t)g.nxr * (j + (int64_t)g.ny * kk)] = pend ? xp[id] + alpha * p[id] : xp[id];
+    });
+}
+
 // ||b - A x||^2 and ||b||^2 in FP64 (x float or double): partials, then one
 // block adds them (out2[0], out2[1]); r_out optionally receives b - A x.
 template <class U, class B>
@@ -1069,177 +1146,18 @@ struct CgShape {
 
 struct CgHost {
     CgDev d;
-    CgShape sh;          // of the tiled iteration
     float *pa, *pb;      // p ping-pong
     double* tr_part;     // true-residual partials
     double* out2;
+    int fast;            // the iteration: kFastConst, kFastVar (tiled) or 0 (generic)
+    bool pad;            // tiled on padded rows: the vectors in rows of gp.nx, the iterate in xp
+    GridK gp;            // the grid of the working vectors
+    float* xp;
+    CgShape sh;          // of the tiled kernels
+    int nb4;             // blocks of the first half
+    int64_t n() const { return (int64_t)gp.nx * gp.ny * gp.nz; }
 };
 
-static_assert(kCgPartDoubles == (size_t)kRedBlocks * 16, "partials region");
-
-static bool cg_needs_dinv(const GridK& gk, int precond) { return precond == NNX_PRECOND_JACOBI && gk.kind == 1; }
-
-static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
-
-size_t cg_mem_bytes(const nnx_grid* g, int precond) {
-    const GridK gk = make_grid(g);
-    const size_t n = (size_t)gk.nx * gk.ny * gk.nz;
-    const size_t vec = align256(n * 4);
-    return align256(kCgPartDoubles * 8) + 512 + 256 + 256 + 4 * vec + (cg_needs_dinv(gk, precond) ? vec : 0);
-}
-
-CgMem cg_mem_carve(void* base, const nnx_grid* g, int precond) {
-    const GridK gk = make_grid(g);
-    const size_t n = (size_t)gk.nx * gk.ny * gk.nz;
-    const size_t vec = align256(n * 4);
-    char* p = (char*)base;
-    CgMem m;
-    m.part = (double*)p;
-    p += align256(kCgPartDoubles * 8);
-    m.sc = (double*)p;
-    p += 512;
-    m.fl = (int32_t*)p;
-    p += 512;
-    m.r = (float*)p, p += vec;
-    m.pa = (float*)p, p += vec;
-    m.pb = (float*)p, p += vec;
-    m.q = (float*)p, p += vec;
-    m.dinv = cg_needs_dinv(gk, precond) ? (float*)p : nullptr;
-    return m;
-}
-
-// the working set from the context's named scratch buffers `prefix`_*
-static nnx_status cg_mem_scratch(nnx_ctx* c, const char* prefix, const GridK& gk, int precond, CgMem* m) {
-    const int64_t n = (int64_t)gk.nx * gk.ny * gk.nz;
-    char nm[64];
-    void* p[8] = {};
-    const char* names[] = {"r", "pa", "pb", "q", "sc", "fl", "part"};
-    const size_t bytes[] = {(size_t)n * 4, (size_t)n * 4, (size_t)n * 4, (size_t)n * 4, 64 * 8, 64 * 4,
-                            kCgPartDoubles * 8};
-    for (int i = 0; i < 7; ++i) {
-        std::snprintf(nm, sizeof nm, "%s_%s", prefix, names[i]);
-        NNX_TRY(scratch(c, nm, bytes[i], i == 4 || i == 5, &p[i]));
-    }
-    m->dinv = nullptr;
-    if (cg_needs_dinv(gk, precond)) {
-        std::snprintf(nm, sizeof nm, "%s_dinv", prefix);
-        void* dvp;
-        NNX_TRY(scratch(c, nm, n * 4, false, &dvp));
-        m->dinv = (float*)dvp;
-    }
-    m->r = (float*)p[0], m->pa = (float*)p[1], m->pb = (float*)p[2], m->q = (float*)p[3];
-    m->sc = (double*)p[4], m->fl = (int32_t*)p[5], m->part = (double*)p[6];
-    return NNX_OK;
-}
-
-// Points h at the working set m; fills the inverse diagonal when the grid
-// needs one (a launch on the context's stream).
-static nnx_status cg_bind(nnx_ctx* c, const GridK& gk, int precond, const CgMem& m, CgHost* h) {
-    const int64_t n = (int64_t)gk.nx * gk.ny * gk.nz;
-    double* P = m.part;
-    h->d.r = m.r;
-    h->d.q = m.q;
-    h->pa = m.pa;
-    h->pb = m.pb;
-    h->d.sc = m.sc;
-    h->d.fl = m.fl;
-    h->d.pu0 = P;                     // 2 x kRedBlocks
-    h->d.pu1 = P + 2 * kRedBlocks;    // 2 x kRedBlocks
-    h->d.ppq = P + 4 * kRedBlocks;    // up to 2048 operator blocks
-    h->d.pb = P + 6 * kRedBlocks;     // kRedBlocks
-    h->tr_part = P + 7 * kRedBlocks;  // 2 x kRedBlocks
-    h->d.ppq1 = P + 11 * kRedBlocks;  // up to 2048 (9 and 10 x kRedBlocks: the paracrine solve's)
-    h->out2 = m.sc + 32;
-    h->d.dinv = nullptr;
-    h->d.dinv_c = 1.0f;
-    if (precond == NNX_PRECOND_JACOBI) {
-        if (gk.kind == 1) {
-            h->d.dinv = m.dinv;
-            k_dinv<<<flat_blocks(n), 256, 0, c->stream>>>(gk, h->d.dinv);
-            NNX_LAUNCHED(c);
-        } else {
-            h->d.dinv_c = gk.kind == 0 ? (float)(1.0 / gk.diagd) : (float)(1.0 / (gk.a0d + 128.0 * gk.wd));
-        }
-    }
-    return NNX_OK;
-}
-
-static nnx_status cg_buffers(nnx_ctx* c, const GridK& gk, int precond, CgHost* h) {
-    CgMem m;
-    NNX_TRY(cg_mem_scratch(c, "cg", gk, precond, &m));
-    return cg_bind(c, gk, precond, m, h);
-}
-
-static nnx_status cg_readback(nnx_ctx* c, CgHost& h, int32_t* fl, double* sc) {
-    NNX_HIP(c, hipMemcpyAsync(c->pinned, h.d.fl, 4 * FL_N, hipMemcpyDeviceToHost, c->stream));
-    NNX_HIP(c, hipMemcpyAsync((char*)c->pinned + 64, h.d.sc, 8 * SC_N, hipMemcpyDeviceToHost, c->stream));
-    NNX_HIP(c, hipStreamSynchronize(c->stream));
-    std::memcpy(fl, c->pinned, 4 * FL_N);
-    std::memcpy(sc, (char*)c->pinned + 64, 8 * SC_N);
-    return NNX_OK;
-}
-
-// Iteration k of CG on the prepared buffers.  Constant 7-point stencil with
-// 16-byte rows and x (fast): the two halves of k_stencil7x4 (modes 2, 3),
-// the x update deferred by one iteration (k_cg_finish applies the last);
-// otherwise the new direction, q = A p, then the update of x and r.  Every
-// kernel returns at once when the device flag says the solve is over, so
-// iterations can be enqueued past convergence.
-static void cg_iter_launch(nnx_ctx* c, const GridK& gk, CgHost& h, int k, float* x, int vec, int fast, int nb4,
-                           int xzero = 0) {
-    const int64_t n = (int64_t)gk.nx * gk.ny * gk.nz;
-    float* pold = (k & 1) ? h.pb : h.pa;
-    float* pnew = (k & 1) ? h.pa : h.pb;
-    const CgShape& sh = h.sh;
-    if (fast == kFastVar) {
-        if (sh.lx == 0)
-            k_stencil7x4<2, kPFv, true, kTYv>
-                <<<nb4, 64 * kTYv, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, 0);
-        else
-            NNX_BY_LX(sh.lx, k_stencil7x4<2, 3, true, 4, false, LX, true>
-                      <<<nb4, 256, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, sh.zd));
-        k_cg_rupd<<<kRedBlocks, 256, 0, c->stream>>>(n, h.d, k);
-        return;
-    }
-    if (fast && gk.block) {
-        k_stencil7x4<2, kPFc, false, kTYc, true>
-            <<<nb4, 64 * kTYc, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, 0);
-        k_stencil7x4<3, kPFc, false, kTYc3, true>
-            <<<std::min(stencil4_blocks(gk, kTYc3), kRedBlocks), 64 * kTYc3, 0, c->stream>>>(
-                gk, h.d, k, pnew, nullptr, nullptr, nullptr, 0, 0);
-        return;
-    }
-    if (fast && sh.lx) {
-        NNX_BY_LX(sh.lx, k_stencil7x4<2, 3, false, 4, false, LX, true>
-                  <<<nb4, 256, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, sh.zd));
-        NNX_BY_LX(sh.lx, k_stencil7x4<3, 3, false, 4, false, LX, true>
-                  <<<std::min(nb4, kRedBlocks), 256, 0, c->stream>>>(gk, h.d, k, pnew, nullptr, nullptr, nullptr, 0,
-                                                                     sh.zd));
-        return;
-    }
-    if (fast) {
-        k_stencil7x4<2, kPFc, false, kTYc>
-            <<<nb4, 64 * kTYc, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, 0);
-        k_stencil7x4<3, kPFc, false, kTYc3>
-            <<<std::min(stencil4_blocks(gk, kTYc3), kRedBlocks), 64 * kTYc3, 0, c->stream>>>(
-                gk, h.d, k, pnew, nullptr, nullptr, nullptr, 0, 0);
-        return;
-    }
-    k_cg_dir<<<kRedBlocks, 256, 0, c->stream>>>(n, h.d, k, pold, pnew);
-    k_cg_spmv_gen<<<kRedBlocks, 256, 0, c->stream>>>(gk, h.d, k, pnew);
-    k_cg_update<<<kRedBlocks, 256, 0, c->stream>>>(n, h.d, k, pnew, x, vec);
-}
-
-// The tiled iteration: kFastConst on the constant 7-point grid, kFastVar on
-// the variable-coefficient one (rows of a multiple of 4 voxels, 16-byte
-// aligned vectors and ky, kz); 0: the generic kernels.
-static int cg_fast(const GridK& gk, const float* x) {
-    // (a block lattice's faces must fall between the 4-voxel groups)
-    if (gk.nx % 4 != 0 || gk.block % 4 != 0 || (uintptr_t)x % 16 != 0) return 0;
-    if (gk.kind == 0) return kFastConst;
-    if (gk.kind == 1 && (uintptr_t)gk.ky % 16 == 0 && (uintptr_t)gk.kz % 16 == 0) return kFastVar;
-    return 0;
-}
 // Shape of a tiled launch on the grid.  The lanes of a row (8, 16, 32 or 64,
 // four voxels each): tiles per row x (lanes + 12), the idle lanes of the last
 // tile against the two halo columns of each (nx 152: 64 lanes 25.4 us per CG
@@ -1284,11 +1202,243 @@ static int fast_blocks(const GridK& g, int fast, const CgShape& sh) {
     return (int)std::min<int64_t>(nt, 2048);
 }
 
-// the pending x update of the fast path (nothing otherwise)
-static void cg_finish_launch(nnx_ctx* c, const GridK& gk, CgHost& h, float* x, int xzero = 0,
-                             double* acc = nullptr) {
-    const int64_t n = (int64_t)gk.nx * gk.ny * gk.nz;
-    k_cg_finish<<<flat_blocks(n / 4), 256, 0, c->stream>>>(n, h.d, h.pa, h.pb, x, xzero, acc);
+static_assert(kCgPartDoubles == (size_t)kRedBlocks * 16, "partials region");
+
+static bool cg_needs_dinv(const GridK& gk, int precond) { return precond == NNX_PRECOND_JACOBI && gk.kind == 1; }
+
+static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+static GridK padded_grid(const GridK& gk) {
+    GridK gp = gk;
+    gp.nx = (gk.nx + 3) & ~3;
+    return gp;
+}
+static size_t cg_bytes(const GridK& gk, int precond, bool pad) {
+    const GridK gp = pad ? padded_grid(gk) : gk;
+    const size_t vec = align256((size_t)gp.nx * gp.ny * gp.nz * 4);
+    const int nv = 4 + cg_needs_dinv(gk, precond) + (pad && gk.kind == 1);
+    return align256(kCgPartDoubles * 8) + 512 + 256 + 256 + nv * vec;
+}
+
+// The iteration a solve of the grid into x takes.  7-point grids: the tiled
+// kernels, in place where x and the rows are 16-byte aligned (and, with
+// variable coefficients, ky and kz), else on working vectors whose rows are
+// padded to a multiple of 4 voxels with zeros (the operator is left out at a
+// pad voxel, so that its residual, direction and iterate stay zero), from 12
+// voxels a row on - shorter rows, 27-point stencils and block lattices off
+// the 4-voxel groups: the generic kernels (150 x 131 x 97: 45 us per
+// iteration against 25 in padded rows).  A grid that only fits
+// nnx_cg_solve_async_noalloc's array unpadded stays generic in every solver,
+// so that the solvers' results agree.
+static int cg_fast(const GridK& gk, int precond, const float* x, bool* pad) {
+    *pad = false;
+    if (gk.kind == 2 || gk.block % 4 != 0) return 0;
+    const int fast = gk.kind == 0 ? kFastConst : kFastVar;
+    const bool faces = gk.kind == 0 || ((uintptr_t)gk.ky % 16 == 0 && (uintptr_t)gk.kz % 16 == 0);
+    if (gk.nx % 4 == 0 && (uintptr_t)x % 16 == 0 && faces) return fast;
+    if (gk.block || gk.nx < 12) return 0;
+    if (cg_bytes(gk, precond, true) > kNoallocBytes && cg_bytes(gk, precond, false) <= kNoallocBytes) return 0;
+    *pad = true;
+    return fast;
+}
+
+size_t cg_mem_bytes(const nnx_grid* g, int precond, const float* x) {
+    const GridK gk = make_grid(g);
+    bool pad;
+    cg_fast(gk, precond, x, &pad);
+    return cg_bytes(gk, precond, pad);
+}
+
+CgMem cg_mem_carve(void* base, const nnx_grid* g, int precond, const float* x) {
+    const GridK gk = make_grid(g);
+    bool pad;
+    cg_fast(gk, precond, x, &pad);
+    const GridK gp = pad ? padded_grid(gk) : gk;
+    const size_t vec = align256((size_t)gp.nx * gp.ny * gp.nz * 4);
+    char* p = (char*)base;
+    CgMem m;
+    m.part = (double*)p;
+    p += align256(kCgPartDoubles * 8);
+    m.sc = (double*)p;
+    p += 512;
+    m.fl = (int32_t*)p;
+    p += 512;
+    m.r = (float*)p, p += vec;
+    m.pa = (float*)p, p += vec;
+    m.pb = (float*)p, p += vec;
+    m.q = (float*)p, p += vec;
+    m.dinv = nullptr;
+    if (cg_needs_dinv(gk, precond)) m.dinv = (float*)p, p += vec;
+    // (constant coefficients: q is not stored, its vector holds the iterate)
+    m.xp = !pad ? nullptr : gk.kind == 1 ? (float*)p : m.q;
+    return m;
+}
+
+// the working set from the context's named scratch buffers `prefix`_*
+static nnx_status cg_mem_scratch(nnx_ctx* c, const char* prefix, const GridK& gk, int precond, const float* x,
+                                 CgMem* m) {
+    bool pad;
+    cg_fast(gk, precond, x, &pad);
+    const GridK gp = pad ? padded_grid(gk) : gk;
+    const int64_t n = (int64_t)gp.nx * gp.ny * gp.nz;
+    char nm[64];
+    void* p[8] = {};
+    const char* names[] = {"r", "pa", "pb", "q", "sc", "fl", "part"};
+    const size_t bytes[] = {(size_t)n * 4, (size_t)n * 4, (size_t)n * 4, (size_t)n * 4, 64 * 8, 64 * 4,
+                            kCgPartDoubles * 8};
+    for (int i = 0; i < 7; ++i) {
+        std::snprintf(nm, sizeof nm, "%s_%s", prefix, names[i]);
+        NNX_TRY(scratch(c, nm, bytes[i], i == 4 || i == 5, &p[i]));
+    }
+    m->dinv = nullptr;
+    if (cg_needs_dinv(gk, precond)) {
+        std::snprintf(nm, sizeof nm, "%s_dinv", prefix);
+        void* dvp;
+        NNX_TRY(scratch(c, nm, n * 4, false, &dvp));
+        m->dinv = (float*)dvp;
+    }
+    m->r = (float*)p[0], m->pa = (float*)p[1], m->pb = (float*)p[2], m->q = (float*)p[3];
+    m->sc = (double*)p[4], m->fl = (int32_t*)p[5], m->part = (double*)p[6];
+    m->xp = pad ? m->q : nullptr;
+    if (pad && gk.kind == 1) {
+        std::snprintf(nm, sizeof nm, "%s_xp", prefix);
+        void* xpp;
+        NNX_TRY(scratch(c, nm, n * 4, false, &xpp));
+        m->xp = (float*)xpp;
+    }
+    return NNX_OK;
+}
+
+// Points h at the working set m of a solve into x and sets its iteration;
+// fills the inverse diagonal when the grid needs one (a launch on the
+// context's stream; fill_dinv false: it is there already).
+static nnx_status cg_bind(nnx_ctx* c, const GridK& gk, int precond, const float* x, const CgMem& m, CgHost* h,
+                          bool fill_dinv = true) {
+    h->fast = cg_fast(gk, precond, x, &h->pad);
+    h->gp = h->pad ? padded_grid(gk) : gk;
+    h->xp = m.xp;
+    h->sh = cg_shape(h->gp, h->fast);
+    if (h->pad && h->fast == kFastVar && !h->sh.lx) h->sh = CgShape{64, 16};
+    h->nb4 = fast_blocks(h->gp, h->fast, h->sh);
+    double* P = m.part;
+    h->d.npq = h->fast ? h->nb4 : kRedBlocks;
+    h->d.r = m.r;
+    h->d.q = m.q;
+    h->pa = m.pa;
+    h->pb = m.pb;
+    h->d.sc = m.sc;
+    h->d.fl = m.fl;
+    h->d.pu0 = P;                     // 2 x kRedBlocks
+    h->d.pu1 = P + 2 * kRedBlocks;    // 2 x kRedBlocks
+    h->d.ppq = P + 4 * kRedBlocks;    // up to 2048 operator blocks
+    h->d.pb = P + 6 * kRedBlocks;     // kRedBlocks
+    h->tr_part = P + 7 * kRedBlocks;  // 2 x kRedBlocks
+    h->d.ppq1 = P + 11 * kRedBlocks;  // up to 2048 (9 and 10 x kRedBlocks: the paracrine solve's)
+    h->out2 = m.sc + 32;
+    h->d.dinv = nullptr;
+    h->d.dinv_c = 1.0f;
+    if (precond == NNX_PRECOND_JACOBI) {
+        if (gk.kind == 1) {
+            h->d.dinv = m.dinv;
+            if (!fill_dinv) return NNX_OK;
+            if (h->pad) k_dinv_pad<<<kRedBlocks, 256, 0, c->stream>>>(gk, h->gp.nx, h->d.dinv);
+            else k_dinv<<<flat_blocks(h->n()), 256, 0, c->stream>>>(gk, h->d.dinv);
+            NNX_LAUNCHED(c);
+        } else {
+            h->d.dinv_c = gk.kind == 0 ? (float)(1.0 / gk.diagd) : (float)(1.0 / (gk.a0d + 128.0 * gk.wd));
+        }
+    }
+    return NNX_OK;
+}
+
+static nnx_status cg_buffers(nnx_ctx* c, const GridK& gk, int precond, const float* x, CgHost* h) {
+    CgMem m;
+    NNX_TRY(cg_mem_scratch(c, "cg", gk, precond, x, &m));
+    return cg_bind(c, gk, precond, x, m, h);
+}
+
+static nnx_status cg_readback(nnx_ctx* c, CgHost& h, int32_t* fl, double* sc) {
+    NNX_HIP(c, hipMemcpyAsync(c->pinned, h.d.fl, 4 * FL_N, hipMemcpyDeviceToHost, c->stream));
+    NNX_HIP(c, hipMemcpyAsync((char*)c->pinned + 64, h.d.sc, 8 * SC_N, hipMemcpyDeviceToHost, c->stream));
+    NNX_HIP(c, hipStreamSynchronize(c->stream));
+    std::memcpy(fl, c->pinned, 4 * FL_N);
+    std::memcpy(sc, (char*)c->pinned + 64, 8 * SC_N);
+    return NNX_OK;
+}
+
+// Iteration k of CG on the prepared buffers.  Constant 7-point stencil with
+// 16-byte rows and x (fast): the two halves of k_stencil7x4 (modes 2, 3),
+// the x update deferred by one iteration (k_cg_finish applies the last);
+// otherwise the new direction, q = A p, then the update of x and r.  Every
+// kernel returns at once when the device flag says the solve is over, so
+// iterations can be enqueued past convergence.
+static void cg_iter_launch(nnx_ctx* c, CgHost& h, int k, float* x, int xzero = 0) {
+    const GridK& gk = h.gp;
+    const int64_t n = h.n();
+    const int fast = h.fast, nb4 = h.nb4;
+    if (h.pad) x = h.xp;
+    float* pold = (k & 1) ? h.pb : h.pa;
+    float* pnew = (k & 1) ? h.pa : h.pb;
+    const CgShape& sh = h.sh;
+    if (fast == kFastVar) {
+        if (h.pad)
+            NNX_BY_LX(sh.lx, k_stencil7x4<2, 3, true, 4, false, LX, true, true>
+                      <<<nb4, 256, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, sh.zd));
+        else if (sh.lx == 0)
+            k_stencil7x4<2, kPFv, true, kTYv>
+                <<<nb4, 64 * kTYv, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, 0);
+        else
+            NNX_BY_LX(sh.lx, k_stencil7x4<2, 3, true, 4, false, LX, true>
+                      <<<nb4, 256, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, sh.zd));
+        k_cg_rupd<<<kRedBlocks, 256, 0, c->stream>>>(n, h.d, k);
+        return;
+    }
+    if (fast && gk.block) {
+        k_stencil7x4<2, kPFc, false, kTYc, true>
+            <<<nb4, 64 * kTYc, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, 0);
+        k_stencil7x4<3, kPFc, false, kTYc3, true>
+            <<<std::min(stencil4_blocks(gk, kTYc3), kRedBlocks), 64 * kTYc3, 0, c->stream>>>(
+                gk, h.d, k, pnew, nullptr, nullptr, nullptr, 0, 0);
+        return;
+    }
+    if (fast && sh.lx) {
+        NNX_BY_LX(sh.lx, k_stencil7x4<2, 3, false, 4, false, LX, true>
+                  <<<nb4, 256, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, sh.zd));
+        NNX_BY_LX(sh.lx, k_stencil7x4<3, 3, false, 4, false, LX, true>
+                  <<<std::min(nb4, kRedBlocks), 256, 0, c->stream>>>(gk, h.d, k, pnew, nullptr, nullptr, nullptr, 0,
+                                                                     sh.zd));
+        return;
+    }
+    if (fast) {
+        k_stencil7x4<2, kPFc, false, kTYc>
+            <<<nb4, 64 * kTYc, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, 0);
+        k_stencil7x4<3, kPFc, false, kTYc3>
+            <<<std::min(stencil4_blocks(gk, kTYc3), kRedBlocks), 64 * kTYc3, 0, c->stream>>>(
+                gk, h.d, k, pnew, nullptr, nullptr, nullptr, 0, 0);
+        return;
+    }
+    k_cg_dir<<<kRedBlocks, 256, 0, c->stream>>>(n, h.d, k, pold, pnew);
+    k_cg_spmv_gen<<<kRedBlocks, 256, 0, c->stream>>>(gk, h.d, k, pnew);
+    k_cg_update<<<kRedBlocks, 256, 0, c->stream>>>(n, h.d, k, pnew, x, (uintptr_t)x % 16 == 0);
+}
+
+// the pending x update of the fast path (nothing otherwise); padded rows:
+// the iterate into x
+static void cg_finish_launch(nnx_ctx* c, CgHost& h, float* x, int xzero = 0, double* acc = nullptr,
+                             int always = 1) {
+    if (h.pad)
+        k_cg_finish_pad<<<kRedBlocks, 256, 0, c->stream>>>(h.gp, h.d, h.pa, h.pb, h.xp, x, always);
+    else
+        k_cg_finish<<<flat_blocks(h.n() / 4), 256, 0, c->stream>>>(h.n(), h.d, h.pa, h.pb, x, xzero, acc);
+}
+
+static void cg_init_launch(nnx_ctx* c, const GridK& gk, CgHost& h, const float* b, float* x, int use_x0, double tol,
+                           int abs_mode, int maxit) {
+    if (h.pad)
+        k_cg_init_pad<<<kRedBlocks, 256, 0, c->stream>>>(gk, h.gp.nx, h.d, b, x, use_x0, h.pa, h.xp);
+    else
+        k_cg_init<<<kRedBlocks, 256, 0, c->stream>>>(gk, h.d, b, x, use_x0, h.pa);
+    k_cg_init_fin<<<1, 256, 0, c->stream>>>(h.d, tol, abs_mode, maxit);
 }
 
 // Runs CG on the prepared buffers; x holds the guess when use_x0.  The host
@@ -1296,28 +1446,21 @@ static void cg_finish_launch(nnx_ctx* c, const GridK& gk, CgHost& h, float* x, i
 static nnx_status cg_run(nnx_ctx* c, const GridK& gk, CgHost& h, const float* b, float* x,
                          int use_x0, double tol, int maxit, int abs_mode, int check_every,
                          nnx_cg_result* res, int* initdone = nullptr) {
-    k_cg_init<<<kRedBlocks, 256, 0, c->stream>>>(gk, h.d, b, x, use_x0, h.pa);
-    k_cg_init_fin<<<1, 256, 0, c->stream>>>(h.d, tol, abs_mode, maxit);
+    cg_init_launch(c, gk, h, b, x, use_x0, tol, abs_mode, maxit);
     NNX_LAUNCHED(c);
     if (check_every < 1) check_every = 1;
-    const int vec = ((uintptr_t)x % 16) == 0;
-    // 7-point grids with 16-byte rows: the LDS float4 kernels
-    const int fast = cg_fast(gk, x);
-    h.sh = cg_shape(gk, fast);
-    const int nb4 = fast_blocks(gk, fast, h.sh);
-    h.d.npq = fast ? nb4 : kRedBlocks;
     int32_t fl[FL_N];
     double sc[SC_N];
     NNX_TRY(cg_readback(c, h, fl, sc));
     if (initdone) *initdone = fl[FL_INITDONE];
     int enq = 0;
     while (!fl[FL_DONE] && enq < maxit) {
-        for (int q = 0; q < check_every && enq < maxit; ++q, ++enq) cg_iter_launch(c, gk, h, enq, x, vec, fast, nb4);
+        for (int q = 0; q < check_every && enq < maxit; ++q, ++enq) cg_iter_launch(c, h, enq, x);
         k_cg_status<<<1, 256, 0, c->stream>>>(h.d);
         NNX_LAUNCHED(c);
         NNX_TRY(cg_readback(c, h, fl, sc));
     }
-    cg_finish_launch(c, gk, h, x);
+    cg_finish_launch(c, h, x);
     NNX_LAUNCHED(c);
     if (res) {
         res->iters = fl[FL_ITERS];
@@ -1366,15 +1509,9 @@ __global__ __launch_bounds__(256) void k_cg_result(CgDev d, double* out) {
 // convergence are launched but return at once.
 static void cg_enqueue_fixed(nnx_ctx* c, const GridK& gk, CgHost& h, const float* b, float* x, int use_x0,
                              double tol, int maxit) {
-    k_cg_init<<<kRedBlocks, 256, 0, c->stream>>>(gk, h.d, b, x, use_x0, h.pa);
-    k_cg_init_fin<<<1, 256, 0, c->stream>>>(h.d, tol, 0, maxit);
-    const int vec = ((uintptr_t)x % 16) == 0;
-    const int fast = cg_fast(gk, x);
-    h.sh = cg_shape(gk, fast);
-    const int nb4 = fast_blocks(gk, fast, h.sh);
-    h.d.npq = fast ? nb4 : kRedBlocks;
-    for (int k = 0; k < maxit; ++k) cg_iter_launch(c, gk, h, k, x, vec, fast, nb4);
-    cg_finish_launch(c, gk, h, x);
+    cg_init_launch(c, gk, h, b, x, use_x0, tol, 0, maxit);
+    for (int k = 0; k < maxit; ++k) cg_iter_launch(c, h, k, x);
+    cg_finish_launch(c, h, x);
 }
 
 // The paracrine solve of a timestep (nnx_paracrine): rhs, then max_outer
@@ -1401,17 +1538,21 @@ __global__ __launch_bounds__(256) void k_para_rhs(int64_t n, const double* __res
 // r = b - A x in FP64 (partials of ||r||^2); unless FINAL also the inner
 // CG's start on r32 = (float) r: residual r32, correction 0, p0 = 0, and
 // the partials k_cg_init would leave.
+// The inner CG's vectors are in rows of px >= nx voxels, zero beyond nx.
 template <bool FINAL>
-__global__ __launch_bounds__(256) void k_para_res(GridK g, const double* __restrict__ x, const double* __restrict__ b,
-                                                  CgDev d, float* __restrict__ xin, float* __restrict__ p0,
-                                                  double* prr, const int32_t* __restrict__ pfl) {
+__global__ __launch_bounds__(256) void k_para_res(GridK g, int px, const double* __restrict__ x,
+                                                  const double* __restrict__ b, CgDev d, float* __restrict__ xin,
+                                                  float* __restrict__ p0, double* prr, const int32_t* __restrict__ pfl) {
     if (pfl[0]) return;
     double vr[1] = {0}, vb[1] = {0}, vu[2] = {0, 0};
-    for_rows(g.nx, g.ny, g.nz, [&](int i, int j, int k, int64_t id) {
-        const double r = b[id] - apply_at<double, double>(x, g, i, j, k);
-        vr[0] += r * r;
+    for_rows(px, g.ny, g.nz, [&](int i, int j, int k, int64_t id) {
+        float r32 = 0.0f;
+        if (i < g.nx) {
+            const double r = b[i + (int64_t)g.nx * (j + (int64_t)g.ny * k)] - apply_at<double, double>(x, g, i, j, k);
+            vr[0] += r * r;
+            r32 = (float)r;
+        }
         if (!FINAL) {
-            const float r32 = (float)r;
             d.r[id] = r32;
             xin[id] = 0.0f;
             p0[id] = 0.0f;
@@ -1755,7 +1896,7 @@ nnx_status nnx_cg_solve(nnx_ctx* c, const nnx_grid* g, const float* b, float* x,
     const GridK gk = make_grid(g);
     auto t0 = std::chrono::steady_clock::now();
     CgHost h;
-    NNX_TRY(cg_buffers(c, gk, o->precond, &h));
+    NNX_TRY(cg_buffers(c, gk, o->precond, x, &h));
     nnx_cg_result r{};
     NNX_TRY(cg_run(c, gk, h, b, x, o->use_x0, o->rtol, o->maxit, 0, o->check_every, &r));
     auto t1 = std::chrono::steady_clock::now();
@@ -1775,12 +1916,12 @@ nnx_status nnx_cg_solve_refine(nnx_ctx* c, const nnx_grid* g, const double* b, d
     const GridK gk = make_grid(g);
     const int64_t n = (int64_t)gk.nx * gk.ny * gk.nz;
     auto t0 = std::chrono::steady_clock::now();
-    CgHost h;
-    NNX_TRY(cg_buffers(c, gk, o->precond, &h));
     void *r64, *rhs, *d;
     NNX_TRY(scratch(c, "ir_r64", n * 8, false, &r64));
     NNX_TRY(scratch(c, "ir_rhs", n * 4, false, &rhs));
     NNX_TRY(scratch(c, "ir_d", n * 4, false, &d));
+    CgHost h;
+    NNX_TRY(cg_buffers(c, gk, o->precond, (const float*)d, &h));
     if (!o->use_x0) NNX_HIP(c, hipMemsetAsync(x, 0, n * 8, c->stream));
     nnx_cg_result out{};
     int outer = 0, inner_total = 0;
@@ -1843,12 +1984,12 @@ nnx_status para_check(nnx_ctx* c, const ParaIo& io) {
 
 static nnx_status para_host(nnx_ctx* c, const nnx_paracrine& q, const GridK& gk, ParaHost* ph) {
     const int64_t n = (int64_t)gk.nx * gk.ny * gk.nz;
-    CgMem m;
-    NNX_TRY(cg_mem_scratch(c, "para", gk, NNX_PRECOND_JACOBI, &m));
     void *b, *xin, *fl;
     NNX_TRY(scratch(c, "para_b", (size_t)n * 8, false, &b));
     NNX_TRY(scratch(c, "para_xin", (size_t)n * 4, false, &xin));
     NNX_TRY(scratch(c, "para_pfl", 64, true, &fl));
+    CgMem m;
+    NNX_TRY(cg_mem_scratch(c, "para", gk, NNX_PRECOND_JACOBI, (const float*)xin, &m));
     ph->b = (double*)b;
     ph->xin = (float*)xin;
     ph->pfl = (int32_t*)fl;
@@ -1864,16 +2005,13 @@ static nnx_status para_host(nnx_ctx* c, const nnx_paracrine& q, const GridK& gk,
         tag |= 1;
         if (bd.tag != tag) {
             NNX_CHECK(c, !c->capturing, "paracrine: grid changed during capture");
-            NNX_TRY(cg_bind(c, gk, NNX_PRECOND_JACOBI, m, &ph->h));
+            NNX_TRY(cg_bind(c, gk, NNX_PRECOND_JACOBI, ph->xin, m, &ph->h));
             bd.tag = tag;
             return NNX_OK;
         }
-        m.dinv = nullptr;  // already filled: bind without relaunching
-        NNX_TRY(cg_bind(c, gk, NNX_PRECOND_NONE, m, &ph->h));
-        ph->h.d.dinv = (float*)bd.p;
-        return NNX_OK;
+        return cg_bind(c, gk, NNX_PRECOND_JACOBI, ph->xin, m, &ph->h, false);
     }
-    return cg_bind(c, gk, NNX_PRECOND_JACOBI, m, &ph->h);
+    return cg_bind(c, gk, NNX_PRECOND_JACOBI, ph->xin, m, &ph->h);
 }
 
 nnx_status para_prepare(nnx_ctx* c, const ParaIo& io) {
@@ -1898,11 +2036,8 @@ nnx_status para_launch(nnx_ctx* c, const ParaIo& io) {
     // 16-byte aligned vectors); on the constant grid also the tiled FP64
     // residual, after which the inner CG starts from a zero correction
     // without storing it and its last update goes straight into the field
-    const int fast = cg_fast(gk, ph.xin);
-    const bool tiled = fast == kFastConst && (uintptr_t)q.conc % 16 == 0;
-    h.sh = cg_shape(gk, fast);
-    const int nb4 = fast_blocks(gk, fast, h.sh), nbr = std::min(stencil4_blocks(gk), kRedBlocks);
-    h.d.npq = fast ? nb4 : kRedBlocks;
+    const bool tiled = h.fast == kFastConst && !h.pad && (uintptr_t)q.conc % 16 == 0;
+    const int nbr = std::min(stencil4_blocks(gk), kRedBlocks);
     k_para_rhs<<<kRedBlocks, 256, 0, c->stream>>>(nv, q.conc, io.voxel_counts, q.release, ph.b, ph.pbb, ph.pfl);
     for (int o = 0; o < max_outer; ++o) {
         // the later refinement steps solve to a looser tolerance: half the budget
@@ -1912,15 +2047,15 @@ nnx_status para_launch(nnx_ctx* c, const ParaIo& io) {
         else if (tiled)
             k_res64x4<false><<<nbr, kT4, 0, c->stream>>>(gk, q.conc, ph.b, h.d, ph.prr, ph.pfl);
         else
-            k_para_res<false><<<kRedBlocks, 256, 0, c->stream>>>(gk, q.conc, ph.b, h.d, ph.xin, h.pa, ph.prr,
-                                                                 ph.pfl);
+            k_para_res<false><<<kRedBlocks, 256, 0, c->stream>>>(gk, h.gp.nx, q.conc, ph.b, h.d,
+                                                                 h.pad ? h.xp : ph.xin, h.pa, ph.prr, ph.pfl);
         k_para_ctl<<<1, 256, 0, c->stream>>>(h.d, ph.prr, ph.pbb, q.rtol, inner_rtol, budget, ph.pfl, q.stats, 0,
                                              o > 0);
-        for (int k = 0; k < budget; ++k) cg_iter_launch(c, gk, h, k, ph.xin, 1, fast, nb4, tiled);
+        for (int k = 0; k < budget; ++k) cg_iter_launch(c, h, k, ph.xin, tiled);
         if (tiled) {
-            cg_finish_launch(c, gk, h, ph.xin, 1, q.conc);
+            cg_finish_launch(c, h, ph.xin, 1, q.conc);
         } else {
-            cg_finish_launch(c, gk, h, ph.xin);
+            cg_finish_launch(c, h, ph.xin, 0, nullptr, 0);
             k_para_axpy<<<flat_blocks(nv), 256, 0, c->stream>>>(nv, ph.xin, q.conc, h.d.fl, ph.pfl);
         }
     }
@@ -1929,7 +2064,7 @@ nnx_status para_launch(nnx_ctx* c, const ParaIo& io) {
     else if (tiled)
         k_res64x4<true><<<nbr, kT4, 0, c->stream>>>(gk, q.conc, ph.b, h.d, ph.prr, ph.pfl);
     else
-        k_para_res<true><<<kRedBlocks, 256, 0, c->stream>>>(gk, q.conc, ph.b, h.d, ph.xin, h.pa, ph.prr, ph.pfl);
+        k_para_res<true><<<kRedBlocks, 256, 0, c->stream>>>(gk, gk.nx, q.conc, ph.b, h.d, ph.xin, h.pa, ph.prr, ph.pfl);
     k_para_ctl<<<1, 256, 0, c->stream>>>(h.d, ph.prr, ph.pbb, q.rtol, inner_rtol, max_inner, ph.pfl, q.stats, 1,
                                          max_outer > 0);
     if (q.at_neurons)
@@ -1954,7 +2089,7 @@ nnx_status nnx::cg_async_launch(nnx_ctx* c, const nnx_grid* g, const float* b, f
                                 double* d_result, const CgMem& m) {
     const GridK gk = make_grid(g);
     CgHost h;
-    NNX_TRY(cg_bind(c, gk, o->precond, m, &h));
+    NNX_TRY(cg_bind(c, gk, o->precond, x, m, &h));
     cg_enqueue_fixed(c, gk, h, b, x, o->use_x0, o->rtol, o->maxit);
     k_cg_result<<<1, 256, 0, c->stream>>>(h.d, d_result);
     NNX_LAUNCHED(c);
@@ -1967,7 +2102,7 @@ extern "C" nnx_status nnx_cg_solve_async(nnx_ctx* c, const nnx_grid* g, const fl
     NNX_TRY(cg_async_check(c, g, b, x, o, d_result));
     const GridK gk = make_grid(g);
     CgMem m;
-    NNX_TRY(cg_mem_scratch(c, "cga", gk, o->precond, &m));
+    NNX_TRY(cg_mem_scratch(c, "cga", gk, o->precond, x, &m));
     return cg_async_launch(c, g, b, x, o, d_result, m);
 }
 
@@ -2135,7 +2270,7 @@ nnx_status nnx_fcg_solve(nnx_ctx* c, const nnx_grid* g, nnx_unet* net, const flo
                     o->smooth, &r));
     auto t1 = std::chrono::steady_clock::now();
     CgHost h;
-    NNX_TRY(cg_buffers(c, gk, NNX_PRECOND_NONE, &h));
+    NNX_TRY(cg_buffers(c, gk, NNX_PRECOND_NONE, nullptr, &h));
     NNX_TRY((true_residual<float, float>(c, gk, h, x, b, &r.true_relres, nullptr, nullptr)));
     r.ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
     if (res) *res = r;
@@ -2153,7 +2288,7 @@ nnx_status nnx_fcg_solve_refine(nnx_ctx* c, const nnx_grid* g, nnx_unet* net, co
     const int64_t n = (int64_t)gk.nx * gk.ny * gk.nz;
     auto t0 = std::chrono::steady_clock::now();
     CgHost h;
-    NNX_TRY(cg_buffers(c, gk, NNX_PRECOND_NONE, &h));
+    NNX_TRY(cg_buffers(c, gk, NNX_PRECOND_NONE, nullptr, &h));
     void *r64, *rhs, *d;
     NNX_TRY(scratch(c, "ir_r64", n * 8, false, &r64));
     NNX_TRY(scratch(c, "ir_rhs", n * 4, false, &rhs));
@@ -2208,10 +2343,10 @@ nnx_status nnx_update_density_reference(nnx_ctx* c, int nx, int ny, int nz, doub
     const int64_t n = (int64_t)nx * ny * nz;
     auto t0 = std::chrono::steady_clock::now();
     CgHost hh;
-    NNX_TRY(cg_buffers(c, gk, NNX_PRECOND_NONE, &hh));
     void *xg, *bb;
     NNX_TRY(scratch(c, "ref_xg", n * 4, false, &xg));
     NNX_TRY(scratch(c, "ref_b", n * 4, false, &bb));
+    NNX_TRY(cg_buffers(c, gk, NNX_PRECOND_NONE, (const float*)xg, &hh));
     k_ref_init<<<grid3(gk), 256, 0, c->stream>>>(gk, data, (float)(1.0 / (h * h * 30.0)),
                                                  (float)(1.0 - dt * k), (float)(dt * D),
                                                  (float)(1.0 - h * k / 2.0), (float)(h * D / 2.0),
