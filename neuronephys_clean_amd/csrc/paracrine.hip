@@ -256,7 +256,7 @@ __global__ __launch_bounds__(256) void k_cg_status(CgDev d) {
 // raw values are loaded two planes ahead at clamped addresses, with no
 // arithmetic and no condition at the load, and finished one step later.
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // 16 bytes at a 4-byte address
-constexpr int kTX4 = 256, kTY4 = 16, kZ4 = 16, kT4 = 64 * kTY4, kRow4 = kTX4 + 8;
+constexpr int kTX4 = 256, kTY4 = 16, kZ4 = 16, kT4 = 64 * kTY4;
 // prefetch forms and tile heights the solver launches (measured at 256^3):
 // the apply and the variable-coefficient first half take the deferred form;
 // the constant-coefficient iteration on 1024-thread tiles stays at PF 2 (the deferred form for
@@ -728,17 +728,18 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
 // 7-point fast path (k_stencil7x4 modes 2 and 3); nothing when none is
 // pending.  p_k is in pa for odd k, pb for even k.  xzero: the solve started
 // from x = 0 without storing it, so after one iteration x = alpha_0 p_0.
-// acc: instead of storing x, acc += (double) x (the refinement's correction
-// added to its FP64 iterate).
+// acc: instead of storing x, acc += scale (double) x (the refinement's
+// correction added to its FP64 iterate).
 __global__ __launch_bounds__(256) void k_cg_finish(int64_t n, CgDev d, const float* __restrict__ pa,
                                                    const float* __restrict__ pb, float* __restrict__ x, int xzero,
-                                                   double* __restrict__ acc) {
+                                                   double* __restrict__ acc, double scale) {
     if (!d.fl[FL_XPEND]) return;
     const int k = d.fl[FL_ITERS] - 1;
     const bool read_x = !(xzero && k == 0);
     const float alpha = (float)d.sc[SC_ALK + (k & 1)];  // stored by iteration k's second half
     const float* __restrict__ p = (k & 1) ? pa : pb;
     const int64_t n4 = n / 4, stride = (int64_t)gridDim.x * 256;
+    const bool a16 = ((uintptr_t)acc & 15) == 0;
     for (int64_t c = blockIdx.x * 256ll + threadIdx.x; c < n4; c += stride) {
         const float4 xv = read_x ? reinterpret_cast<const float4*>(x)[c] : make_float4(0.f, 0.f, 0.f, 0.f);
         const float4 pv = reinterpret_cast<const float4*>(p)[c];
@@ -747,15 +748,21 @@ __global__ __launch_bounds__(256) void k_cg_finish(int64_t n, CgDev d, const flo
         xo.y = xv.y + alpha * pv.y;
         xo.z = xv.z + alpha * pv.z;
         xo.w = xv.w + alpha * pv.w;
-        if (acc) {
+        if (acc && a16) {
             double2* a2 = reinterpret_cast<double2*>(acc) + 2 * c;
             double2 lo = a2[0], hi = a2[1];
-            lo.x = lo.x + (double)xo.x;
-            lo.y = lo.y + (double)xo.y;
-            hi.x = hi.x + (double)xo.z;
-            hi.y = hi.y + (double)xo.w;
+            lo.x = lo.x + scale * (double)xo.x;
+            lo.y = lo.y + scale * (double)xo.y;
+            hi.x = hi.x + scale * (double)xo.z;
+            hi.y = hi.y + scale * (double)xo.w;
             a2[0] = lo;
             a2[1] = hi;
+        } else if (acc) {
+            double* a = acc + 4 * c;
+            a[0] = a[0] + scale * (double)xo.x;
+            a[1] = a[1] + scale * (double)xo.y;
+            a[2] = a[2] + scale * (double)xo.z;
+            a[3] = a[3] + scale * (double)xo.w;
         } else {
             reinterpret_cast<float4*>(x)[c] = xo;
         }
@@ -807,38 +814,53 @@ __global__ __launch_bounds__(256) void k_cg_rupd(int64_t n, CgDev d, int k) {
 }
 
 // The FP64 residual of the refinement on the constant 7-point grid, tiled
-// as k_stencil7x4: r = b - A x, A x in the operation order of
-// apply_at<double, double>, and the partials of ||r||^2; unless FINAL also
-// the inner CG's start on r32 = (float) r - residual r32 and the partials
-// k_cg_init would leave (the inner CG's direction and iterate start from
-// zero without being stored: k_stencil7x4 and k_cg_finish with xzero).
-// 20 B per voxel (16 when FINAL).  Launched with at most kRedBlocks
-// workgroups; block 0 zeroes the partial slots beyond them.
-template <bool FINAL, bool BLK = false>
-__global__ __launch_bounds__(kT4) void k_res64x4(GridK g, const double* __restrict__ x,
-                                                 const double* __restrict__ b, CgDev d, double* prr,
-                                                 const int32_t* __restrict__ pfl) {
-    if (pfl[0]) return;
-    __shared__ double t[2][kTY4 + 2][kRow4];
-    const int nx = g.nx, ny = g.ny, nz = g.nz;
-    const int tx = (nx + kTX4 - 1) / kTX4, ty = (ny + kTY4 - 1) / kTY4, tz = (nz + kZ4 - 1) / kZ4;
+// as k_stencil7x4 (TY, LX, DYN, zdyn alike): r = b - A x, A x in the operation
+// order of apply_at<double, double>.
+//   OUT 0: the in-step solve - the partials of ||r||^2, and the inner CG's
+//          start on r32 = (float) r: residual r32 and the partials k_cg_init
+//          would leave (the inner CG's direction and iterate start from zero
+//          without being stored: k_stencil7x4 and k_cg_finish with xzero).
+//          20 B per voxel.  Returns at once when pfl says the solve is over.
+//   OUT 1: its final check, the partials of ||r||^2 only.  16 B.
+//   OUT 2: r stored in FP64, partials of (||r||^2, ||b||^2).  24 B.
+// RAG: x, b and r64 in rows of nxr voxels at 8-byte alignment, r32 in padded
+// rows of nx.  Launched with at most kRedBlocks workgroups; block 0 zeroes the
+// partial slots beyond them.  Bound by HBM: OUT 0 64 us at 256^3 (16-row tiles
+// of 1024 threads; 223 as rows through the cache); on small grids by a latency
+// per plane, hence tile_shape.
+template <int OUT, bool BLK = false, int TY = kTY4, int LX = 64, bool DYN = false, bool RAG = false>
+__global__ __launch_bounds__(64 * TY) void k_res64x4(GridK g, const double* __restrict__ x,
+                                                     const double* __restrict__ b, CgDev d, double* prr,
+                                                     const int32_t* __restrict__ pfl, double* __restrict__ r64,
+                                                     int zdyn) {
+    if (OUT != 2 && pfl[0]) return;
+    constexpr int R = 64 * TY / LX, kTXs = 4 * LX;
+    const int kZs = DYN ? zdyn : kZ4;
+    __shared__ double t[2][R + 2][kTXs + 8];
+    const int nx = g.nx, ny = g.ny, nz = g.nz, nr = RAG ? g.nxr : g.nx;
+    const int tx = (nx + kTXs - 1) / kTXs, ty = (ny + R - 1) / R, tz = (nz + kZs - 1) / kZs;
     const int ntiles = tx * ty * tz;
-    const int64_t sxy = (int64_t)nx * ny;
-    const int tt = threadIdx.x, lx = tt & 63, ly = tt >> 6;
-    const bool hrow = tt < 128, hcol = tt >= 128 && tt < 128 + 2 * kTY4;
-    const int hy = tt < 64 ? -1 : tt < 128 ? kTY4 : (tt < 128 + kTY4 ? tt - 128 : tt - 128 - kTY4);
-    const int hl = tt < 64 ? tt : tt - 64;
-    const int hslot = tt < 128 + kTY4 ? 3 : 4 + kTX4;
+    const int64_t sxy = (int64_t)nr * ny;
+    const int tt = threadIdx.x, lx = tt & (LX - 1), ly = tt / LX;
+    const bool hrow = tt < 2 * LX, hcol = tt >= 2 * LX && tt < 2 * LX + 2 * R;
+    const int hy = tt < LX ? -1 : tt < 2 * LX ? R : (tt < 2 * LX + R ? tt - 2 * LX : tt - 2 * LX - R);
+    const int hl = tt < LX ? tt : tt - LX;
+    const int hslot = tt < 2 * LX + R ? 3 : 4 + kTXs;
     const double cdiag = g.diagd, cc = g.cd;
     const float di = d.dinv_c;
     const int blk = BLK ? g.block : 0;
-    // (||r32||^2 is both the inner CG's bb and its first rr)
-    double vr[1] = {0}, vu[2] = {0, 0};
+    // OUT 0: ||r32||^2 (vu[1]) is both the inner CG's bb and its first rr
+    double vr[2] = {0, 0}, vu[2] = {0, 0};
     struct D4 {
         double x, y, z, w;
     };
-    auto ld4 = [&](bool ok, const double* p) -> D4 {
+    // the four values from p on, `in` of them inside the row (RAG), zeros beyond
+    auto ld4 = [&](bool ok, const double* p, int in) -> D4 {
         if (!ok) return D4{0, 0, 0, 0};
+        if (RAG) {
+            const double v1 = p[in > 1 ? 1 : 0], v2 = p[in > 2 ? 2 : 0], v3 = p[in > 3 ? 3 : 0];
+            return D4{p[0], in > 1 ? v1 : 0, in > 2 ? v2 : 0, in > 3 ? v3 : 0};
+        }
         const double2 a = reinterpret_cast<const double2*>(p)[0], c2 = reinterpret_cast<const double2*>(p)[1];
         return D4{a.x, a.y, c2.x, c2.y};
     };
@@ -850,30 +872,32 @@ __global__ __launch_bounds__(kT4) void k_res64x4(GridK g, const double* __restri
         const int tile = xcd_tile(blockIdx.x, round, gridDim.x);
         if (tile >= ntiles) break;
         const int bx = tile % tx, by = (tile / tx) % ty, bz = tile / (tx * ty);
-        const int x0 = bx * kTX4, k0 = bz * kZ4, kend = min(k0 + kZ4, nz);
-        const int j = by * kTY4 + ly;
+        const int x0 = bx * kTXs, k0 = bz * kZs, kend = min(k0 + kZs, nz);
+        const int j = by * R + ly;
         const int xo = x0 + 4 * lx;
         const bool own = xo < nx && j < ny;
-        const int gj = by * kTY4 + hy;
-        const bool hr_ok = hrow && gj >= 0 && gj < ny && x0 + 4 * hl < nx;
-        const int hx = tt < 128 + kTY4 ? x0 - 1 : x0 + kTX4;
-        const bool hc_ok = hcol && gj < ny && hx >= 0 && hx < nx;
-        const int64_t ocol = xo + (int64_t)nx * j;
-        const int64_t rcol = x0 + 4 * hl + (int64_t)nx * gj;
-        const int64_t ccol = hx + (int64_t)nx * gj;
+        const int gj = by * R + hy;
+        const int xh = x0 + 4 * hl;
+        const bool hr_ok = hrow && gj >= 0 && gj < ny && xh < nx;
+        const int hx = tt < 2 * LX + R ? x0 - 1 : x0 + kTXs;
+        const bool hc_ok = hcol && gj < ny && hx >= 0 && hx < nr;
+        const int in_o = nr - xo, in_h = nr - xh;
+        const int64_t ocol = xo + (int64_t)nr * j;
+        const int64_t rcol = xh + (int64_t)nr * gj;
+        const int64_t ccol = hx + (int64_t)nr * gj;
         const bool cut_xm = blk && xo % blk == 0, cut_xp = blk && (xo + 4) % blk == 0;
         const bool cut_ym = blk && j % blk == 0, cut_yp = blk && (j + 1) % blk == 0;
-        D4 pm = ld4(own && k0 > 0, x + ocol + sxy * (k0 - 1));
-        D4 pc = ld4(own, x + ocol + sxy * k0);
+        D4 pm = ld4(own && k0 > 0, x + ocol + sxy * (k0 - 1), in_o);
+        D4 pc = ld4(own, x + ocol + sxy * k0, in_o);
         st4(&t[0][ly + 1][4 + 4 * lx], pc);
-        if (hrow) st4(&t[0][hy + 1][4 + 4 * hl], ld4(hr_ok, x + rcol + sxy * k0));
+        if (hrow) st4(&t[0][hy + 1][4 + 4 * hl], ld4(hr_ok, x + rcol + sxy * k0, in_h));
         if (hcol) t[0][hy + 1][hslot] = hc_ok ? x[ccol + sxy * k0] : 0.0;
         auto plane = [&](int kz) {
             const int bf = (kz - k0) & 1;
             const bool nxt = kz + 1 < nz;
-            const D4 pp = ld4(own && nxt, x + ocol + sxy * (kz + 1));
-            const D4 bc = ld4(own, b + ocol + sxy * kz);
-            const D4 hr = ld4(hr_ok && nxt, x + rcol + sxy * (kz + 1));
+            const D4 pp = ld4(own && nxt, x + ocol + sxy * (kz + 1), in_o);
+            const D4 bc = ld4(own, b + ocol + sxy * kz, in_o);
+            const D4 hr = ld4(hr_ok && nxt, x + rcol + sxy * (kz + 1), in_h);
             const double hc = hc_ok && nxt ? x[ccol + sxy * (kz + 1)] : 0.0;
             __syncthreads();
             if (own) {
@@ -895,12 +919,18 @@ __global__ __launch_bounds__(kT4) void k_res64x4(GridK g, const double* __restri
                     s = s + (cut_yp ? 0.0 : yp[q]);
                     s = s + (cz_m ? 0.0 : ms[q]);
                     s = s + (cz_p ? 0.0 : ps[q]);
-                    const double r = bs[q] - (cdiag * xs[q + 1] - cc * s);
+                    double r = bs[q] - (cdiag * xs[q + 1] - cc * s);
+                    if (RAG && q >= in_o) r = 0.0;
                     vr[0] += r * r;
+                    if (OUT == 2) {
+                        vr[1] += bs[q] * bs[q];
+                        if (!RAG || q < in_o) r64[ocol + sxy * kz + q] = r;
+                    }
                     r32[q] = (float)r;
                 }
-                if (!FINAL) {
-                    *reinterpret_cast<float4*>(d.r + ocol + sxy * kz) = make_float4(r32[0], r32[1], r32[2], r32[3]);
+                if (OUT == 0) {
+                    *reinterpret_cast<float4*>(d.r + xo + (int64_t)nx * (j + (int64_t)ny * kz)) =
+                        make_float4(r32[0], r32[1], r32[2], r32[3]);
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
                         vu[0] += (double)r32[q] * (r32[q] * di);
@@ -914,7 +944,7 @@ __global__ __launch_bounds__(kT4) void k_res64x4(GridK g, const double* __restri
             pm = pc;
             pc = pp;
         };
-        if (kend - k0 == kZ4) {
+        if (!DYN && kend - k0 == kZ4) {
 #pragma unroll
             for (int q = 0; q < kZ4; ++q) plane(k0 + q);
         } else {
@@ -922,15 +952,20 @@ __global__ __launch_bounds__(kT4) void k_res64x4(GridK g, const double* __restri
         }
         __syncthreads();
     }
-    put_partial<1>(vr, prr);
-    if (!FINAL) {
+    constexpr int NV = OUT == 2 ? 2 : 1;
+    double vo[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) vo[q] = vr[q];
+    put_partial<NV>(vo, prr);
+    if (OUT == 0) {
         put_partial<2>(vu, d.pu0);
         if (threadIdx.x == 0) d.pb[blockIdx.x] = vu[1];
     }
     if (blockIdx.x == 0)
         for (int i = (int)gridDim.x + (int)threadIdx.x; i < kRedBlocks; i += (int)blockDim.x) {
-            prr[i] = 0.0;
-            if (!FINAL) {
+#pragma unroll
+            for (int q = 0; q < NV; ++q) prr[NV * i + q] = 0.0;
+            if (OUT == 0) {
                 d.pb[i] = 0.0;
                 d.pu0[2 * i] = 0.0;
                 d.pu0[2 * i + 1] = 0.0;
@@ -1067,18 +1102,43 @@ __global__ __launch_bounds__(256) void k_cg_init_pad(GridK g, int px, CgDev d, c
     put_partial<2>(vu, d.pu0);
 }
 // x = xp + the deferred alpha_k p_k of the last executed iteration (without
-// one: x = xp, or nothing unless `always`)
+// one: x = xp); acc: acc += scale times that instead (nothing without one);
+// xzero as in k_cg_finish
 __global__ __launch_bounds__(256) void k_cg_finish_pad(GridK g, CgDev d, const float* __restrict__ pa,
                                                        const float* __restrict__ pb, const float* __restrict__ xp,
-                                                       float* __restrict__ x, int always) {
+                                                       float* __restrict__ x, int xzero, double* __restrict__ acc,
+                                                       double scale) {
     const bool pend = d.fl[FL_XPEND] != 0;
-    if (!pend && !always) return;
+    if (!pend && acc) return;
     const int k = d.fl[FL_ITERS] - 1;
+    const bool read_x = !(xzero && k == 0);
     const float alpha = pend ? (float)d.sc[SC_ALK + (k & 1)] : 0.0f;
     const float* __restrict__ p = (k & 1) ? pa : pb;
     for_rows(g.nx, g.ny, g.nz, [&](int i, int j, int kk, int64_t id) {
-        if (i < g.nxr) x[i + (int64_t)g.nxr * (j + (int64_t)g.ny * kk)] = pend ? xp[id] + alpha * p[id] : xp[id];
+        if (i >= g.nxr) return;
+        const int64_t e = i + (int64_t)g.nxr * (j + (int64_t)g.ny * kk);
+        const float xv = read_x ? xp[id] : 0.0f;
+        const float xo = pend ? xv + alpha * p[id] : xv;
+        if (acc) acc[e] = acc[e] + scale * (double)xo;
+        else x[e] = xo;
     });
+}
+
+// The refinement's inner CG from the FP64 residual: r = (float)(s r64) in rows
+// of px >= nx voxels (zero beyond nx), and the partials k_cg_init would leave
+// on that right-hand side from a zero guess; the direction and the iterate
+// start from zero without being stored (xzero).  12 B per voxel.
+__global__ __launch_bounds__(256) void k_cg_init64(GridK g, int px, CgDev d, const double* __restrict__ r64,
+                                                   double s) {
+    double vu[2] = {0, 0};
+    for_rows(px, g.ny, g.nz, [&](int i, int j, int k, int64_t id) {
+        const float ri = i < g.nx ? (float)(r64[i + (int64_t)g.nx * (j + (int64_t)g.ny * k)] * s) : 0.0f;
+        d.r[id] = ri;
+        vu[0] += (double)ri * (ri * dv(d, id));
+        vu[1] += (double)ri * ri;
+    });
+    put_partial<2>(vu, d.pu0);
+    if (threadIdx.x == 0) d.pb[blockIdx.x] = vu[1];
 }
 
 // ||b - A x||^2 and ||b||^2 in FP64 (x float or double): partials, then one
@@ -1087,15 +1147,13 @@ template <class U, class B>
 __global__ __launch_bounds__(256) void k_true_res(GridK g, const U* __restrict__ x,
                                                   const B* __restrict__ b, double* part,
                                                   double* __restrict__ r_out) {
-    const int64_t n = (int64_t)g.nx * g.ny * g.nz;
     double v[2] = {0, 0};
-    for (int64_t id = blockIdx.x * 256ll + threadIdx.x; id < n; id += (int64_t)gridDim.x * 256) {
-        const int i = (int)(id % g.nx), j = (int)((id / g.nx) % g.ny), k = (int)(id / ((int64_t)g.nx * g.ny));
-        const double r = (double)b[id] - apply_at<double, U>(x, g, i, j, k);
+    for_rows(g.nx, g.ny, g.nz, [&](int i, int j, int k, int64_t id) {
+        const double bi = (double)b[id], r = bi - apply_at<double, U>(x, g, i, j, k);
         if (r_out) r_out[id] = r;
         v[0] += r * r;
-        v[1] += (double)b[id] * (double)b[id];
-    }
+        v[1] += bi * bi;
+    });
     put_partial<2>(v, part);
 }
 __global__ __launch_bounds__(256) void k_sum2(const double* part, double* out2) {
@@ -1422,14 +1480,41 @@ static void cg_iter_launch(nnx_ctx* c, CgHost& h, int k, float* x, int xzero = 0
     k_cg_update<<<kRedBlocks, 256, 0, c->stream>>>(n, h.d, k, pnew, x, (uintptr_t)x % 16 == 0);
 }
 
-// the pending x update of the fast path (nothing otherwise); padded rows:
-// the iterate into x
+// the pending x update of the fast path (nothing otherwise; padded rows: the
+// iterate into x); acc: the iterate times scale added to acc instead
 static void cg_finish_launch(nnx_ctx* c, CgHost& h, float* x, int xzero = 0, double* acc = nullptr,
-                             int always = 1) {
+                             double scale = 1.0) {
     if (h.pad)
-        k_cg_finish_pad<<<kRedBlocks, 256, 0, c->stream>>>(h.gp, h.d, h.pa, h.pb, h.xp, x, always);
+        k_cg_finish_pad<<<kRedBlocks, 256, 0, c->stream>>>(h.gp, h.d, h.pa, h.pb, h.xp, x, xzero, acc, scale);
     else
-        k_cg_finish<<<flat_blocks(h.n() / 4), 256, 0, c->stream>>>(h.n(), h.d, h.pa, h.pb, x, xzero, acc);
+        k_cg_finish<<<flat_blocks(h.n() / 4), 256, 0, c->stream>>>(h.n(), h.d, h.pa, h.pb, x, xzero, acc, scale);
+}
+
+// the tiled FP64 residual on the constant 7-point grid of h (res64_ok: a
+// block lattice on vectors off the 16-byte grid keeps the generic passes)
+static bool res64_ok(const CgHost& h, const double* x, const double* b) {
+    return h.fast == kFastConst && (!h.gp.block || ((uintptr_t)x | (uintptr_t)b) % 16 == 0);
+}
+template <int OUT>
+static void res64_launch(nnx_ctx* c, const CgHost& h, const double* x, const double* b, double* prr,
+                         const int32_t* pfl, double* r64) {
+    const GridK& gp = h.gp;
+    if (gp.block) {
+        k_res64x4<OUT, true><<<std::min(stencil4_blocks(gp), kRedBlocks), kT4, 0, c->stream>>>(gp, x, b, h.d, prr, pfl,
+                                                                                           r64, 0);
+        return;
+    }
+    const CgShape sh = h.sh.lx ? h.sh : CgShape{64, 16};
+    const int nb = std::min(fast_blocks(gp, kFastConst, sh), kRedBlocks);
+    if (gp.nx != gp.nxr || ((uintptr_t)x | (uintptr_t)b | (uintptr_t)r64) % 16 != 0)
+        NNX_BY_LX(sh.lx, k_res64x4<OUT, false, 4, LX, true, true>
+                  <<<nb, 256, 0, c->stream>>>(gp, x, b, h.d, prr, pfl, r64, sh.zd));
+    else if (h.sh.lx)
+        NNX_BY_LX(sh.lx, k_res64x4<OUT, false, 4, LX, true>
+                  <<<nb, 256, 0, c->stream>>>(gp, x, b, h.d, prr, pfl, r64, sh.zd));
+    else
+        k_res64x4<OUT><<<std::min(stencil4_blocks(gp), kRedBlocks), kT4, 0, c->stream>>>(gp, x, b, h.d, prr, pfl, r64,
+                                                                                     0);
 }
 
 static void cg_init_launch(nnx_ctx* c, const GridK& gk, CgHost& h, const float* b, float* x, int use_x0, double tol,
@@ -1441,25 +1526,31 @@ static void cg_init_launch(nnx_ctx* c, const GridK& gk, CgHost& h, const float* 
     k_cg_init_fin<<<1, 256, 0, c->stream>>>(h.d, tol, abs_mode, maxit);
 }
 
-// Runs CG on the prepared buffers; x holds the guess when use_x0.  The host
-// enqueues check_every iterations, then one status kernel and a read-back.
+// The iterations after an init: check_every at a time, then one status
+// kernel and a read-back (the first batch without waiting for the init: its
+// launches return at once if the init met the tolerance).
+static nnx_status cg_loop(nnx_ctx* c, CgHost& h, float* x, int maxit, int check_every, int xzero, int32_t* fl,
+                          double* sc) {
+    if (check_every < 1) check_every = 1;
+    int enq = 0;
+    do {
+        for (int q = 0; q < check_every && enq < maxit; ++q, ++enq) cg_iter_launch(c, h, enq, x, xzero);
+        k_cg_status<<<1, 256, 0, c->stream>>>(h.d);
+        NNX_LAUNCHED(c);
+        NNX_TRY(cg_readback(c, h, fl, sc));
+    } while (!fl[FL_DONE] && enq < maxit);
+    return NNX_OK;
+}
+
+// Runs CG on the prepared buffers; x holds the guess when use_x0.
 static nnx_status cg_run(nnx_ctx* c, const GridK& gk, CgHost& h, const float* b, float* x,
                          int use_x0, double tol, int maxit, int abs_mode, int check_every,
                          nnx_cg_result* res, int* initdone = nullptr) {
     cg_init_launch(c, gk, h, b, x, use_x0, tol, abs_mode, maxit);
-    NNX_LAUNCHED(c);
-    if (check_every < 1) check_every = 1;
     int32_t fl[FL_N];
     double sc[SC_N];
-    NNX_TRY(cg_readback(c, h, fl, sc));
+    NNX_TRY(cg_loop(c, h, x, maxit, check_every, 0, fl, sc));
     if (initdone) *initdone = fl[FL_INITDONE];
-    int enq = 0;
-    while (!fl[FL_DONE] && enq < maxit) {
-        for (int q = 0; q < check_every && enq < maxit; ++q, ++enq) cg_iter_launch(c, h, enq, x);
-        k_cg_status<<<1, 256, 0, c->stream>>>(h.d);
-        NNX_LAUNCHED(c);
-        NNX_TRY(cg_readback(c, h, fl, sc));
-    }
     cg_finish_launch(c, h, x);
     NNX_LAUNCHED(c);
     if (res) {
@@ -1471,15 +1562,22 @@ static nnx_status cg_run(nnx_ctx* c, const GridK& gk, CgHost& h, const float* b,
     return NNX_OK;
 }
 
-template <class U, class B>
-static nnx_status true_residual(nnx_ctx* c, const GridK& gk, CgHost& h, const U* x, const B* b,
-                                double* rel, double* rr_out, double* r_out) {
-    k_true_res<U, B><<<kRedBlocks, 256, 0, c->stream>>>(gk, x, b, h.tr_part, r_out);
+// ||b - A x||^2 and ||b||^2 (FP64) from their partials
+static nnx_status read_norms(nnx_ctx* c, CgHost& h, double* rb) {
     k_sum2<<<1, 256, 0, c->stream>>>(h.tr_part, h.out2);
     NNX_LAUNCHED(c);
     NNX_HIP(c, hipMemcpyAsync(c->pinned, h.out2, 16, hipMemcpyDeviceToHost, c->stream));
     NNX_HIP(c, hipStreamSynchronize(c->stream));
-    const double* o = (const double*)c->pinned;
+    std::memcpy(rb, c->pinned, 16);
+    return NNX_OK;
+}
+
+template <class U, class B>
+static nnx_status true_residual(nnx_ctx* c, const GridK& gk, CgHost& h, const U* x, const B* b,
+                                double* rel, double* rr_out, double* r_out) {
+    k_true_res<U, B><<<kRedBlocks, 256, 0, c->stream>>>(gk, x, b, h.tr_part, r_out);
+    double o[2];
+    NNX_TRY(read_norms(c, h, o));
     if (rel) *rel = std::sqrt(o[0] / (o[1] > 0 ? o[1] : 1.0));
     if (rr_out) {
         rr_out[0] = o[0];
@@ -1928,22 +2026,39 @@ nnx_status nnx_cg_solve_refine(nnx_ctx* c, const nnx_grid* g, const double* b, d
     double rel = 0;
     for (;;) {
         double rb[2];
-        NNX_TRY((true_residual<double, double>(c, gk, h, x, b, nullptr, rb, (double*)r64)));
+        if (res64_ok(h, x, b)) {
+            res64_launch<2>(c, h, x, b, h.tr_part, nullptr, (double*)r64);
+            NNX_TRY(read_norms(c, h, rb));
+        } else {
+            NNX_TRY((true_residual<double, double>(c, gk, h, x, b, nullptr, rb, (double*)r64)));
+        }
         const double rr = rb[0], bb = rb[1];
         rel = std::sqrt(rr / (bb > 0 ? bb : 1.0));
         if (rel <= o->rtol || outer >= max_outer || rr == 0) break;
-        // inner solve on the residual scaled to unit norm
+        // inner solve on the residual scaled to unit norm, no tighter than
+        // the outer target needs
         const double s = 1.0 / std::sqrt(rr);
-        k_f64_to_f32_scaled<<<flat_blocks(n), 256, 0, c->stream>>>(n, (const double*)r64, s, (float*)rhs);
-        NNX_LAUNCHED(c);
-        // solve the correction no tighter than the outer target needs
         const double tol = std::max(inner_rtol, 0.5 * o->rtol / rel);
-        nnx_cg_result ir{};
-        NNX_TRY(cg_run(c, gk, h, (const float*)rhs, (float*)d, 0, tol, o->maxit, 0,
-                       o->check_every, &ir));
-        inner_total += ir.iters;
-        k_axpy_f64<<<flat_blocks(n), 256, 0, c->stream>>>(n, 1.0 / s, (const float*)d, x);
-        NNX_LAUNCHED(c);
+        if (h.fast) {
+            // the scaling, the start and the correction's addition to x folded
+            // into the tiled CG's passes
+            int32_t fl[FL_N];
+            double sc[SC_N];
+            k_cg_init64<<<kRedBlocks, 256, 0, c->stream>>>(gk, h.gp.nx, h.d, (const double*)r64, s);
+            k_cg_init_fin<<<1, 256, 0, c->stream>>>(h.d, tol, 0, o->maxit);
+            NNX_TRY(cg_loop(c, h, (float*)d, o->maxit, o->check_every, 1, fl, sc));
+            cg_finish_launch(c, h, (float*)d, 1, x, 1.0 / s);
+            NNX_LAUNCHED(c);
+            inner_total += fl[FL_ITERS];
+        } else {
+            k_f64_to_f32_scaled<<<flat_blocks(n), 256, 0, c->stream>>>(n, (const double*)r64, s, (float*)rhs);
+            NNX_LAUNCHED(c);
+            nnx_cg_result ir{};
+            NNX_TRY(cg_run(c, gk, h, (const float*)rhs, (float*)d, 0, tol, o->maxit, 0, o->check_every, &ir));
+            inner_total += ir.iters;
+            k_axpy_f64<<<flat_blocks(n), 256, 0, c->stream>>>(n, 1.0 / s, (const float*)d, x);
+            NNX_LAUNCHED(c);
+        }
         ++outer;
     }
     auto t1 = std::chrono::steady_clock::now();
@@ -2032,37 +2147,31 @@ nnx_status para_launch(nnx_ctx* c, const ParaIo& io) {
     const int max_inner = q.max_inner > 0 ? q.max_inner : 64;
     const int max_outer = q.max_outer > 0 ? q.max_outer : 3;
     const double inner_rtol = q.inner_rtol > 0 ? q.inner_rtol : 1e-6;
-    // the tiled iteration (7-point grids, rows of a multiple of 4 voxels,
-    // 16-byte aligned vectors); on the constant grid also the tiled FP64
+    // on the constant 7-point grid with the tiled iteration also the tiled FP64
     // residual, after which the inner CG starts from a zero correction
     // without storing it and its last update goes straight into the field
-    const bool tiled = h.fast == kFastConst && !h.pad && (uintptr_t)q.conc % 16 == 0;
-    const int nbr = std::min(stencil4_blocks(gk), kRedBlocks);
+    const bool tiled = res64_ok(h, q.conc, ph.b);
     k_para_rhs<<<kRedBlocks, 256, 0, c->stream>>>(nv, q.conc, io.voxel_counts, q.release, ph.b, ph.pbb, ph.pfl);
     for (int o = 0; o < max_outer; ++o) {
         // the later refinement steps solve to a looser tolerance: half the budget
         const int budget = o == 0 ? max_inner : std::max(1, max_inner / 2);
-        if (tiled && gk.block)
-            k_res64x4<false, true><<<nbr, kT4, 0, c->stream>>>(gk, q.conc, ph.b, h.d, ph.prr, ph.pfl);
-        else if (tiled)
-            k_res64x4<false><<<nbr, kT4, 0, c->stream>>>(gk, q.conc, ph.b, h.d, ph.prr, ph.pfl);
+        if (tiled)
+            res64_launch<0>(c, h, q.conc, ph.b, ph.prr, ph.pfl, nullptr);
         else
             k_para_res<false><<<kRedBlocks, 256, 0, c->stream>>>(gk, h.gp.nx, q.conc, ph.b, h.d,
                                                                  h.pad ? h.xp : ph.xin, h.pa, ph.prr, ph.pfl);
         k_para_ctl<<<1, 256, 0, c->stream>>>(h.d, ph.prr, ph.pbb, q.rtol, inner_rtol, budget, ph.pfl, q.stats, 0,
                                              o > 0);
         for (int k = 0; k < budget; ++k) cg_iter_launch(c, h, k, ph.xin, tiled);
-        if (tiled) {
-            cg_finish_launch(c, h, ph.xin, 1, q.conc);
+        if (h.fast) {
+            cg_finish_launch(c, h, ph.xin, tiled, q.conc);
         } else {
-            cg_finish_launch(c, h, ph.xin, 0, nullptr, 0);
+            cg_finish_launch(c, h, ph.xin);
             k_para_axpy<<<flat_blocks(nv), 256, 0, c->stream>>>(nv, ph.xin, q.conc, h.d.fl, ph.pfl);
         }
     }
-    if (tiled && gk.block)
-        k_res64x4<true, true><<<nbr, kT4, 0, c->stream>>>(gk, q.conc, ph.b, h.d, ph.prr, ph.pfl);
-    else if (tiled)
-        k_res64x4<true><<<nbr, kT4, 0, c->stream>>>(gk, q.conc, ph.b, h.d, ph.prr, ph.pfl);
+    if (tiled)
+        res64_launch<1>(c, h, q.conc, ph.b, ph.prr, ph.pfl, nullptr);
     else
         k_para_res<true><<<kRedBlocks, 256, 0, c->stream>>>(gk, gk.nx, q.conc, ph.b, h.d, ph.xin, h.pa, ph.prr, ph.pfl);
     k_para_ctl<<<1, 256, 0, c->stream>>>(h.d, ph.prr, ph.pbb, q.rtol, inner_rtol, max_inner, ph.pfl, q.stats, 1,

@@ -160,3 +160,34 @@ def test_paracrine_step_on_ragged_grids(ctx, dims):
     say("ragged in-step", dims, np.linalg.norm(conc - ref) / np.linalg.norm(ref), sim.paracrine_stats())
     assert np.linalg.norm(conc - ref) <= 1.3e-7 * np.linalg.norm(ref)
     assert sim.paracrine_stats()["unconverged"] == 0
+
+
+@pytest.mark.parametrize("dims,block,off", [((64, 33, 20), 0, 1), ((50, 33, 20), 0, 1), ((32, 32, 16), 16, 1),
+                                            ((32, 32, 16), 16, 0), ((256, 256, 208), 0, 0), ((8, 9, 10), 0, 1)])
+def test_refinement_on_unaligned_fields(ctx, dims, block, off):
+    """FP64 refinement to 1e-10 on fields at 8- and 16-byte addresses (off: 1,
+    0), plain and on a block lattice, and on a grid of the 1024-thread tiles;
+    the residual with the oracle's operator (block by block)."""
+    import oracle
+    nx, ny, nz = dims
+    n = nx * ny * nz
+    say("refine", dims, block, off)
+    g = _lib.Grid(nx, ny, nz, 7, 1.3, 0.0, None, None, None, block)
+    b = np.random.default_rng(n).standard_normal(n)
+    db = DA.from_numpy(ctx, np.concatenate([np.zeros(off), b]))
+    dx = DA.from_numpy(ctx, np.full(n + off, 3.0))
+    o = _lib.CgOpts(rtol=1e-10, maxit=500, precond=_lib.PRECOND_JACOBI, check_every=4)
+    ctx.call("nnx_cg_solve_refine", C.byref(g), db.ptr + 8 * off, dx.ptr + 8 * off, C.byref(o), 1e-6, 10, None)
+    x = dx.numpy()
+    assert (x[:off] == 3.0).all()
+    X, B = x[off:].reshape(nz, ny, nx), b.reshape(nz, ny, nx)
+    m = block or max(dims)
+    res = 0.0
+    for k in range(0, nz, m):
+        for j in range(0, ny, m):
+            for i in range(0, nx, m):
+                s = np.s_[k:k + m, j:j + m, i:i + m]
+                xs = np.ascontiguousarray(X[s])
+                og = oracle.grid(xs.shape[2], xs.shape[1], xs.shape[0], 7, 1.3)
+                res += ((B[s] - oracle.apply(og, xs.ravel()).reshape(xs.shape)) ** 2).sum()
+    assert np.sqrt(res) <= 1.001e-10 * np.linalg.norm(b)
