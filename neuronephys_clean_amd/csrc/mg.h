@@ -11,8 +11,7 @@ constexpr int kMgMaxLevels = 12;
 // cycled by one workgroup in one launch, always as a V-cycle
 constexpr int kMgSubCells = 4096;
 
-// One step of a cycle, executed either as a kernel launch (large levels) or
-// by the one-workgroup kernel (small levels).  `level` is the level the
+// One step of a cycle.  `level` is the level the
 // operator of the step belongs to (the fine level for RESTRICT/PROLONG).
 enum MgOpType { MG_CHEB = 0, MG_JAC, MG_RESTRICT, MG_RESID, MG_PROLONG, MG_ADD };
 struct MgOp {
@@ -23,6 +22,16 @@ struct MgOp {
     float* dvec;        // CHEB: direction
     const float* dinv;  // CHEB/JAC
     float c1, c2;       // CHEB: d = c1 d + c2 D^-1 r; JAC: c1 = weight
+};
+
+// A visit of the small levels: up to three, the finest first.
+struct MgSubArgs {
+    GridK g[3];
+    const float* dinv[3];
+    const float* rhs;  // of the finest
+    float* out;
+    int nlev, nu, coarse_sweeps, jac;
+    float w, c1[16], c2[16];
 };
 
 // One hierarchy: level 0 is the caller's grid; level l+1 halves every
@@ -39,16 +48,12 @@ struct Mg {
     float* x[2][kMgMaxLevels];      // per visit set: iterate and its ping-pong partner
     float* t[2][kMgMaxLevels];
     int sub = -1;                   // first level cycled in one workgroup (-1: none)
-    const MgOp* sub_ops[2] = {nullptr, nullptr};  // device op lists of a visit of level `sub`, per set
-    int sub_nops[2] = {0, 0};
-    float* sub_res[2] = {nullptr, nullptr};       // where each of those visits leaves its result
-    const GridK* d_gk = nullptr;    // device copy of g[]
+    MgSubArgs sub_args;             // of a visit of level `sub` (rhs and out per visit)
 };
 
 // Builds the hierarchy of a variable-coefficient 7-point grid (coarse face
-// coefficients, diagonals, buffers, the small levels' op lists); nu =
-// smoothing sweeps per level, gamma = visits of each coarser level (1 V,
-// 2 W).
+// coefficients, diagonals, buffers); nu = smoothing sweeps per level, gamma =
+// visits of each coarser level (1 V, 2 W).
 nnx_status mg_setup(nnx_ctx* c, const GridK& g0, int nu, int smoother, int gamma, Mg* m);
 // z = M(r): one cycle from a zero initial guess.
 nnx_status mg_vcycle(nnx_ctx* c, Mg& m, const float* r, float* z);

@@ -20,11 +20,9 @@
 // pair, so the cycle is used inside flexible CG.
 //
 // One generator produces the cycle as a sequence of steps (sweep, restrict,
-// residual, prolong-add, add).  Steps on large levels are kernel launches;
-// the steps of a visit of the first level of <= 4096 cells and below are
-// built once per hierarchy and run by a single workgroup in one launch
-// (tens of steps of a few microseconds' latency each would otherwise be
-// tens of launches).
+// residual, prolong-add, add), each a kernel launch; a visit of the first
+// level of <= 4096 cells and below is one step, run by a single workgroup
+// (k_mg_sub).
 //
 // No counterpart in the reference, whose CG is unpreconditioned
 // (src/paracrine.cu:106-129).
@@ -153,40 +151,181 @@ template <int T> __global__ __launch_bounds__(256) void k_mg_op(MgOp o, GridK g,
     for_rows(d.nx, d.ny, d.nz, [&](int i, int j, int k, int64_t id) { op_at<T>(g, gc, o, i, j, k, id); });
 }
 
-// a whole sequence of steps over small levels by one workgroup
-__global__ __launch_bounds__(1024) void k_mg_sub(const MgOp* __restrict__ ops, int nops, const GridK* __restrict__ gk) {
-    for (int q = 0; q < nops; ++q) {
-        const MgOp o = ops[q];
-        const GridK g = gk[o.level];
-        const GridK gc = gk[o.level + 1 < kMgMaxLevels ? o.level + 1 : o.level];
-        const GridK& d = o.type == MG_RESTRICT ? gc : g;
-        const int nx = d.nx, ny = d.ny, n = d.nx * d.ny * d.nz;
-        for (int id = threadIdx.x; id < n; id += blockDim.x) {
-            const int i = id % nx, j = (id / nx) % ny, k = id / (nx * ny);
-            switch (o.type) {
-                case MG_CHEB: op_at<MG_CHEB>(g, gc, o, i, j, k, id); break;
-                case MG_JAC: op_at<MG_JAC>(g, gc, o, i, j, k, id); break;
-                case MG_RESTRICT: op_at<MG_RESTRICT>(g, gc, o, i, j, k, id); break;
-                case MG_RESID: op_at<MG_RESID>(g, gc, o, i, j, k, id); break;
-                case MG_PROLONG: op_at<MG_PROLONG>(g, gc, o, i, j, k, id); break;
-                default: op_at<MG_ADD>(g, gc, o, i, j, k, id); break;
-            }
+// One visit (a V-cycle) of the levels of at most kMgSubCells cells by one
+// workgroup: a thread keeps its cells' operator, right-hand side, Chebyshev
+// direction and value in registers (4 cells of the finest of the levels, one
+// of the others), the values go through double-buffered LDS with a zero
+// border, so a step costs LDS reads and one barrier.  The coarser levels of
+// 4096 cells have at most 512 and 64 (a level is coarsened only while every
+// dimension is at least 8), so three levels are the most.  Bound by the
+// latency of its ~35 dependent steps: 16^3 with nu = 3 21.7 us where the same
+// steps on buffers in global memory, interpreted from a list, took 91.
+constexpr int kSubThreads = 1024, kSubCpt = kMgSubCells / kSubThreads;
+// border included: the largest box of 4096 (512, 64) cells whose dimensions
+// are all at least 4
+constexpr int kSubBox0 = 6 * 6 * 258, kSubBox1 = 6 * 6 * 34, kSubBox2 = 6 * 6 * 6;
+
+template <int CPT> struct SubLevel {
+    GridK g;
+    float *cur, *oth;  // LDS, border of one: the values, and the spare buffer
+    int n, sy, sz;
+    float k[CPT][6], dg[CPT], di[CPT], b[CPT], x[CPT], d[CPT];
+    int pos[CPT];  // LDS index of the cell (0: none)
+
+    __device__ __forceinline__ void load(const GridK& gk, const float* __restrict__ dinv,
+                                         const float* __restrict__ rhs, float* b0, float* b1, int box) {
+        g = gk, cur = b0, oth = b1;
+        n = g.nx * g.ny * g.nz, sy = g.nx + 2, sz = sy * (g.ny + 2);
+        for (int i = threadIdx.x; i < box; i += kSubThreads) b0[i] = 0.0f, b1[i] = 0.0f;
+#pragma unroll
+        for (int q = 0; q < CPT; ++q) {
+            const int id = (int)threadIdx.x + q * kSubThreads;
+            pos[q] = 0, x[q] = 0.0f, d[q] = 0.0f, b[q] = 0.0f, dg[q] = 0.0f, di[q] = 0.0f;
+#pragma unroll
+            for (int f = 0; f < 6; ++f) k[q][f] = 0.0f;
+            if (id >= n) continue;
+            const int i = id % g.nx, j = (id / g.nx) % g.ny, kk = id / (g.nx * g.ny);
+            pos[q] = (i + 1) + sy * (j + 1) + sz * (kk + 1);
+            const int fx = i + (g.nx + 1) * (j + g.ny * kk), fy = i + g.nx * (j + (g.ny + 1) * kk);
+            k[q][0] = g.kx[fx], k[q][1] = g.kx[fx + 1];
+            k[q][2] = g.ky[fy], k[q][3] = g.ky[fy + g.nx];
+            k[q][4] = g.kz[id], k[q][5] = g.kz[id + g.nx * g.ny];
+            dg[q] = 1.0f + k[q][0] + k[q][1] + k[q][2] + k[q][3] + k[q][4] + k[q][5];
+            di[q] = dinv[id];
+            if (rhs) b[q] = rhs[id];
+        }
+    }
+    // b - A x at cell q (apply_at's operation order)
+    __device__ __forceinline__ float resid(int q) const {
+        const float* v = cur + pos[q];
+        float s = k[q][0] * v[-1] + k[q][1] * v[1];
+        s = s + k[q][2] * v[-sy];
+        s = s + k[q][3] * v[sy];
+        s = s + k[q][4] * v[-sz];
+        s = s + k[q][5] * v[sz];
+        return b[q] - (dg[q] * x[q] - s);
+    }
+    // the new values into the other buffer
+    __device__ __forceinline__ void publish() {
+#pragma unroll
+        for (int q = 0; q < CPT; ++q)
+            if (pos[q]) oth[pos[q]] = x[q];
+        float* t = cur;
+        cur = oth, oth = t;
+        __syncthreads();
+    }
+    // zero: from x = 0 (nothing read)
+    __device__ __forceinline__ void cheb(float c1, float c2, bool zero) {
+#pragma unroll
+        for (int q = 0; q < CPT; ++q) {
+            if (!pos[q]) continue;
+            const float t = c2 * di[q] * (zero ? b[q] : resid(q));
+            const float dn = c1 != 0.0f ? c1 * d[q] + t : t;
+            d[q] = dn;
+            x[q] = zero ? dn : x[q] + dn;
+        }
+        publish();
+    }
+    __device__ __forceinline__ void jacobi(float w, bool zero) {
+#pragma unroll
+        for (int q = 0; q < CPT; ++q) {
+            if (!pos[q]) continue;
+            x[q] = zero ? w * di[q] * b[q] : x[q] + w * di[q] * resid(q);
+        }
+        publish();
+    }
+    __device__ __forceinline__ void sweeps(const MgSubArgs& a, bool zero) {
+        for (int s = 0; s < a.nu; ++s) {
+            if (a.jac) jacobi(a.w, zero && s == 0);
+            else cheb(a.c1[s], a.c2[s], zero && s == 0);
+        }
+    }
+    __device__ __forceinline__ void solve(const MgSubArgs& a) {
+        for (int s = 0; s < a.coarse_sweeps; ++s) jacobi(a.w, s == 0);
+    }
+    // this level's residual into its spare buffer, its block means into c's b
+    template <int C2> __device__ __forceinline__ void restrict_to(SubLevel<C2>& c) {
+        float* o = oth;
+#pragma unroll
+        for (int q = 0; q < CPT; ++q)
+            if (pos[q]) o[pos[q]] = resid(q);
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < C2; ++q) {
+            if (!c.pos[q]) continue;
+            const int id = (int)threadIdx.x + q * kSubThreads;
+            const int I = id % c.g.nx, J = (id / c.g.nx) % c.g.ny, K = id / (c.g.nx * c.g.ny);
+            float s = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                s = s + o[(2 * I + (e & 1) + 1) + sy * (2 * J + ((e >> 1) & 1) + 1) + sz * (2 * K + (e >> 2) + 1)];
+            c.b[q] = 0.125f * s;
         }
         __syncthreads();
     }
+    // x += P (c's x): op_prolong's weights, its zeros outside from the border
+    template <int C2> __device__ __forceinline__ void prolong_from(const SubLevel<C2>& c) {
+        const float* e = c.cur;
+#pragma unroll
+        for (int q = 0; q < CPT; ++q) {
+            if (!pos[q]) continue;
+            const int id = (int)threadIdx.x + q * kSubThreads;
+            const int i = id % g.nx, j = (id / g.nx) % g.ny, kk = id / (g.nx * g.ny);
+            const int p = ((i >> 1) + 1) + c.sy * ((j >> 1) + 1) + c.sz * ((kk >> 1) + 1);
+            const int di_ = (i & 1) ? 1 : -1, dj = (j & 1) ? c.sy : -c.sy, dk = (kk & 1) ? c.sz : -c.sz;
+            const float v0 = 0.75f * e[p] + 0.25f * e[p + di_];
+            const float v1 = 0.75f * e[p + dj] + 0.25f * e[p + dj + di_];
+            const float v2 = 0.75f * e[p + dk] + 0.25f * e[p + dk + di_];
+            const float v3 = 0.75f * e[p + dj + dk] + 0.25f * e[p + dj + dk + di_];
+            const float u0 = 0.75f * v0 + 0.25f * v1;
+            const float u1 = 0.75f * v2 + 0.25f * v3;
+            x[q] = x[q] + (0.75f * u0 + 0.25f * u1);
+        }
+        publish();
+    }
+};
+
+__global__ __launch_bounds__(kSubThreads) void k_mg_sub(MgSubArgs a) {
+    __shared__ float s0[2][kSubBox0], s1[2][kSubBox1], s2[2][kSubBox2];
+    SubLevel<kSubCpt> l0;
+    SubLevel<1> l1, l2;
+    l0.load(a.g[0], a.dinv[0], a.rhs, s0[0], s0[1], kSubBox0);
+    if (a.nlev > 1) l1.load(a.g[1], a.dinv[1], nullptr, s1[0], s1[1], kSubBox1);
+    if (a.nlev > 2) l2.load(a.g[2], a.dinv[2], nullptr, s2[0], s2[1], kSubBox2);
+    __syncthreads();
+    if (a.nlev == 1) {
+        l0.solve(a);
+    } else {
+        l0.sweeps(a, true);
+        l0.restrict_to(l1);
+        if (a.nlev == 2) {
+            l1.solve(a);
+        } else {
+            l1.sweeps(a, true);
+            l1.restrict_to(l2);
+            l2.solve(a);
+            l1.prolong_from(l2);
+            l1.sweeps(a, false);
+        }
+        l0.prolong_from(l1);
+        l0.sweeps(a, false);
+    }
+#pragma unroll
+    for (int q = 0; q < kSubCpt; ++q)
+        if (l0.pos[q]) a.out[(int)threadIdx.x + q * kSubThreads] = l0.x[q];
 }
 
 // The steps of one visit of level l (right-hand side rhs, buffer set `set`),
-// appended to ops; returns the buffer that holds the visit's result.  With
-// `host`, a visit of the level cycled in one workgroup is one MG_SUB marker
-// (type -1, c1 = set).  Level 0 starts its sweeps in t so that an even
+// appended to ops; returns the buffer that holds the visit's result.  A
+// visit of the level cycled in one workgroup is one marker (type -1, xout its
+// result).  Level 0 starts its sweeps in t so that an even
 // number of sweeps ends in `z0`.
-float* gen_visit(const Mg& m, int l, const float* rhs, int set, std::vector<MgOp>& ops, bool host, float* z0) {
-    if (host && l == m.sub) {
+float* gen_visit(const Mg& m, int l, const float* rhs, int set, std::vector<MgOp>& ops, float* z0) {
+    if (l == m.sub) {
         MgOp o{};
-        o.type = -1, o.level = l, o.c1 = (float)set;
+        o.type = -1, o.level = l, o.rhs = rhs, o.xout = m.x[set][l];
         ops.push_back(o);
-        return m.sub_res[set];
+        return o.xout;
     }
     float* X = l == 0 ? z0 : m.x[set][l];
     float* T = m.t[set][l];
@@ -226,14 +365,14 @@ float* gen_visit(const Mg& m, int l, const float* rhs, int set, std::vector<MgOp
         o.type = MG_RESTRICT, o.level = l, o.rhs = rhs, o.xin = cur, o.xout = m.b[l + 1];
         ops.push_back(o);
     }
-    float* e = gen_visit(m, l + 1, m.b[l + 1], 0, ops, host, z0);
+    float* e = gen_visit(m, l + 1, m.b[l + 1], 0, ops, z0);
     // the W-cycle's second visit only for levels above the one-workgroup ones
     const int gam = (m.sub < 0 || l + 1 < m.sub) ? m.gamma : 1;
     for (int v = 1; v < gam; ++v) {
         MgOp r{};
         r.type = MG_RESID, r.level = l + 1, r.xin = e, r.xout = m.b[l + 1];
         ops.push_back(r);
-        float* e2 = gen_visit(m, l + 1, m.b[l + 1], 1, ops, host, z0);
+        float* e2 = gen_visit(m, l + 1, m.b[l + 1], 1, ops, z0);
         MgOp a{};
         a.type = MG_ADD, a.level = l + 1, a.xin = e2, a.xout = e;
         ops.push_back(a);
@@ -327,23 +466,12 @@ nnx_status mg_setup(nnx_ctx* c, const GridK& g0, int nu, int smoother, int gamma
             break;
         }
     if (m->sub > 0) {
-        std::vector<MgOp> lists[2];
-        for (int set = 0; set < 2; ++set)
-            m->sub_res[set] = gen_visit(*m, m->sub, m->b[m->sub], set, lists[set], false, nullptr);
-        const size_t n0 = lists[0].size(), n1 = lists[1].size();
-        void *ops, *gk;
-        NNX_TRY(scratch(c, "mg_ops", (n0 + n1) * sizeof(MgOp), false, &ops));
-        NNX_TRY(scratch(c, "mg_gk", sizeof(m->g), false, &gk));
-        std::vector<MgOp> all(lists[0]);
-        all.insert(all.end(), lists[1].begin(), lists[1].end());
-        NNX_HIP(c, hipMemcpyAsync(ops, all.data(), all.size() * sizeof(MgOp), hipMemcpyHostToDevice, c->stream));
-        NNX_HIP(c, hipMemcpyAsync(gk, m->g, sizeof(m->g), hipMemcpyHostToDevice, c->stream));
-        NNX_HIP(c, hipStreamSynchronize(c->stream));  // host temporaries
-        m->sub_ops[0] = (const MgOp*)ops;
-        m->sub_ops[1] = (const MgOp*)ops + n0;
-        m->sub_nops[0] = (int)n0;
-        m->sub_nops[1] = (int)n1;
-        m->d_gk = (const GridK*)gk;
+        NNX_CHECK(c, m->nlev - m->sub <= 3, "multigrid: more than three small levels");
+        MgSubArgs& a = m->sub_args;
+        a.nlev = m->nlev - m->sub;
+        for (int q = 0; q < a.nlev; ++q) a.g[q] = m->g[m->sub + q], a.dinv[q] = m->dinv[m->sub + q];
+        a.nu = m->nu, a.coarse_sweeps = m->coarse_sweeps, a.jac = m->smoother == NNX_MG_JACOBI, a.w = m->w;
+        for (int q = 0; q < 16; ++q) a.c1[q] = m->c1[q], a.c2[q] = m->c2[q];
     }
     return NNX_OK;
 }
@@ -351,11 +479,12 @@ nnx_status mg_setup(nnx_ctx* c, const GridK& g0, int nu, int smoother, int gamma
 nnx_status mg_vcycle(nnx_ctx* c, Mg& m, const float* r, float* z) {
     std::vector<MgOp> ops;
     ops.reserve(256);
-    float* res = gen_visit(m, 0, r, 0, ops, true, z);
+    float* res = gen_visit(m, 0, r, 0, ops, z);
     for (const MgOp& o : ops) {
         if (o.type < 0) {
-            const int set = (int)o.c1;
-            k_mg_sub<<<1, 1024, 0, c->stream>>>(m.sub_ops[set], m.sub_nops[set], m.d_gk);
+            MgSubArgs sa = m.sub_args;
+            sa.rhs = o.rhs, sa.out = o.xout;
+            k_mg_sub<<<1, kSubThreads, 0, c->stream>>>(sa);
             NNX_LAUNCHED(c);
             continue;
         }

@@ -191,3 +191,30 @@ def test_refinement_on_unaligned_fields(ctx, dims, block, off):
                 og = oracle.grid(xs.shape[2], xs.shape[1], xs.shape[0], 7, 1.3)
                 res += ((B[s] - oracle.apply(og, xs.ravel()).reshape(xs.shape)) ** 2).sum()
     assert np.sqrt(res) <= 1.001e-10 * np.linalg.norm(b)
+
+
+# small levels run by one workgroup: one, two and three of them, boxes long in
+# each direction, 4096 cells exactly, and sizes above which another level goes
+# by launches
+@pytest.mark.parametrize("dims", [(8, 10, 12), (16, 16, 16), (32, 32, 32), (8, 8, 512), (8, 512, 8), (512, 8, 8),
+                                  (48, 24, 16), (64, 32, 16), (40, 36, 28)])
+@pytest.mark.parametrize("nu,smoother,cycle", [(3, 0, 2), (1, 1, 1), (5, 0, 1)])
+def test_multigrid_small_levels(ctx, dims, nu, smoother, cycle):
+    """One cycle against the numpy restatement in FP64: a cycle's fp32 sums
+    carry a few hundred roundings of 2^-24 each, 1e-4 of the norm."""
+    import mg_ref
+    from neuronephys_clean_amd import host
+    nx, ny, nz = dims
+    say("mg small", dims, nu, smoother, cycle)
+    rng = np.random.default_rng(nx + ny + nz)
+    c = (20.0 * np.exp(0.5 * rng.standard_normal((nz, ny, nx)))).astype(np.float32)
+    k = host.face_coefficients(c)
+    d = [DA.from_numpy(ctx, a) for a in k]
+    g = _lib.Grid(nx, ny, nz, 7, 0.0, 0.0, *(a.ptr for a in d))
+    r = rng.standard_normal((nz, ny, nx)).astype(np.float32)
+    dr, dz = DA.from_numpy(ctx, r.ravel()), DA.zeros(ctx, r.size, np.float32)
+    ctx.call("nnx_mg_apply", C.byref(g), nu, smoother, cycle, dr.ptr, dz.ptr)
+    ref = mg_ref.vcycle(r.astype(np.float64), *(a.astype(np.float64) for a in k), nu=nu,
+                        smoother=("chebyshev", "jacobi")[smoother], gamma=cycle)
+    got = dz.numpy().reshape(r.shape)
+    assert np.linalg.norm(got - ref) <= 1e-4 * np.linalg.norm(ref)
