@@ -30,22 +30,25 @@ __global__ __launch_bounds__(256) void k_threshold(int64_t n, const T* __restric
 }
 
 // ------------------------------------------------------------------------
-// compaction: one workgroup of 1024 threads walks the bitmap in tiles of
-// 4096 words; each thread owns 4 consecutive words of a tile, a block scan
-// of the per-thread popcounts gives every thread its output offset.
-// Optionally appends (step, neuron) raster pairs and counts releases per
-// voxel (integer atomics: order-independent).
-// ------------------------------------------------------------------------
-// Multi-block compaction: block b owns words [1024b, 1024b + 1024), four
-// consecutive words per thread (65,536 neurons per block).  Its output offset
-// is the popcount of every preceding word, summed by the block itself
+// compaction: block b of 256 threads owns words [W b, W b + W).  Its output
+// offset is the popcount of every preceding word, summed by the block itself
 // (integers: exact, no inter-block communication; 16-byte loads, four
-// independent accumulators); a block scan orders its own words.  The last
-// block finalises the count, the raster length and the step counter.  Raster
-// length and step live in parity pairs: the launch of parity s reads slot s
-// and its last block writes slot s^1, so no block reads a value that another
-// block of the same launch updates.
-constexpr int kCB = 256, kCW = 4, kCBW = kCB * kCW;
+// independent accumulators); a block scan orders its own words.  Optionally
+// appends (step, neuron) raster pairs and counts releases per voxel (integer
+// atomics: order-independent).  The last block finalises the count, the
+// raster length and the step counter.  Raster length and step live in parity
+// pairs: the launch of parity s reads slot s and its last block writes slot
+// s^1, so no block reads a value that another block of the same launch
+// updates.
+// A thread emits the spikes of its own word one after the other where no word
+// of the block has more than kSerialSpikes; in other blocks the 64 lanes of a
+// wavefront emit a word's at once, the words and their offsets read back from
+// LDS (a third of 20,000 neurons firing: 4.6 us, 9.6 as up to 256 dependent
+// stores of a thread that owned four words).  W: 64 words up to kSmallWords
+// (more blocks, each with a short prefix), else 256.
+// ------------------------------------------------------------------------
+constexpr int kCB = 256, kSerialSpikes = 8;
+constexpr int64_t kSmallWords = 16384;
 
 __device__ __forceinline__ int block_scan256(int v, int* total) {
     __shared__ int sh[4];
@@ -65,14 +68,19 @@ __device__ __forceinline__ int block_scan256(int v, int* total) {
     return before + x - v;
 }
 
+template <int W>
 __global__ __launch_bounds__(kCB) void k_compact(int64_t nwords, const uint64_t* __restrict__ bits,
                                                  int32_t* __restrict__ list,
                                                  int32_t* __restrict__ count, CompactExtras ex) {
-    const int64_t b0 = blockIdx.x * (int64_t)kCBW;  // first word of this block (< nwords)
+    const int64_t b0 = blockIdx.x * (int64_t)W;  // first word of this block (< nwords)
     const bool a16 = ((uintptr_t)bits & 15) == 0;
+    __shared__ uint64_t sw[W];
+    __shared__ int so[W];
+    __shared__ int dense;
+    if (threadIdx.x == 0) dense = 0;  // (the prefix's scan has a barrier before the next use)
     int p0 = 0, p1 = 0, p2 = 0, p3 = 0;
     if (a16) {
-        // b0 is a multiple of 1024 words: pairs of words are 16-byte aligned
+        // b0 is a multiple of W words: pairs of words are 16-byte aligned
         const ulonglong2* B2 = reinterpret_cast<const ulonglong2*>(bits);
         const int64_t n2 = b0 / 2;
         int64_t q = threadIdx.x;
@@ -92,38 +100,44 @@ __global__ __launch_bounds__(kCB) void k_compact(int64_t nwords, const uint64_t*
     }
     int pre_tot;
     block_scan256((p0 + p1) + (p2 + p3), &pre_tot);
-    const int64_t w0 = b0 + (int64_t)threadIdx.x * kCW;
-    uint64_t w[kCW];
-#pragma unroll
-    for (int q = 0; q < kCW; ++q) w[q] = w0 + q < nwords ? bits[w0 + q] : 0ull;
-    int cnt = 0;
-#pragma unroll
-    for (int q = 0; q < kCW; ++q) cnt += __popcll(w[q]);
+    const int64_t w0 = b0 + (int64_t)threadIdx.x;
+    const uint64_t w = threadIdx.x < W && w0 < nwords ? bits[w0] : 0ull;
+    const int cnt = __popcll(w);
+    if (cnt > kSerialSpikes) dense = 1;  // (read after the scan's barriers)
     int tot;
     const int off = block_scan256(cnt, &tot);
     const int par = ex.parity;
     const int64_t rbase = ex.raster ? ex.len2[par] : 0;
     const int32_t step = ex.step2 ? (int32_t)ex.step2[par] : 0;
-    int64_t o = (int64_t)pre_tot + off;
-    if (cnt) {
-#pragma unroll
-        for (int q = 0; q < kCW; ++q) {
-            uint64_t x = w[q];
-            while (x) {
-                const int b = __ffsll((unsigned long long)x) - 1;
-                x &= x - 1;
-                const int32_t idx = (int32_t)((w0 + q) * 64 + b);
-                list[o] = idx;
-                if (ex.raster) {
-                    const int64_t r = rbase + o;
-                    if (r < ex.raster_cap) {
-                        ex.raster[2 * r] = step;
-                        ex.raster[2 * r + 1] = idx;
-                    }
-                }
-                if (ex.voxel_of) atomicAdd(&ex.voxel_counts[ex.voxel_of[idx]], 1);
-                ++o;
+    // one spike: its place in the list, its raster row, its release
+    auto emit = [&](int64_t o, int32_t idx) {
+        list[o] = idx;
+        if (ex.raster) {
+            const int64_t r = rbase + o;
+            if (r < ex.raster_cap) {
+                ex.raster[2 * r] = step;
+                ex.raster[2 * r + 1] = idx;
             }
+        }
+        if (ex.voxel_of) atomicAdd(&ex.voxel_counts[ex.voxel_of[idx]], 1);
+    };
+    if (dense) {
+        if (threadIdx.x < W) sw[threadIdx.x] = w, so[threadIdx.x] = off;
+        __syncthreads();
+        const int lane = threadIdx.x & 63;
+#pragma unroll 4
+        for (int q = threadIdx.x >> 6; q < W; q += kCB / 64) {
+            const uint64_t x = sw[q];
+            if ((x >> lane) & 1ull)
+                emit((int64_t)pre_tot + so[q] + __popcll(x & ((1ull << lane) - 1ull)), (int32_t)((b0 + q) * 64 + lane));
+        }
+    } else if (cnt) {
+        int64_t o = (int64_t)pre_tot + off;
+        uint64_t x = w;
+        while (x) {
+            const int b = __ffsll((unsigned long long)x) - 1;
+            x &= x - 1;
+            emit(o++, (int32_t)(w0 * 64 + b));
         }
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
@@ -613,8 +627,11 @@ namespace nnx {
 nnx_status compact_launch(nnx_ctx* c, int64_t n, const uint64_t* bits, int32_t* list,
                           int32_t* count, const CompactExtras& ex) {
     const int64_t nwords = ceil_div(n, 64);
-    k_compact<<<(unsigned)std::max<int64_t>(1, ceil_div(nwords, kCBW)), kCB, 0, c->stream>>>(
-        nwords, bits, list, count, ex);
+    if (nwords <= kSmallWords)
+        k_compact<64><<<(unsigned)std::max<int64_t>(1, ceil_div(nwords, 64)), kCB, 0, c->stream>>>(nwords, bits, list,
+                                                                                               count, ex);
+    else
+        k_compact<256><<<(unsigned)ceil_div(nwords, 256), kCB, 0, c->stream>>>(nwords, bits, list, count, ex);
     NNX_LAUNCHED(c);
     return NNX_OK;
 }

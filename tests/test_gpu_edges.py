@@ -218,3 +218,24 @@ def test_multigrid_small_levels(ctx, dims, nu, smoother, cycle):
                         smoother=("chebyshev", "jacobi")[smoother], gamma=cycle)
     got = dz.numpy().reshape(r.shape)
     assert np.linalg.norm(got - ref) <= 1e-4 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 4095, 4097, 262_145, (1 << 20) - 1, (1 << 20) + 1, 1_700_003])
+def test_compaction_splits(ctx, n):
+    """The ascending list and its length on bitmaps that are empty, sparse,
+    full and mixed (full words among empty ones), at the block sizes' edges;
+    nothing written past the list."""
+    rng = np.random.default_rng(n)
+    say("compact", n)
+    d_list, d_count = DA(ctx, n + 8, np.int32), DA.zeros(ctx, 1, np.int32)
+    for frac in (0.0, 0.0005, 0.02, 0.4, 1.0, -1.0):
+        if frac < 0:
+            fire = np.repeat(rng.random(-(-n // 64)) < 0.1, 64)[:n]
+        else:
+            fire = rng.random(n) < frac
+        words = np.packbits(np.concatenate([fire, np.zeros(-n % 64, bool)]), bitorder="little").view(np.uint64)
+        d_list.upload(np.full(n + 8, -7, np.int32))
+        ctx.call("nnx_spike_compact", n, DA.from_numpy(ctx, words).ptr, d_list.ptr, d_count.ptr)
+        want, got = np.flatnonzero(fire), d_list.numpy()
+        assert int(d_count.numpy()[0]) == len(want)
+        assert np.array_equal(got[:len(want)], want) and (got[len(want):] == -7).all()
