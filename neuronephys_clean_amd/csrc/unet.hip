@@ -750,7 +750,8 @@ __global__ __launch_bounds__(256) void k_wgrad(WgArgs a) {
     }
 }
 
-// dW[co][k] (k < 27 CIN) and db[co] from the workgroups' partials: a block
+// dW[co][k] (k < 27 CIN) and db[co] (zero with hold: biases that training
+// holds at zero) from the workgroups' partials: a block
 // takes 64 consecutive columns of the [co][kp] partial rows (the blocks past
 // them: the bias), wave s of 16 adds rows s, s + 16, ... of its column - four
 // loads in flight - and the 16 sums are added in order, so the order is fixed.
@@ -760,7 +761,7 @@ __global__ __launch_bounds__(256) void k_wgrad(WgArgs a) {
 constexpr int kWrSlices = 16;
 __global__ __launch_bounds__(1024) void k_wgrad_reduce(const float* __restrict__ part, const float* __restrict__ bpart,
                                                        int nwg, int cout, int kp, int kreal, float* __restrict__ dw,
-                                                       float* __restrict__ db) {
+                                                       float* __restrict__ db, int hold) {
     __shared__ float sh[kWrSlices][64];
     const int cols = cout * kp, nblk = (cols + 63) / 64;
     const bool bias = (int)blockIdx.x >= nblk;
@@ -786,7 +787,7 @@ __global__ __launch_bounds__(1024) void k_wgrad_reduce(const float* __restrict__
 #pragma unroll
     for (int q = 1; q < kWrSlices; ++q) t += sh[q][lane];
     if (bias) {
-        db[col] = t;
+        db[col] = hold ? 0.f : t;
     } else {
         const int co = col / kp, k = col - co * kp;
         if (k < kreal) dw[(size_t)co * kreal + k] = t;
@@ -798,9 +799,19 @@ __global__ __launch_bounds__(1024) void k_wgrad_reduce(const float* __restrict__
 // ---------------------------------------------------------------------------
 // fp32 [cout][27 cin] -> bf16 [cout][kpad(cin)] (flip = 0), or the flipped
 // transpose for the data gradient: bf16 [cin][kpad(cout)] with
-// out[ci][(26 - tap) cout + co] = w[co][tap cin + ci] (flip = 1)
-__global__ void k_prep_w(const float* __restrict__ w, int cin, int cout, int flip, uint16_t* __restrict__ out) {
-    const int ci_out = flip ? cout : cin, rows = flip ? cin : cout;
+// out[ci][(26 - tap) cout + co] = w[co][tap cin + ci] (flip = 1).  blockIdx.y
+// picks one of the jobs: a network's ten copies are one launch.
+struct PrepW {
+    const float* w;
+    uint16_t* out;
+    int cin, cout, flip;
+};
+struct PrepJobs {
+    PrepW j[10];
+};
+__global__ void k_prep_w(PrepJobs jobs) {
+    const PrepW a = jobs.j[blockIdx.y];
+    const int ci_out = a.flip ? a.cout : a.cin, rows = a.flip ? a.cin : a.cout;
     const int kp = kpad(ci_out);
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= rows * kp) return;
@@ -808,14 +819,10 @@ __global__ void k_prep_w(const float* __restrict__ w, int cin, int cout, int fli
     float v = 0.f;
     if (k < 27 * ci_out) {
         const int tap = k / ci_out, c = k - tap * ci_out;
-        v = flip ? w[(size_t)c * 27 * cin + (26 - tap) * cin + row] : w[(size_t)row * 27 * cin + k];
+        v = a.flip ? a.w[(size_t)c * 27 * a.cin + (26 - tap) * a.cin + row] : a.w[(size_t)row * 27 * a.cin + k];
     }
-    out[i] = (uint16_t)f2bf(v);
+    a.out[i] = (uint16_t)f2bf(v);
 }
-
-// per-batch sum of squares of a fp32 field: partials [batch][256]
-// per-block FP64 partial sums of x^2 over batch member blockIdx.y (nper a
-// multiple of 4: the network's grids are)
 __global__ __launch_bounds__(256) void k_sumsq(const float* __restrict__ x, int64_t nper, double* __restrict__ part) {
     __shared__ double sh[4];
     const int b = blockIdx.y;
@@ -878,17 +885,19 @@ __global__ void k_grad_combine(int nx, int ny, int nz, int batch, int C, const u
                                uint16_t* __restrict__ out) {
     const int64_t nv = (int64_t)nx * ny * nz * batch, nch = nv * (C / 8);
     for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < nch; i += (int64_t)gridDim.x * 256) {
-        const int64_t v = i / (C / 8);
-        const int c8 = (int)(i - v * (C / 8));
-        u32x4_t s = skip ? *(const u32x4_t*)&skip[v * C + 8 * c8] : u32x4_t{0u, 0u, 0u, 0u};
+        // (every count here is below 2^32: 32-bit divisions)
+        const uint32_t v = (uint32_t)i / (uint32_t)(C / 8);
+        const int c8 = (int)((uint32_t)i - v * (uint32_t)(C / 8));
+        const size_t at = (size_t)v * C + 8 * c8;
+        u32x4_t s = skip ? *(const u32x4_t*)&skip[at] : u32x4_t{0u, 0u, 0u, 0u};
         if (coarse) {
-            const int x = (int)(v % nx), y = (int)((v / nx) % ny);
-            const int64_t zb = v / ((int64_t)nx * ny);
-            const int z = (int)(zb % nz), b = (int)(zb / nz);
+            const uint32_t r = v / (uint32_t)nx, zb = r / (uint32_t)ny;
+            const int x = (int)(v - r * nx), y = (int)(r - zb * ny);
+            const int b = (int)(zb / (uint32_t)nz), z = (int)(zb - (uint32_t)b * nz);
             const size_t pv = (((size_t)b * (nz >> 1) + (z >> 1)) * (ny >> 1) + (y >> 1)) * (nx >> 1) + (x >> 1);
             s = add_scaled8(s, *(const u32x4_t*)&coarse[pv * C + 8 * c8], cscale);
         }
-        const u32x4_t m = *(const u32x4_t*)&act[v * C + 8 * c8];
+        const u32x4_t m = *(const u32x4_t*)&act[at];
         u32x4_t o;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -896,27 +905,37 @@ __global__ void k_grad_combine(int nx, int ny, int nz, int batch, int C, const u
             o[q] = f2bf(bf2f(m[q] & 0xffffu) > 0.f ? lo : kLeak * lo) |
                    (f2bf(bf2f(m[q] >> 16) > 0.f ? hi : kLeak * hi) << 16);
         }
-        *(u32x4_t*)&out[v * C + 8 * c8] = o;
+        *(u32x4_t*)&out[at] = o;
     }
 }
 
-// out[u] = sum of the 8 children of coarse voxel u (adjoint of nearest upsampling)
+// out[u] = sum of the 8 children of coarse voxel u (adjoint of nearest
+// upsampling), eight channels (16 bytes) per thread: 8 x 64^3, 16 channels
+// 12.5 us, 28 as one channel per thread
 __global__ void k_sumpool8(int cx, int cy, int cz, int batch, int C, const uint16_t* __restrict__ in,
                            uint16_t* __restrict__ out) {
-    const int64_t nv = (int64_t)cx * cy * cz * batch;
+    const int64_t nch = (int64_t)cx * cy * cz * batch * (C / 8);
     const int fx = 2 * cx, fy = 2 * cy, fz = 2 * cz;
-    for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < nv * C; i += (int64_t)gridDim.x * 256) {
-        const int64_t u = i / C;
-        const int c = (int)(i - u * C);
-        const int x = (int)(u % cx), y = (int)((u / cx) % cy);
-        const int64_t zb = u / ((int64_t)cx * cy);
-        const int z = (int)(zb % cz), b = (int)(zb / cz);
-        float s = 0.f;
-        for (int d = 0; d < 8; ++d) {
-            const size_t fv = (((size_t)b * fz + 2 * z + (d >> 2)) * fy + 2 * y + ((d >> 1) & 1)) * fx + 2 * x + (d & 1);
-            s += bf2f(in[fv * C + c]);
+    for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < nch; i += (int64_t)gridDim.x * 256) {
+        const uint32_t u = (uint32_t)i / (uint32_t)(C / 8);
+        const int c8 = (int)((uint32_t)i - u * (uint32_t)(C / 8));
+        const uint32_t r = u / (uint32_t)cx, zb = r / (uint32_t)cy;
+        const int x = (int)(u - r * cx), y = (int)(r - zb * cy);
+        const int b = (int)(zb / (uint32_t)cz), z = (int)(zb - (uint32_t)b * cz);
+        u32x4_t v[8];
+#pragma unroll
+        for (int d = 0; d < 8; ++d)
+            v[d] = *(const u32x4_t*)&in[((((size_t)b * fz + 2 * z + (d >> 2)) * fy + 2 * y + ((d >> 1) & 1)) * fx + 2 * x +
+                                         (d & 1)) * C + 8 * c8];
+        u32x4_t o;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float lo = 0.f, hi = 0.f;
+#pragma unroll
+            for (int d = 0; d < 8; ++d) lo += bf2f(v[d][q] & 0xffffu), hi += bf2f(v[d][q] >> 16);
+            o[q] = f2bf(lo) | (f2bf(hi) << 16);
         }
-        out[i] = (uint16_t)f2bf(s);
+        *(u32x4_t*)&out[(size_t)u * C + 8 * c8] = o;
     }
 }
 
@@ -1041,7 +1060,8 @@ __global__ __launch_bounds__(256) void k_anorm(int nx, int ny, int nz, const flo
     const float* fz = kz + (int64_t)b * nx * ny * (nz + 1);
     double acc = 0;
     for (int64_t id = blockIdx.x * 256ll + threadIdx.x; id < nper; id += (int64_t)gridDim.x * 256) {
-        const int i = (int)(id % nx), j = (int)((id / nx) % ny), k = (int)(id / ((int64_t)nx * ny));
+        const uint32_t row = (uint32_t)id / (uint32_t)nx;
+        const int i = (int)((uint32_t)id - row * nx), k = (int)(row / (uint32_t)ny), j = (int)(row - (uint32_t)k * ny);
         const int64_t ix = i + (int64_t)(nx + 1) * (j + (int64_t)ny * k), iy = i + (int64_t)nx * (j + (int64_t)(ny + 1) * k);
         const float kxm = fx[ix], kxp = fx[ix + 1], kym = fy[iy], kyp = fy[iy + nx], kzm = fz[id],
                     kzp = fz[id + (int64_t)nx * ny];
@@ -1076,9 +1096,10 @@ __global__ __launch_bounds__(256) void k_sample_op(int nx, int ny, int nz, int b
                                                    const float* __restrict__ kz, float* __restrict__ out) {
     const int64_t nper = (int64_t)nx * ny * nz;
     for (int64_t g = blockIdx.x * 256ll + threadIdx.x; g < nper * batch; g += (int64_t)gridDim.x * 256) {
-        const int b = (int)(g / nper);
+        const int b = (int)((uint32_t)g / (uint32_t)nper);  // (counts below 2^31: 32-bit divisions)
         const int64_t id = g - b * nper;
-        const int i = (int)(id % nx), j = (int)((id / nx) % ny), k = (int)(id / ((int64_t)nx * ny));
+        const uint32_t row = (uint32_t)id / (uint32_t)nx;
+        const int i = (int)((uint32_t)id - row * nx), k = (int)(row / (uint32_t)ny), j = (int)(row - (uint32_t)k * ny);
         const float* fx = kx + (int64_t)b * (nx + 1) * ny * nz;
         const float* fy = ky + (int64_t)b * nx * (ny + 1) * nz;
         const float* fz = kz + (int64_t)b * nx * ny * (nz + 1);
@@ -1108,7 +1129,7 @@ __global__ __launch_bounds__(256) void k_sample_op(int nx, int ny, int nz, int b
 __global__ void k_diff(const float* __restrict__ z, const float* __restrict__ e, const float* __restrict__ inv,
                        int64_t nper, int batch, float* __restrict__ d) {
     for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < nper * batch; i += (int64_t)gridDim.x * 256)
-        d[i] = z[i] - e[i] * inv[i / nper];
+        d[i] = z[i] - e[i] * inv[(uint32_t)i / (uint32_t)nper];
 }
 
 // Loss (1/B) sum_b |d_b|^2 / T2_b (or, with Ad, d_b.A_b d_b / t_b.A_b t_b)
@@ -1124,7 +1145,7 @@ __global__ __launch_bounds__(256) void k_loss_grad(const float* __restrict__ z, 
     double acc = 0;
     const int64_t n = nper * batch;
     for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-        const int b = (int)(i / nper);
+        const int b = (int)((uint32_t)i / (uint32_t)nper);
         const float diff = z[i] - e[i] * inv[b];
         const float gd = Ad ? Ad[i] : diff;
         dz[i] = (float)(2.0 * gd / ((double)batch * t2[b]));
@@ -1188,7 +1209,7 @@ __global__ __launch_bounds__(1024) void k_head_fin(const double* __restrict__ pa
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
         if (lane == 0) {
-            if (q < 17) ghead[q] = (float)s;
+            if (q < 17) ghead[q] = q < 16 ? (float)s : 0.f;  // (the bias is held at zero, as the layers')
             else *loss = s / batch;
         }
     }
@@ -1342,7 +1363,7 @@ nnx_status conv_dispatch(nnx_ctx* c, int cin, int cout, const ConvArgs& a) {
 constexpr int kWgMax = 512;
 
 template <int CIN, int COUT>
-nnx_status launch_wgrad(nnx_ctx* c, WgArgs a, float* dw, float* db) {
+nnx_status launch_wgrad(nnx_ctx* c, WgArgs a, float* dw, float* db, int hold) {
     NNX_CHECK(c, a.nx % 16 == 0 && a.ny % 4 == 0 && a.nz % 4 == 0, "wgrad dims must be multiples of (16,4,4)");
     if (a.coarse) NNX_CHECK(c, a.nx % 32 == 0 && a.ny % 8 == 0 && a.nz % 8 == 0, "upsampled wgrad needs even dims");
     a.ntiles = (a.nx / 16) * (a.ny / 4) * (a.nz / 4) * a.batch;
@@ -1354,17 +1375,17 @@ nnx_status launch_wgrad(nnx_ctx* c, WgArgs a, float* dw, float* db) {
     a.bpart = (float*)bpart;
     k_wgrad<CIN, COUT><<<nwg, 256, 0, c->stream>>>(a);
     k_wgrad_reduce<<<ceil_div(COUT * kpad(CIN), 64) + 1, 64 * kWrSlices, 0, c->stream>>>(
-        a.part, a.bpart, nwg, COUT, kpad(CIN), 27 * CIN, dw, db);
+        a.part, a.bpart, nwg, COUT, kpad(CIN), 27 * CIN, dw, db, hold);
     NNX_LAUNCHED(c);
     return NNX_OK;
 }
 
-nnx_status wgrad_dispatch(nnx_ctx* c, int cin, int cout, const WgArgs& a, float* dw, float* db) {
-    if (cin == 2 && cout == 16) return launch_wgrad<2, 16>(c, a, dw, db);
-    if (cin == 16 && cout == 16) return launch_wgrad<16, 16>(c, a, dw, db);
-    if (cin == 16 && cout == 32) return launch_wgrad<16, 32>(c, a, dw, db);
-    if (cin == 32 && cout == 16) return launch_wgrad<32, 16>(c, a, dw, db);
-    if (cin == 32 && cout == 32) return launch_wgrad<32, 32>(c, a, dw, db);
+nnx_status wgrad_dispatch(nnx_ctx* c, int cin, int cout, const WgArgs& a, float* dw, float* db, int hold) {
+    if (cin == 2 && cout == 16) return launch_wgrad<2, 16>(c, a, dw, db, hold);
+    if (cin == 16 && cout == 16) return launch_wgrad<16, 16>(c, a, dw, db, hold);
+    if (cin == 16 && cout == 32) return launch_wgrad<16, 32>(c, a, dw, db, hold);
+    if (cin == 32 && cout == 16) return launch_wgrad<32, 16>(c, a, dw, db, hold);
+    if (cin == 32 && cout == 32) return launch_wgrad<32, 32>(c, a, dw, db, hold);
     return fail(c, NNX_ERR_UNSUPPORTED, "wgrad %d->%d not instantiated", cin, cout);
 }
 
@@ -1373,12 +1394,15 @@ unsigned eblocks(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int
 nnx_status prep_weights(nnx_ctx* c, nnx_unet* u) {
     if (!u->dirty) return NNX_OK;
     const Plan& P = plan();
+    PrepJobs jobs;
+    int most = 0;
     for (int i = 0; i < 5; ++i) {
         const Layer& L = P.L[i];
-        const int nf = L.cout * kpad(L.cin), nb = L.cin * kpad(L.cout);
-        k_prep_w<<<ceil_div(nf, 256), 256, 0, c->stream>>>(u->p + L.w_off, L.cin, L.cout, 0, u->wf[i]);
-        k_prep_w<<<ceil_div(nb, 256), 256, 0, c->stream>>>(u->p + L.w_off, L.cin, L.cout, 1, u->wb[i]);
+        jobs.j[2 * i] = PrepW{u->p + L.w_off, u->wf[i], L.cin, L.cout, 0};
+        jobs.j[2 * i + 1] = PrepW{u->p + L.w_off, u->wb[i], L.cin, L.cout, 1};
+        most = std::max(most, std::max(L.cout * kpad(L.cin), L.cin * kpad(L.cout)));
     }
+    k_prep_w<<<dim3((unsigned)ceil_div(most, 256), 10), 256, 0, c->stream>>>(jobs);
     NNX_LAUNCHED(c);
     u->dirty = false;
     return NNX_OK;
@@ -1702,37 +1726,33 @@ nnx_status nnx_unet_train_step(nnx_ctx* c, nnx_unet* u, int nx, int ny, int nz, 
     };
     // d0: input e0 + up(d1), gradient G0
     NNX_TRY(wgrad_dispatch(c, 16, 16, WG(mx, my, mz, A.e0, A.d1, 1.f, G0), u->grad + P.L[4].w_off,
-                           u->grad + P.L[4].b_off));
+                           u->grad + P.L[4].b_off, 1));
     NNX_TRY(conv_dispatch(c, 16, 16, BD(mx, my, mz, G0, u->wb[4], U0)));  // dU0 (skip part of e0's gradient)
-    k_sumpool8<<<eblocks(n1 * 16), 256, 0, c->stream>>>(nx1, ny1, nz1, batch, 16, U0, L1a);  // d(d1)
+    k_sumpool8<<<eblocks(n1 * 2), 256, 0, c->stream>>>(nx1, ny1, nz1, batch, 16, U0, L1a);  // d(d1)
     k_grad_combine<<<eblocks(n1 * 2), 256, 0, c->stream>>>(nx1, ny1, nz1, batch, 16, A.d1, L1a, nullptr, 0.f, L1b);
     NNX_LAUNCHED(c);
     // d1: input e1 + up(e2), gradient L1b (16 ch)
     NNX_TRY(wgrad_dispatch(c, 32, 16, WG(nx1, ny1, nz1, A.e1, A.e2, 1.f, L1b), u->grad + P.L[3].w_off,
-                           u->grad + P.L[3].b_off));
+                           u->grad + P.L[3].b_off, 1));
     NNX_TRY(conv_dispatch(c, 16, 32, BD(nx1, ny1, nz1, L1b, u->wb[3], L1c)));  // dU1 (32 ch)
-    k_sumpool8<<<eblocks(n2 * 32), 256, 0, c->stream>>>(nx2, ny2, nz2, batch, 32, L1c, L2a);  // d(e2)
+    k_sumpool8<<<eblocks(n2 * 4), 256, 0, c->stream>>>(nx2, ny2, nz2, batch, 32, L1c, L2a);  // d(e2)
     k_grad_combine<<<eblocks(n2 * 4), 256, 0, c->stream>>>(nx2, ny2, nz2, batch, 32, A.e2, L2a, nullptr, 0.f, L2b);
     NNX_LAUNCHED(c);
     // e2: input p1, gradient L2b
     NNX_TRY(wgrad_dispatch(c, 32, 32, WG(nx2, ny2, nz2, A.p1, nullptr, 0.f, L2b), u->grad + P.L[2].w_off,
-                           u->grad + P.L[2].b_off));
+                           u->grad + P.L[2].b_off, 1));
     NNX_TRY(conv_dispatch(c, 32, 32, BD(nx2, ny2, nz2, L2b, u->wb[2], L2a)));  // d(p1)
     // e1 gradient: skip part dU1 + pooled part d(p1)/8
     k_grad_combine<<<eblocks(n1 * 4), 256, 0, c->stream>>>(nx1, ny1, nz1, batch, 32, A.e1, L1c, L2a, 0.125f, L1a);
     NNX_LAUNCHED(c);
     NNX_TRY(wgrad_dispatch(c, 16, 32, WG(nx1, ny1, nz1, A.p0, nullptr, 0.f, L1a), u->grad + P.L[1].w_off,
-                           u->grad + P.L[1].b_off));
+                           u->grad + P.L[1].b_off, 1));
     NNX_TRY(conv_dispatch(c, 32, 16, BD(nx1, ny1, nz1, L1a, u->wb[1], L1b)));  // d(p0) (16 ch)
     // e0 gradient: dU0 + d(p0)/8
     k_grad_combine<<<eblocks(n0 * 2), 256, 0, c->stream>>>(mx, my, mz, batch, 16, A.e0, U0, L1b, 0.125f, G0);
     NNX_LAUNCHED(c);
     NNX_TRY(wgrad_dispatch(c, 2, 16, WG(mx, my, mz, A.x, nullptr, 0.f, G0), u->grad + P.L[0].w_off,
-                           u->grad + P.L[0].b_off));
-    // the biases are held at zero (the network must map r = 0 to 0)
-    for (int l = 0; l < 5; ++l)
-        NNX_HIP(c, hipMemsetAsync(u->grad + P.L[l].b_off, 0, P.L[l].cout * 4, c->stream));
-    NNX_HIP(c, hipMemsetAsync(u->grad + P.head_off + 16, 0, 4, c->stream));
+                           u->grad + P.L[0].b_off, 1));
     // Adam
     u->step += 1;
     const float b1 = 0.9f, b2 = 0.999f;
@@ -1769,7 +1789,9 @@ nnx_status nnx_conv3_bf16(nnx_ctx* c, int cin, int cout, int nx, int ny, int nz,
     NNX_CHECK(c, cin != 2 || !d_coarse, "the 2-channel input layer takes no upsampled term");
     void* wp;
     NNX_TRY(scratch(c, "un_prim_w", (size_t)cout * kpad(cin) * 2, false, &wp));
-    k_prep_w<<<ceil_div(cout * kpad(cin), 256), 256, 0, c->stream>>>(d_w, cin, cout, 0, (uint16_t*)wp);
+    PrepJobs job{};
+    job.j[0] = PrepW{d_w, (uint16_t*)wp, cin, cout, 0};
+    k_prep_w<<<(unsigned)ceil_div(cout * kpad(cin), 256), 256, 0, c->stream>>>(job);
     NNX_LAUNCHED(c);
     ConvArgs a{};
     a.nx = nx, a.ny = ny, a.nz = nz, a.batch = batch, a.in = d_in, a.coarse = d_coarse, a.cscale = (float)coarse_scale;
@@ -1785,7 +1807,7 @@ nnx_status nnx_conv3_wgrad_bf16(nnx_ctx* c, int cin, int cout, int nx, int ny, i
     WgArgs w{};
     w.nx = nx, w.ny = ny, w.nz = nz, w.batch = batch, w.in = d_in, w.coarse = d_coarse,
     w.cscale = (float)coarse_scale, w.g = d_g;
-    return wgrad_dispatch(c, cin, cout, w, d_dw, d_db);
+    return wgrad_dispatch(c, cin, cout, w, d_dw, d_db, 0);
 }
 
 }  // extern "C"
