@@ -648,54 +648,70 @@ __global__ __launch_bounds__(256) void k_wgrad(WgArgs a) {
         const int bz = rest % tz, b = rest / tz;
         const int x0 = 16 * bx, y0 = 4 * by, z0 = 4 * bz;
         __syncthreads();
-        constexpr int CH = CIN == 2 ? 1 : CIN / 8;
-        for (int i = tid; i < 18 * 36 * CH; i += 256) {
-            const int hv = i / CH, c8 = i - hv * CH;
-            const int hx = hv % 18, hy = (hv / 18) % 6, hz = hv / 108;
-            const int gx = x0 - 1 + hx, gy = y0 - 1 + hy, gz = z0 - 1 + hz;
-            const bool in = gx >= 0 && gx < nx && gy >= 0 && gy < ny && gz >= 0 && gz < nz;
-            const size_t gv = (((size_t)b * nz + gz) * ny + gy) * nx + gx;
-            uint16_t val[8];
-            if (CIN == 2) {
-                const uint32_t v = in ? *(const uint32_t*)&a.in[gv * 2] : 0u;
-                val[0] = (uint16_t)(v & 0xffffu);
-                val[1] = (uint16_t)(v >> 16);
-            } else {
-                u32x4_t v = {0u, 0u, 0u, 0u};
+        // input: a thread takes eight channels of half a halo row (ten
+        // voxels of 16 bytes) and writes each channel's eight voxels for the
+        // three x shifts with one 16-byte store each.  Two-byte stores, one
+        // voxel a thread, made staging half of the kernel: 16 -> 16 at
+        // 8 x 64^3 151 us, 125 so (2 -> 16 59 -> 39, 16 -> 32 at 32^3 26 ->
+        // 20).  Fetching the next tile's registers under the products and
+        // XCD-contiguous tiles give 120 for 16 -> 16 but 49 and 32 for the
+        // others, so the tile is staged in line.
+        constexpr int CH = CIN == 2 ? 1 : CIN / 8, NC = CIN == 2 ? 2 : 8;
+        for (int i = tid; i < 36 * 2 * CH; i += 256) {
+            const int c8 = i % CH, half = (i / CH) & 1, row = i / (2 * CH);
+            const int hy = row % 6, hz = row / 6;
+            const int gx0 = x0 - 1 + 8 * half, gy = y0 - 1 + hy, gz = z0 - 1 + hz;
+            const bool rin = gy >= 0 && gy < ny && gz >= 0 && gz < nz;
+            const size_t gr = (((size_t)b * nz + gz) * ny + gy) * nx;
+            u32x4_t v[10];
+#pragma unroll
+            for (int k = 0; k < 10; ++k) {
+                const int gx = gx0 + k;
+                const bool in = rin && gx >= 0 && gx < nx;
+                v[k] = u32x4_t{0u, 0u, 0u, 0u};
                 if (in) {
-                    v = *(const u32x4_t*)&a.in[gv * CIN + 8 * c8];
-                    if (a.coarse) {
-                        const int cx = nx >> 1, cy = ny >> 1, cz = nz >> 1;
-                        const u32x4_t cv = *(const u32x4_t*)&a.coarse
-                            [((((size_t)b * cz + (gz >> 1)) * cy + (gy >> 1)) * cx + (gx >> 1)) * CIN + 8 * c8];
-                        v = add_scaled8(v, cv, a.cscale);
-                    }
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    val[2 * q] = (uint16_t)(v[q] & 0xffffu);
-                    val[2 * q + 1] = (uint16_t)(v[q] >> 16);
+                    if (CIN == 2) v[k][0] = *(const uint32_t*)&a.in[(gr + gx) * 2];
+                    else v[k] = *(const u32x4_t*)&a.in[(gr + gx) * CIN + 8 * c8];
                 }
             }
-            constexpr int NC = CIN == 2 ? 2 : 8;
+            if (CIN != 2 && a.coarse && rin) {
+                const int cx = nx >> 1, cy = ny >> 1, cz = nz >> 1;
+                const size_t cr = (((size_t)b * cz + (gz >> 1)) * cy + (gy >> 1)) * cx;
 #pragma unroll
-            for (int dx = 0; dx < 3; ++dx) {
-                const int xs = hx - dx;
-                if (xs < 0 || xs >= 16) continue;
-#pragma unroll
-                for (int c = 0; c < NC; ++c)
-                    s_in[(dx * CIN + (CIN == 2 ? c : 8 * c8 + c)) * PLANE + (hz * 6 + hy) * 16 + xs] = val[c];
+                for (int k = 0; k < 10; ++k) {
+                    const int gx = gx0 + k;
+                    if (gx >= 0 && gx < nx)
+                        v[k] = add_scaled8(v[k], *(const u32x4_t*)&a.coarse[(cr + (gx >> 1)) * CIN + 8 * c8], a.cscale);
+                }
             }
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int dx = 0; dx < 3; ++dx) {
+                    u32x4_t o;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        o[q] = __builtin_amdgcn_perm(v[dx + 2 * q + 1][c >> 1], v[dx + 2 * q][c >> 1],
+                                                     c & 1 ? 0x07060302u : 0x05040100u);
+                    *(u32x4_t*)&s_in[(dx * CIN + (CIN == 2 ? c : 8 * c8 + c)) * PLANE + row * 16 + 8 * half] = o;
+                }
         }
-        for (int i = tid; i < 256 * (COUT / 8); i += 256) {
-            const int v = i / (COUT / 8), c8 = i - v * (COUT / 8);
-            const int xs = v % 16, rr = v / 16;
-            const size_t gv = (((size_t)b * nz + z0 + (rr >> 2)) * ny + y0 + (rr & 3)) * nx + x0 + xs;
-            const u32x4_t gg = *(const u32x4_t*)&a.g[gv * COUT + 8 * c8];
+        // gradient: eight channels of eight voxels a thread (from the last
+        // threads down, the ones without input)
+        for (int i = 255 - tid; i < 32 * (COUT / 8); i += 256) {
+            const int c8 = i % (COUT / 8), half = (i / (COUT / 8)) & 1, rr = i / (2 * (COUT / 8));
+            const size_t gv = (((size_t)b * nz + z0 + (rr >> 2)) * ny + y0 + (rr & 3)) * nx + x0 + 8 * half;
+            u32x4_t v[8];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                s_g[(8 * c8 + 2 * q) * kWgRows + v] = (uint16_t)(gg[q] & 0xffffu);
-                s_g[(8 * c8 + 2 * q + 1) * kWgRows + v] = (uint16_t)(gg[q] >> 16);
+            for (int k = 0; k < 8; ++k) v[k] = *(const u32x4_t*)&a.g[(gv + k) * COUT + 8 * c8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                u32x4_t o;
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    o[q] = __builtin_amdgcn_perm(v[2 * q + 1][c >> 1], v[2 * q][c >> 1],
+                                                 c & 1 ? 0x07060302u : 0x05040100u);
+                *(u32x4_t*)&s_g[(8 * c8 + c) * kWgRows + rr * 16 + 8 * half] = o;
             }
         }
         __syncthreads();
