@@ -220,6 +220,37 @@ def test_multigrid_small_levels(ctx, dims, nu, smoother, cycle):
     assert np.linalg.norm(got - ref) <= 1e-4 * np.linalg.norm(ref)
 
 
+# levels above the one-workgroup ones: rows of whole 16-byte groups (fewer and
+# more than a wavefront's 64, last workgroup partly empty, one coarse level
+# off the rule) and rows that are not, every smoother, fields off 16 bytes
+@pytest.mark.parametrize("dims", [(12, 40, 40), (20, 34, 22), (68, 20, 24), (260, 12, 10), (516, 8, 10), (18, 24, 24),
+                                  (36, 24, 48)])
+@pytest.mark.parametrize("nu,smoother,cycle,off", [(3, 0, 2, 0), (2, 1, 2, 1), (1, 0, 1, 3)])
+def test_multigrid_row_groups(ctx, dims, nu, smoother, cycle, off):
+    """One cycle against the numpy restatement in FP64, with the bound of
+    test_multigrid_small_levels."""
+    import mg_ref
+    from neuronephys_clean_amd import host
+    nx, ny, nz = dims
+    say("mg rows", dims, nu, smoother, cycle, off)
+    rng = np.random.default_rng(nx + ny + nz)
+    c = (20.0 * np.exp(0.5 * rng.standard_normal((nz, ny, nx)))).astype(np.float32)
+    k = host.face_coefficients(c)
+    pad = np.zeros(off, np.float32)
+    d = [DA.from_numpy(ctx, np.concatenate([pad, a.ravel()])) for a in k]
+    g = _lib.Grid(nx, ny, nz, 7, 0.0, 0.0, *(a.ptr + 4 * off for a in d))
+    r = rng.standard_normal((nz, ny, nx)).astype(np.float32)
+    dr = DA.from_numpy(ctx, np.concatenate([pad, r.ravel(), pad]))
+    dz = DA.from_numpy(ctx, np.full(r.size + 2 * off, 7.0, np.float32))
+    ctx.call("nnx_mg_apply", C.byref(g), nu, smoother, cycle, dr.ptr + 4 * off, dz.ptr + 4 * off)
+    ref = mg_ref.vcycle(r.astype(np.float64), *(a.astype(np.float64) for a in k), nu=nu,
+                        smoother=("chebyshev", "jacobi")[smoother], gamma=cycle)
+    z = dz.numpy()
+    got = z[off:off + r.size].reshape(r.shape)
+    assert np.linalg.norm(got - ref) <= 1e-4 * np.linalg.norm(ref)
+    assert (z[:off] == 7.0).all() and (z[off + r.size:] == 7.0).all()
+
+
 @pytest.mark.parametrize("n", [1, 64, 65, 4095, 4097, 262_145, (1 << 20) - 1, (1 << 20) + 1, 1_700_003])
 def test_compaction_splits(ctx, n):
     """The ascending list and its length on bitmaps that are empty, sparse,
