@@ -1106,40 +1106,77 @@ __global__ __launch_bounds__(256) void k_anorm(int nx, int ny, int nz, const flo
 //   mode 0: out = A x;  mode 1: out = x - w D^-1 A x  (S x);
 //   mode 2: out = D^-1 x;  mode 3: out = x2 - w A x  (with x = D^-1 x2: S^T x2).
 constexpr float kSmoothWTrain = 2.0f / 3.0f;
-__global__ __launch_bounds__(256) void k_sample_op(int nx, int ny, int nz, int batch, int mode,
-                                                   const float* __restrict__ x, const float* __restrict__ x2,
-                                                   const float* __restrict__ kx, const float* __restrict__ ky,
-                                                   const float* __restrict__ kz, float* __restrict__ out) {
-    const int64_t nper = (int64_t)nx * ny * nz;
-    for (int64_t g = blockIdx.x * 256ll + threadIdx.x; g < nper * batch; g += (int64_t)gridDim.x * 256) {
-        const int b = (int)((uint32_t)g / (uint32_t)nper);  // (counts below 2^31: 32-bit divisions)
-        const int64_t id = g - b * nper;
-        const uint32_t row = (uint32_t)id / (uint32_t)nx;
-        const int i = (int)((uint32_t)id - row * nx), k = (int)(row / (uint32_t)ny), j = (int)(row - (uint32_t)k * ny);
-        const float* fx = kx + (int64_t)b * (nx + 1) * ny * nz;
-        const float* fy = ky + (int64_t)b * nx * (ny + 1) * nz;
-        const float* fz = kz + (int64_t)b * nx * ny * (nz + 1);
-        const int64_t ix = i + (int64_t)(nx + 1) * (j + (int64_t)ny * k), iy = i + (int64_t)nx * (j + (int64_t)(ny + 1) * k);
-        const float kxm = fx[ix], kxp = fx[ix + 1], kym = fy[iy], kyp = fy[iy + nx], kzm = fz[id],
-                    kzp = fz[id + (int64_t)nx * ny];
-        const float dg = 1.f + kxm + kxp + kym + kyp + kzm + kzp;
-        const float* xb = x + b * nper;
-        if (mode == 2) {
-            out[g] = xb[id] / dg;
-            continue;
+// Rows are whole 16-byte groups (check_dims: a multiple of 64)
+// and a batch has fewer than 2^31 voxels: a lane takes 16 bytes of a row (any
+// 4-byte alignment), the x neighbours and the row's last face come from the
+// lanes beside it, and each XCD (workgroups are dealt to the eight in turn)
+// takes a contiguous eighth of the batch, so the rows above and below are in
+// its own L2.  Bound by memory (faces, field and result once): 8 x 64^3 16 us
+// by single voxels, 8 so (the division alone 6.3).
+typedef float f4_t __attribute__((ext_vector_type(4)));
+typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ f4_t ld4(const float* __restrict__ p) { return *reinterpret_cast<const f4u_t*>(p); }
+template <int MODE>
+__global__ __launch_bounds__(256) void k_sample_op(int nx, int ny, int nz, int batch, const float* __restrict__ x,
+                                                    const float* __restrict__ x2, const float* __restrict__ kx,
+                                                    const float* __restrict__ ky, const float* __restrict__ kz,
+                                                    float* __restrict__ out) {
+    const int q8 = (int)(gridDim.x >> 3), r8 = (int)(gridDim.x & 7), xcd = (int)(blockIdx.x & 7);
+    const int blk = xcd * q8 + min(xcd, r8) + (int)(blockIdx.x >> 3);
+    const uint32_t nq = (uint32_t)nx >> 2, n4 = nq * (uint32_t)ny * (uint32_t)nz * (uint32_t)batch;
+    const uint32_t mine = (uint32_t)blk * 256u + threadIdx.x;
+    const uint32_t at = min(mine, n4 - 1u);  // (lanes past the end repeat the last voxels and store nothing)
+    const uint32_t row = at / nq, zb = row / (uint32_t)ny, b = zb / (uint32_t)nz;
+    const int i = 4 * (int)(at - row * nq), j = (int)(row - zb * ny), k = (int)(zb - b * nz);
+    const int lane = threadIdx.x & 63;
+    const int64_t g = 4 * (int64_t)at, nxy = (int64_t)nx * ny;
+    // face rows: row r of the batch starts at (nx + 1) r in x, one row (one
+    // plane) more per plane (sample) in y (z)
+    const float* __restrict__ fx = kx + (int64_t)(nx + 1) * row + i;
+    const float* __restrict__ fy = ky + (int64_t)nx * ((int64_t)row + zb) + i;
+    const float* __restrict__ fz = kz + g + nxy * b;
+    const f4_t kxm = ld4(fx), kym = ld4(fy), kyp = ld4(fy + nx), kzm = ld4(fz), kzp = ld4(fz + nxy);
+    float k4 = __shfl_down(kxm[0], 1, 64);
+    const bool last = i + 4 >= nx;
+    if (lane == 63 || last) k4 = fx[4];
+    const f4_t kxp = {kxm[1], kxm[2], kxm[3], k4};
+    const f4_t xc = ld4(x + g), zero = {0.f, 0.f, 0.f, 0.f};
+    f4_t o;
+    if (MODE == 2) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = xc[e] / (1.f + kxm[e] + kxp[e] + kym[e] + kyp[e] + kzm[e] + kzp[e]);
+    } else {
+        const f4_t ym = j > 0 ? ld4(x + g - nx) : zero, yp = j < ny - 1 ? ld4(x + g + nx) : zero;
+        const f4_t zm = k > 0 ? ld4(x + g - nxy) : zero, zp = k < nz - 1 ? ld4(x + g + nxy) : zero;
+        float l = __shfl_up(xc[3], 1, 64), r = __shfl_down(xc[0], 1, 64);
+        if (lane == 0 && i > 0) l = x[g - 1];
+        if (lane == 63 && !last) r = x[g + 4];
+        const f4_t xm = {l, xc[0], xc[1], xc[2]}, xp = {xc[1], xc[2], xc[3], r};
+        const f4_t o2 = MODE == 3 ? ld4(x2 + g) : zero;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float dg = 1.f + kxm[e] + kxp[e] + kym[e] + kyp[e] + kzm[e] + kzp[e];
+            float sn = 0.f;
+            if (e > 0 || i > 0) sn += kxm[e] * xm[e];
+            if (e < 3 || !last) sn += kxp[e] * xp[e];
+            if (j > 0) sn += kym[e] * ym[e];
+            if (j < ny - 1) sn += kyp[e] * yp[e];
+            if (k > 0) sn += kzm[e] * zm[e];
+            if (k < nz - 1) sn += kzp[e] * zp[e];
+            const float ax = dg * xc[e] - sn;
+            o[e] = MODE == 0 ? ax : MODE == 1 ? xc[e] - kSmoothWTrain * ax / dg : o2[e] - kSmoothWTrain * ax;
         }
-        float sn = 0.f;
-        if (i > 0) sn += kxm * xb[id - 1];
-        if (i < nx - 1) sn += kxp * xb[id + 1];
-        if (j > 0) sn += kym * xb[id - nx];
-        if (j < ny - 1) sn += kyp * xb[id + nx];
-        if (k > 0) sn += kzm * xb[id - (int64_t)nx * ny];
-        if (k < nz - 1) sn += kzp * xb[id + (int64_t)nx * ny];
-        const float ax = dg * xb[id] - sn;
-        if (mode == 0) out[g] = ax;
-        else if (mode == 1) out[g] = xb[id] - kSmoothWTrain * ax / dg;
-        else out[g] = x2[g] - kSmoothWTrain * ax;
     }
+    if (mine < n4) *reinterpret_cast<f4u_t*>(out + g) = o;
+}
+void sample_op(nnx_ctx* c, int nx, int ny, int nz, int batch, int mode, const float* x, const float* x2,
+               const float* kx, const float* ky, const float* kz, float* out) {
+    const unsigned blocks = (unsigned)(((int64_t)nx * ny * nz * batch / 4 + 255) / 256);
+    auto go = [&](auto kernel) { kernel<<<blocks, 256, 0, c->stream>>>(nx, ny, nz, batch, x, x2, kx, ky, kz, out); };
+    if (mode == 0) go(k_sample_op<0>);
+    else if (mode == 1) go(k_sample_op<1>);
+    else if (mode == 2) go(k_sample_op<2>);
+    else go(k_sample_op<3>);
 }
 // d = z - e inv[b]
 __global__ void k_diff(const float* __restrict__ z, const float* __restrict__ e, const float* __restrict__ inv,
@@ -1695,14 +1732,14 @@ nnx_status nnx_unet_train_step(nnx_ctx* c, nnx_unet* u, int nx, int ny, int nz, 
             k_diff<<<eb, 256, 0, c->stream>>>(A.z, d_e, A.inv, nper, batch, Ad);
             float *src = Ad, *dst = U;
             for (int m = 0; m < smooth; ++m) {  // src <- S src
-                k_sample_op<<<eb, 256, 0, c->stream>>>(nx, ny, nz, batch, 1, src, nullptr, d_kx, d_ky, d_kz, dst);
+                sample_op(c, nx, ny, nz, batch, 1, src, nullptr, d_kx, d_ky, d_kz, dst);
                 std::swap(src, dst);
             }
-            k_sample_op<<<eb, 256, 0, c->stream>>>(nx, ny, nz, batch, 0, src, nullptr, d_kx, d_ky, d_kz, dst);
+            sample_op(c, nx, ny, nz, batch, 0, src, nullptr, d_kx, d_ky, d_kz, dst);
             std::swap(src, dst);  // src = A S^m d
             for (int m = 0; m < smooth; ++m) {  // src <- S^T src
-                k_sample_op<<<eb, 256, 0, c->stream>>>(nx, ny, nz, batch, 2, src, nullptr, d_kx, d_ky, d_kz, dst);
-                k_sample_op<<<eb, 256, 0, c->stream>>>(nx, ny, nz, batch, 3, dst, src, d_kx, d_ky, d_kz, V);
+                sample_op(c, nx, ny, nz, batch, 2, src, nullptr, d_kx, d_ky, d_kz, dst);
+                sample_op(c, nx, ny, nz, batch, 3, dst, src, d_kx, d_ky, d_kz, V);
                 std::swap(src, V);
                 if (V == Ad) std::swap(V, dst);
             }

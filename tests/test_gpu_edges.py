@@ -270,3 +270,37 @@ def test_compaction_splits(ctx, n):
         want, got = np.flatnonzero(fire), d_list.numpy()
         assert int(d_count.numpy()[0]) == len(want)
         assert np.array_equal(got[:len(want)], want) and (got[len(want):] == -7).all()
+
+
+# the smoothed A-norm loss's operator: rows of 16, 32 and 80 lanes (a row's
+# group in one wavefront, rows in one, a row over two), samples beside samples
+@pytest.mark.parametrize("nx,batch,smooth", [(64, 3, 1), (128, 1, 2), (320, 2, 1), (576, 1, 0)])
+def test_training_operator_rows(ctx, nx, batch, smooth):
+    """With all-zero parameters the network's output is zero and the loss is
+    (S^m t . A S^m t) / (t . A t).  Values carry a few dozen roundings of 2^-24
+    of what S and A subtract, the quotient is some 0.05 of that: 1e-4."""
+    import torch
+    from test_gpu_unet import apply_A, diag_A
+
+    from neuronephys_clean_amd.precond import UNet
+    ny, nz = 32, 32
+    rng = np.random.default_rng(nx)
+    r = rng.standard_normal((batch, nz, ny, nx)).astype(np.float32)
+    # the largest values where a row leaves a wavefront, and at the box's ends
+    e = (0.05 * rng.standard_normal(r.shape)).astype(np.float32)
+    for q in (0, nx - 1, min(255, nx - 1), min(256, nx - 1)):
+        e[..., q] = rng.standard_normal(r.shape[:-1])
+    faces = [rng.uniform(1, 60, sh).astype(np.float32) for sh in
+             ((batch, nz, ny, nx + 1), (batch, nz, ny + 1, nx), (batch, nz + 1, ny, nx))]
+    say("training operator", nx, batch, smooth)
+    net = UNet(ctx, params=np.zeros_like(UNet(ctx, seed=1).params()))
+    dr, de = DA.from_numpy(ctx, r), DA.from_numpy(ctx, e)
+    loss = net.train_step((nx, ny, nz), batch, dr, dr, de, 0.0, faces=[DA.from_numpy(ctx, a) for a in faces],
+                          smooth=smooth)
+    K = [torch.from_numpy(a.astype(np.float64)) for a in faces]
+    t = torch.from_numpy(e.astype(np.float64))
+    u = t
+    for _ in range(smooth):
+        u = u - (2.0 / 3.0) * apply_A(u, *K) / diag_A(*K)
+    ref = float(((u * apply_A(u, *K)).sum(dim=(1, 2, 3)) / (t * apply_A(t, *K)).sum(dim=(1, 2, 3))).mean())
+    assert abs(loss - ref) <= 1e-4 * ref
