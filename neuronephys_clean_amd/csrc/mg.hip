@@ -160,47 +160,8 @@ template <int T> __global__ __launch_bounds__(256) void k_mg_op(MgOp o, GridK g,
 // are dealt to the eight in turn) takes a contiguous eighth of the level.
 // Bound by memory: a Chebyshev sweep moves 36 bytes a cell, 256^3 150 -> 118
 // us (5.1 TB/s), 128^3 20 -> 11.6; the restricted residual 138 -> 87.
-typedef float f4_t __attribute__((ext_vector_type(4)));
-typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ f4_t ld4(const float* __restrict__ p) { return *reinterpret_cast<const f4u_t*>(p); }
-__device__ __forceinline__ void st4(float* p, f4_t v) { *reinterpret_cast<f4u_t*>(p) = v; }
-
-// A x at cells i .. i + 3 of a row, each in apply_at's operation order.
-// Every lane of the wavefront calls it (the lanes beside may hold the x
-// neighbours).
-__device__ __forceinline__ f4_t apply4(const float* __restrict__ x, const GridK& g, int i, int j, int k, f4_t& xc) {
-    const int64_t nx = g.nx, ny = g.ny, nxy = nx * ny;
-    const int64_t id = i + nx * (j + ny * k), fx = i + (nx + 1) * (j + ny * k), fy = i + nx * (j + (ny + 1) * k);
-    const f4_t zero = {0.f, 0.f, 0.f, 0.f};
-    const int lane = threadIdx.x & 63;
-    xc = ld4(x + id);
-    const f4_t kx = ld4(g.kx + fx), kym = ld4(g.ky + fy), kyp = ld4(g.ky + fy + nx), kzm = ld4(g.kz + id),
-               kzp = ld4(g.kz + id + nxy);
-    const f4_t ym = j > 0 ? ld4(x + id - nx) : zero, yp = j + 1 < g.ny ? ld4(x + id + nx) : zero;
-    const f4_t zm = k > 0 ? ld4(x + id - nxy) : zero, zp = k + 1 < g.nz ? ld4(x + id + nxy) : zero;
-    float l = __shfl_up(xc[3], 1, 64), r = __shfl_down(xc[0], 1, 64), k4 = __shfl_down(kx[0], 1, 64);
-    if (lane == 0 && i > 0) l = x[id - 1];
-    if (lane == 63 && i + 4 < g.nx) r = x[id + 4];
-    if (lane == 63 || i + 4 >= g.nx) k4 = g.kx[fx + 4];
-    if (i == 0) l = 0.f;
-    if (i + 4 >= g.nx) r = 0.f;
-    const float xl[4] = {l, xc[0], xc[1], xc[2]}, xr[4] = {xc[1], xc[2], xc[3], r}, kr[4] = {kx[1], kx[2], kx[3], k4};
-    f4_t o;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const float d = 1.0f + kx[e] + kr[e] + kym[e] + kyp[e] + kzm[e] + kzp[e];
-        float t = kx[e] * xl[e] + kr[e] * xr[e];
-        t = t + kym[e] * ym[e];
-        t = t + kyp[e] * yp[e];
-        t = t + kzm[e] * zm[e];
-        t = t + kzp[e] * zp[e];
-        o[e] = d * xc[e] - t;
-    }
-    return o;
-}
-
 // CHEB, JAC, RESTRICT and RESID on a level whose rows are a multiple of four
-// cells (mg_quads); a lane takes four fine cells of a row (RESTRICT: of the
+// cells (row_quads); a lane takes four fine cells of a row (RESTRICT: of the
 // four rows of two coarse cells).
 template <int T> __global__ __launch_bounds__(256) void k_mg_op4(MgOp o, GridK g, GridK gc) {
     const int q8 = (int)(gridDim.x >> 3), r8 = (int)(gridDim.x & 7), xcd = (int)(blockIdx.x & 7);
@@ -262,9 +223,6 @@ template <int T> __global__ __launch_bounds__(256) void k_mg_op4(MgOp o, GridK g
     if (T == MG_CHEB) st4(o.dvec + id, dn);
     st4(o.xout + id, out);
 }
-
-// whole 16-byte groups in a row and 32-bit cell counts
-bool mg_quads(const GridK& g) { return g.nx % 4 == 0 && (int64_t)g.nx * g.ny * g.nz < (int64_t)1 << 31; }
 
 // One visit (a V-cycle) of the levels of at most kMgSubCells cells by one
 // workgroup: a thread keeps its cells' operator, right-hand side, Chebyshev
@@ -607,7 +565,7 @@ nnx_status mg_vcycle(nnx_ctx* c, Mg& m, const float* r, float* z) {
         const GridK& gc = m.g[o.level + 1 < m.nlev ? o.level + 1 : o.level];
         const GridK& d = o.type == MG_RESTRICT ? gc : g;
         const unsigned blocks = row_blocks(d.ny, d.nz);
-        if (mg_quads(g) && o.type <= MG_RESID) {
+        if (row_quads(g) && o.type <= MG_RESID) {
             const unsigned b4 = (unsigned)(((int64_t)(g.nx / 4) * d.ny * d.nz + 255) / 256);
             switch (o.type) {
                 case MG_CHEB: k_mg_op4<MG_CHEB><<<b4, 256, 0, c->stream>>>(o, g, gc); break;

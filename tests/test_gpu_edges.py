@@ -251,6 +251,32 @@ def test_multigrid_row_groups(ctx, dims, nu, smoother, cycle, off):
     assert (z[:off] == 7.0).all() and (z[off + r.size:] == 7.0).all()
 
 
+# flexible CG's product: rows of whole 16-byte groups (eighths of the grid that
+# start inside a row, fewer groups than lanes) and rows that are not
+@pytest.mark.parametrize("dims", [(4, 4, 4), (12, 7, 5), (20, 33, 9), (260, 6, 7), (18, 9, 11)])
+def test_flexible_cg_row_groups(ctx, dims):
+    """The solution's residual against FP64 is what the solver reports:
+    fp32 solves stop at 1e-5, so 2e-5 (the vectors' own roundings, 2^-24 per
+    iteration, are far below)."""
+    import mg_ref
+    from neuronephys_clean_amd import host
+    nx, ny, nz = dims
+    say("fcg", dims)
+    rng = np.random.default_rng(nx + ny + nz)
+    c = (5.0 * np.exp(0.5 * rng.standard_normal((nz, ny, nx)))).astype(np.float32)
+    k = host.face_coefficients(c)
+    d = [DA.from_numpy(ctx, a) for a in k]
+    g = _lib.Grid(nx, ny, nz, 7, 0.0, 0.0, *(a.ptr for a in d))
+    b = rng.standard_normal((nz, ny, nx)).astype(np.float32)
+    db, dx = DA.from_numpy(ctx, b.ravel()), DA.zeros(ctx, b.size, np.float32)
+    o = _lib.CgOpts(rtol=1e-5, maxit=2000, precond=_lib.PRECOND_JACOBI, check_every=1, stall_iters=10)
+    res = _lib.CgResult()
+    ctx.call("nnx_fcg_solve", C.byref(g), None, None, db.ptr, dx.ptr, C.byref(o), C.byref(res))
+    assert res.converged
+    ax = mg_ref.apply(dx.numpy().reshape(b.shape).astype(np.float64), *(a.astype(np.float64) for a in k))
+    assert np.linalg.norm(b - ax) <= 2e-5 * np.linalg.norm(b)
+
+
 @pytest.mark.parametrize("n", [1, 64, 65, 4095, 4097, 262_145, (1 << 20) - 1, (1 << 20) + 1, 1_700_003])
 def test_compaction_splits(ctx, n):
     """The ascending list and its length on bitmaps that are empty, sparse,
