@@ -6,8 +6,8 @@
 // firing neurons, compacts them with thrust::copy_if, reads the count back to
 // the host and scatters with fp32 atomicAdd (order-nondeterministic).  Here:
 //   - spikes are a bitmap (one ballot word per 64 neurons);
-//   - the ascending list is built by one workgroup with a block scan, the
-//     count stays on the device;
+//   - the ascending list is built by blocks that each order their own words
+//     behind the popcount of the words before, the count stays on the device;
 //   - every target's input is summed over its spiking sources in ascending
 //     source order, so all modes are deterministic and WEIGHTED_PULL and
 //     WEIGHTED_EVENT are bit-identical.

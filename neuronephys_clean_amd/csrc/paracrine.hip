@@ -1358,11 +1358,13 @@ static nnx_status cg_mem_scratch(nnx_ctx* c, const char* prefix, const GridK& gk
     m->r = (float*)p[0], m->pa = (float*)p[1], m->pb = (float*)p[2], m->q = (float*)p[3];
     m->sc = (double*)p[4], m->fl = (int32_t*)p[5], m->part = (double*)p[6];
     m->xp = pad ? m->q : nullptr;
-    if (pad && gk.kind == 1) {
+    // (rows of whole groups: also where this x needs none, so that a captured
+    // solve of the same grid into an unaligned one finds it)
+    if (gk.kind == 1 && (pad || (gk.nx % 4 == 0 && gk.nx >= 12 && !gk.block))) {
         std::snprintf(nm, sizeof nm, "%s_xp", prefix);
         void* xpp;
         NNX_TRY(scratch(c, nm, n * 4, false, &xpp));
-        m->xp = (float*)xpp;
+        if (pad) m->xp = (float*)xpp;
     }
     return NNX_OK;
 }
