@@ -132,6 +132,18 @@ template <class F> __device__ __forceinline__ void for_rows(int nx, int ny, int 
     }
 }
 
+// The same flat over the grid, for any shape: for_rows leaves lanes idle on
+// rows shorter than a wavefront and wavefronts idle on grids of few long rows
+// (a pass of 1,000,000 x 1 x 1 in one wavefront: 1.1 ms; 3 us flat).  Two 32-bit
+// divisions a voxel (fewer than 2^32 of them, rows padded to four included).
+template <class F> __device__ __forceinline__ void for_voxels(int nx, int ny, int nz, F&& f) {
+    const int64_t n = (int64_t)nx * ny * nz, stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t id = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; id < n; id += stride) {
+        const uint32_t row = (uint32_t)id / (uint32_t)nx, k = row / (uint32_t)ny;
+        f((int)((uint32_t)id - row * (uint32_t)nx), (int)(row - k * (uint32_t)ny), (int)k, id);
+    }
+}
+
 // ---- four cells of a row per lane (variable coefficients) ----
 typedef float f4_t __attribute__((ext_vector_type(4)));
 typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));

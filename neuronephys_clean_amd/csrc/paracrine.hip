@@ -1072,7 +1072,7 @@ __global__ void k_dinv(GridK g, float* dinv) {
 
 // ---- the same on working vectors in rows of px >= nx voxels, zero beyond nx ----
 __global__ __launch_bounds__(256) void k_dinv_pad(GridK g, int px, float* __restrict__ dinv) {
-    for_rows(px, g.ny, g.nz, [&](int i, int j, int k, int64_t id) {
+    for_voxels(px, g.ny, g.nz, [&](int i, int j, int k, int64_t id) {
         dinv[id] = i < g.nx ? dinv_at(g, i + (int64_t)g.nx * (j + (int64_t)g.ny * k)) : 0.0f;
     });
 }
@@ -1081,7 +1081,7 @@ __global__ __launch_bounds__(256) void k_cg_init_pad(GridK g, int px, CgDev d, c
                                                      const float* __restrict__ x, int use_x0,
                                                      float* __restrict__ p0, float* __restrict__ xp) {
     double vb[1] = {0}, vu[2] = {0, 0};
-    for_rows(px, g.ny, g.nz, [&](int i, int j, int k, int64_t id) {
+    for_voxels(px, g.ny, g.nz, [&](int i, int j, int k, int64_t id) {
         float ri = 0.0f, xi = 0.0f;
         if (i < g.nx) {
             const int64_t e = i + (int64_t)g.nx * (j + (int64_t)g.ny * k);
@@ -1114,7 +1114,7 @@ __global__ __launch_bounds__(256) void k_cg_finish_pad(GridK g, CgDev d, const f
     const bool read_x = !(xzero && k == 0);
     const float alpha = pend ? (float)d.sc[SC_ALK + (k & 1)] : 0.0f;
     const float* __restrict__ p = (k & 1) ? pa : pb;
-    for_rows(g.nx, g.ny, g.nz, [&](int i, int j, int kk, int64_t id) {
+    for_voxels(g.nx, g.ny, g.nz, [&](int i, int j, int kk, int64_t id) {
         if (i >= g.nxr) return;
         const int64_t e = i + (int64_t)g.nxr * (j + (int64_t)g.ny * kk);
         const float xv = read_x ? xp[id] : 0.0f;
@@ -1131,7 +1131,7 @@ __global__ __launch_bounds__(256) void k_cg_finish_pad(GridK g, CgDev d, const f
 __global__ __launch_bounds__(256) void k_cg_init64(GridK g, int px, CgDev d, const double* __restrict__ r64,
                                                    double s) {
     double vu[2] = {0, 0};
-    for_rows(px, g.ny, g.nz, [&](int i, int j, int k, int64_t id) {
+    for_voxels(px, g.ny, g.nz, [&](int i, int j, int k, int64_t id) {
         const float ri = i < g.nx ? (float)(r64[i + (int64_t)g.nx * (j + (int64_t)g.ny * k)] * s) : 0.0f;
         d.r[id] = ri;
         vu[0] += (double)ri * (ri * dv(d, id));
@@ -1148,7 +1148,7 @@ __global__ __launch_bounds__(256) void k_true_res(GridK g, const U* __restrict__
                                                   const B* __restrict__ b, double* part,
                                                   double* __restrict__ r_out) {
     double v[2] = {0, 0};
-    for_rows(g.nx, g.ny, g.nz, [&](int i, int j, int k, int64_t id) {
+    for_voxels(g.nx, g.ny, g.nz, [&](int i, int j, int k, int64_t id) {
         const double bi = (double)b[id], r = bi - apply_at<double, U>(x, g, i, j, k);
         if (r_out) r_out[id] = r;
         v[0] += r * r;

@@ -158,6 +158,46 @@ def test_capturable_solve_allocates_once(var):
     assert free[1] == free[0]
 
 
+def _time(ctx, call, reps=4):
+    """Shortest of a few calls after one to warm up, in seconds."""
+    import time
+    ts = []
+    for _ in range(reps + 1):
+        ctx.synchronize()
+        t = time.perf_counter()
+        call()
+        ctx.synchronize()
+        ts.append(time.perf_counter() - t)
+    return min(ts[1:])
+
+
+@pytest.mark.parametrize("var", [False, True])
+@pytest.mark.parametrize("refine", [False, True])
+def test_solves_on_one_long_row(ctx, var, refine):
+    """Ten iterations and the closing FP64 residual on 1,000,000 x 1 x 1 cost a
+    small multiple of the same voxels as 100 x 100 x 100: no pass leaves a row to
+    one wavefront.  (A tile holds one row of its 4 to 32, and of its planes one:
+    1.4-2.8 times the cube's; 22-64 with single-wavefront passes.)"""
+    t = []
+    for dims in ((100, 100, 100), (1_000_000, 1, 1)):
+        g, og, keep = _operator(ctx, *dims, var)
+        n = 1_000_000
+        b = np.random.default_rng(1).standard_normal(n)
+        if refine:
+            db, dx = DA.from_numpy(ctx, b), DA.zeros(ctx, n, np.float64)
+            o = _lib.CgOpts(rtol=1e-14, maxit=10, precond=_lib.PRECOND_JACOBI, check_every=5)
+            t.append(_time(ctx, lambda: ctx._l.nnx_cg_solve_refine(ctx.h, C.byref(g), db.ptr, dx.ptr, C.byref(o), 1e-6,
+                                                                   2, None)))
+        else:
+            db, dx = DA.from_numpy(ctx, b.astype(np.float32)), DA.zeros(ctx, n, np.float32)
+            o = _lib.CgOpts(rtol=0.0, maxit=10, precond=_lib.PRECOND_JACOBI, check_every=5)
+            res = _lib.CgResult()
+            t.append(_time(ctx, lambda: ctx._l.nnx_cg_solve(ctx.h, C.byref(g), db.ptr, dx.ptr, C.byref(o),
+                                                            C.byref(res))))
+    say("one long row", var, refine, t, t[1] / t[0])
+    assert t[1] <= 10 * t[0]
+
+
 def _dst(b, c, axes=(0, 1, 2)):
     import scipy.fft
     lam = np.ones(b.shape)
