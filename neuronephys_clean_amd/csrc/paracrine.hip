@@ -1529,11 +1529,18 @@ static void cg_init_launch(nnx_ctx* c, const GridK& gk, CgHost& h, const float* 
 }
 
 // The iterations after an init: check_every at a time, then one status
-// kernel and a read-back (the first batch without waiting for the init: its
-// launches return at once if the init met the tolerance).
-static nnx_status cg_loop(nnx_ctx* c, CgHost& h, float* x, int maxit, int check_every, int xzero, int32_t* fl,
-                          double* sc) {
+// kernel and a read-back.  `started`: the start cannot meet the tolerance, so
+// the first batch goes out without a read-back (12 us) of the init; otherwise
+// the init is read first - check_every iterations past the end are two
+// launches each, 7.5 ms for 1000 of them.
+static nnx_status cg_loop(nnx_ctx* c, CgHost& h, float* x, int maxit, int check_every, int xzero, bool started,
+                          int32_t* fl, double* sc) {
     if (check_every < 1) check_every = 1;
+    if (!started) {
+        NNX_LAUNCHED(c);
+        NNX_TRY(cg_readback(c, h, fl, sc));
+        if (fl[FL_DONE]) return NNX_OK;
+    }
     int enq = 0;
     do {
         for (int q = 0; q < check_every && enq < maxit; ++q, ++enq) cg_iter_launch(c, h, enq, x, xzero);
@@ -1551,7 +1558,7 @@ static nnx_status cg_run(nnx_ctx* c, const GridK& gk, CgHost& h, const float* b,
     cg_init_launch(c, gk, h, b, x, use_x0, tol, abs_mode, maxit);
     int32_t fl[FL_N];
     double sc[SC_N];
-    NNX_TRY(cg_loop(c, h, x, maxit, check_every, 0, fl, sc));
+    NNX_TRY(cg_loop(c, h, x, maxit, check_every, 0, false, fl, sc));
     if (initdone) *initdone = fl[FL_INITDONE];
     cg_finish_launch(c, h, x);
     NNX_LAUNCHED(c);
@@ -2076,7 +2083,8 @@ nnx_status nnx_cg_solve_refine(nnx_ctx* c, const nnx_grid* g, const double* b, d
             double sc[SC_N];
             k_cg_init64<<<kRedBlocks, 256, 0, c->stream>>>(gk, h.gp.nx, h.d, (const double*)r64, s);
             k_cg_init_fin<<<1, 256, 0, c->stream>>>(h.d, tol, 0, o->maxit);
-            NNX_TRY(cg_loop(c, h, (float*)d, o->maxit, o->check_every, 1, fl, sc));
+            // (from zero, so only a tolerance of 1 or more is met at the start)
+            NNX_TRY(cg_loop(c, h, (float*)d, o->maxit, o->check_every, 1, tol < 1.0 && o->maxit > 0, fl, sc));
             cg_finish_launch(c, h, (float*)d, 1, x, 1.0 / s);
             NNX_LAUNCHED(c);
             inner_total += fl[FL_ITERS];

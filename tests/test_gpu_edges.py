@@ -198,6 +198,39 @@ def test_solves_on_one_long_row(ctx, var, refine):
     assert t[1] <= 10 * t[0]
 
 
+@pytest.mark.parametrize("dims,var", [((32, 32, 32), False), ((33, 20, 31), True)])
+def test_converged_guess_enqueues_nothing(ctx, dims, var):
+    """A solve whose start meets the tolerance (its own solution as the guess;
+    a zero right-hand side; a refinement whose inner tolerance is 1) costs the
+    same whatever check_every is: the iterations of a batch are not enqueued
+    before the start is known.  (1000 of them past the end: 7.5 ms, the solve 50 us.)"""
+    n = int(np.prod(dims))
+    g, og, keep = _operator(ctx, *dims, var)
+    b = np.random.default_rng(1).standard_normal(n).astype(np.float32)
+    db, dx, zero = DA.from_numpy(ctx, b), DA.zeros(ctx, n, np.float32), DA.zeros(ctx, n, np.float32)
+    o = _lib.CgOpts(rtol=1e-6, maxit=500, precond=_lib.PRECOND_JACOBI, check_every=1)
+    ctx.call("nnx_cg_solve", C.byref(g), db.ptr, dx.ptr, C.byref(o), None)
+    x = dx.numpy()
+    b64, x64 = DA.from_numpy(ctx, b.astype(np.float64)), DA.zeros(ctx, n, np.float64)
+    t = {}
+    for every in (1, 1000):
+        o = _lib.CgOpts(rtol=1e-5, maxit=2000, precond=_lib.PRECOND_JACOBI, check_every=every, use_x0=1)
+        res = _lib.CgResult()
+        t["guess", every] = _time(ctx, lambda: ctx.call("nnx_cg_solve", C.byref(g), db.ptr, dx.ptr, C.byref(o),
+                                                        C.byref(res)))
+        assert res.iters == 0 and res.converged and np.array_equal(dx.numpy(), x)
+        o2 = _lib.CgOpts(rtol=1e-5, maxit=2000, precond=_lib.PRECOND_JACOBI, check_every=every)
+        d0 = DA.from_numpy(ctx, b)
+        t["zero", every] = _time(ctx, lambda: ctx.call("nnx_cg_solve", C.byref(g), zero.ptr, d0.ptr, C.byref(o2), None))
+        assert not d0.numpy().any()
+        t["inner", every] = _time(ctx, lambda: ctx._l.nnx_cg_solve_refine(ctx.h, C.byref(g), b64.ptr, x64.ptr,
+                                                                          C.byref(o2), 1.0, 1, None))
+        assert not x64.numpy().any()
+    say("converged guess", dims, var, {k: f"{v * 1e6:.0f} us" for k, v in t.items()})
+    for k in ("guess", "zero", "inner"):
+        assert t[k, 1000] <= 5 * t[k, 1]
+
+
 def _dst(b, c, axes=(0, 1, 2)):
     import scipy.fft
     lam = np.ones(b.shape)
