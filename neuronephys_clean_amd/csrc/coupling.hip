@@ -40,15 +40,23 @@ __global__ __launch_bounds__(256) void k_threshold(int64_t n, const T* __restric
 // pairs: the launch of parity s reads slot s and its last block writes slot
 // s^1, so no block reads a value that another block of the same launch
 // updates.
-// A thread emits the spikes of its own word one after the other where no word
-// of the block has more than kSerialSpikes; in other blocks the 64 lanes of a
+// A thread emits the spikes of its own words one after the other where no
+// thread of the block has more than kSerial; in other blocks the 64 lanes of a
 // wavefront emit a word's at once, the words and their offsets read back from
 // LDS (a third of 20,000 neurons firing: 4.6 us, 9.6 as up to 256 dependent
-// stores of a thread that owned four words).  W: 64 words up to kSmallWords
-// (more blocks, each with a short prefix), else 256.
+// stores of a thread that owned four words).  The lanes take a step for each
+// of the wavefront's W / 4 words, so the more words the later they pay.
+// W: 64 words up to kSmallWords (more blocks, each with a short prefix), 256 up
+// to kMidWords, 1024 (four words a thread) beyond: the prefixes read nwords^2 /
+// (2 W) words in all.  Times at no, 5% and 40% firing by blocks of 64, 256 and
+// 1024 words: 2,097,152 neurons 6.0, 8.1, 8.6 us against 5.2, 6.0, 12.6 and 5.2,
+// 7.8, 19.8; 4,194,304 13, 15, 17 against 7.8, 8.6, 15.7 and 7.7, 10.3, 23.1;
+// 8,388,608 by 256 and 1024 words 15.0, 15.9, 24.2 against 12.7, 15.5, 31.3;
+// 16,777,216 41, 43, 54 against 23, 26, 63; 67,108,864 595, 600, 619 against 193,
+// 204, 237.
 // ------------------------------------------------------------------------
-constexpr int kCB = 256, kSerialSpikes = 8;
-constexpr int64_t kSmallWords = 16384;
+constexpr int kCB = 256;
+constexpr int64_t kSmallWords = 16384, kMidWords = 65536;
 
 __device__ __forceinline__ int block_scan256(int v, int* total) {
     __shared__ int sh[4];
@@ -72,6 +80,8 @@ template <int W>
 __global__ __launch_bounds__(kCB) void k_compact(int64_t nwords, const uint64_t* __restrict__ bits,
                                                  int32_t* __restrict__ list,
                                                  int32_t* __restrict__ count, CompactExtras ex) {
+    constexpr int CW = W > kCB ? W / kCB : 1;    // consecutive words of a thread
+    constexpr int kSerial = W == 64 ? 8 : W == 256 ? 32 : 160;
     const int64_t b0 = blockIdx.x * (int64_t)W;  // first word of this block (< nwords)
     const bool a16 = ((uintptr_t)bits & 15) == 0;
     __shared__ uint64_t sw[W];
@@ -100,10 +110,14 @@ __global__ __launch_bounds__(kCB) void k_compact(int64_t nwords, const uint64_t*
     }
     int pre_tot;
     block_scan256((p0 + p1) + (p2 + p3), &pre_tot);
-    const int64_t w0 = b0 + (int64_t)threadIdx.x;
-    const uint64_t w = threadIdx.x < W && w0 < nwords ? bits[w0] : 0ull;
-    const int cnt = __popcll(w);
-    if (cnt > kSerialSpikes) dense = 1;  // (read after the scan's barriers)
+    const int64_t w0 = b0 + (int64_t)threadIdx.x * CW;
+    uint64_t w[CW];
+    int cnt = 0;
+#pragma unroll
+    for (int q = 0; q < CW; ++q) w[q] = threadIdx.x * CW < W && w0 + q < nwords ? bits[w0 + q] : 0ull;
+#pragma unroll
+    for (int q = 0; q < CW; ++q) cnt += __popcll(w[q]);
+    if (cnt > kSerial) dense = 1;  // (read after the scan's barriers)
     int tot;
     const int off = block_scan256(cnt, &tot);
     const int par = ex.parity;
@@ -122,7 +136,14 @@ __global__ __launch_bounds__(kCB) void k_compact(int64_t nwords, const uint64_t*
         if (ex.voxel_of) atomicAdd(&ex.voxel_counts[ex.voxel_of[idx]], 1);
     };
     if (dense) {
-        if (threadIdx.x < W) sw[threadIdx.x] = w, so[threadIdx.x] = off;
+        if (threadIdx.x * CW < W) {
+            int o = off;
+#pragma unroll
+            for (int q = 0; q < CW; ++q) {
+                sw[threadIdx.x * CW + q] = w[q], so[threadIdx.x * CW + q] = o;
+                o += __popcll(w[q]);
+            }
+        }
         __syncthreads();
         const int lane = threadIdx.x & 63;
 #pragma unroll 4
@@ -133,11 +154,14 @@ __global__ __launch_bounds__(kCB) void k_compact(int64_t nwords, const uint64_t*
         }
     } else if (cnt) {
         int64_t o = (int64_t)pre_tot + off;
-        uint64_t x = w;
-        while (x) {
-            const int b = __ffsll((unsigned long long)x) - 1;
-            x &= x - 1;
-            emit(o++, (int32_t)(w0 * 64 + b));
+#pragma unroll
+        for (int q = 0; q < CW; ++q) {
+            uint64_t x = w[q];
+            while (x) {
+                const int b = __ffsll((unsigned long long)x) - 1;
+                x &= x - 1;
+                emit(o++, (int32_t)((w0 + q) * 64 + b));
+            }
         }
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
@@ -627,11 +651,12 @@ namespace nnx {
 nnx_status compact_launch(nnx_ctx* c, int64_t n, const uint64_t* bits, int32_t* list,
                           int32_t* count, const CompactExtras& ex) {
     const int64_t nwords = ceil_div(n, 64);
-    if (nwords <= kSmallWords)
-        k_compact<64><<<(unsigned)std::max<int64_t>(1, ceil_div(nwords, 64)), kCB, 0, c->stream>>>(nwords, bits, list,
-                                                                                               count, ex);
-    else
-        k_compact<256><<<(unsigned)ceil_div(nwords, 256), kCB, 0, c->stream>>>(nwords, bits, list, count, ex);
+    auto go = [&](auto kernel, int W) {
+        kernel<<<(unsigned)std::max<int64_t>(1, ceil_div(nwords, W)), kCB, 0, c->stream>>>(nwords, bits, list, count, ex);
+    };
+    if (nwords <= kSmallWords) go(k_compact<64>, 64);
+    else if (nwords <= kMidWords) go(k_compact<256>, 256);
+    else go(k_compact<1024>, 1024);
     NNX_LAUNCHED(c);
     return NNX_OK;
 }

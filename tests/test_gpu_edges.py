@@ -379,7 +379,8 @@ def test_flexible_cg_row_groups(ctx, dims):
     assert np.linalg.norm(b - ax) <= 2e-5 * np.linalg.norm(b)
 
 
-@pytest.mark.parametrize("n", [1, 64, 65, 4095, 4097, 262_145, (1 << 20) - 1, (1 << 20) + 1, 1_700_003])
+@pytest.mark.parametrize("n", [1, 64, 65, 4095, 4097, 262_145, (1 << 20) - 1, (1 << 20) + 1, 1_700_003, 1 << 22,
+                               (1 << 22) + 1, 5_000_003])
 def test_compaction_splits(ctx, n):
     """The ascending list and its length on bitmaps that are empty, sparse,
     full and mixed (full words among empty ones), at the block sizes' edges;
@@ -398,6 +399,27 @@ def test_compaction_splits(ctx, n):
         want, got = np.flatnonzero(fire), d_list.numpy()
         assert int(d_count.numpy()[0]) == len(want)
         assert np.array_equal(got[:len(want)], want) and (got[len(want):] == -7).all()
+
+
+def test_compaction_of_large_networks(ctx):
+    """A spike list takes a time that grows with the network, not much faster:
+    eight times the neurons, none firing, at most six times as long (4.5; 8 with
+    a prefix over every 256 words), and at 5% firing at most twice as long as
+    without spikes (1.2; 2.3 with the words emitted one by one)."""
+    def words(n, frac):
+        fire = np.random.default_rng(n).random(n, dtype=np.float32) < frac
+        return DA.from_numpy(ctx, np.packbits(fire, bitorder="little").view(np.uint64))
+
+    def seconds(n, frac):
+        w, d_list, d_count = words(n, frac), DA(ctx, n, np.int32), DA.zeros(ctx, 1, np.int32)
+
+        def many():
+            for _ in range(50):
+                ctx.call("nnx_spike_compact", n, w.ptr, d_list.ptr, d_count.ptr)
+        return _time(ctx, many) / 50
+    small, large, firing = seconds(1 << 21, 0.0), seconds(1 << 24, 0.0), seconds(1 << 21, 0.05)
+    say("compact times", small, large, firing)
+    assert large <= 6 * small and firing <= 2 * small
 
 
 # the smoothed A-norm loss's operator: rows of 16, 32 and 80 lanes (a row's
