@@ -450,8 +450,10 @@ __global__ __launch_bounds__(1024) void k_pull_count(int64_t n, int64_t nnz, con
             const int32_t src[4] = {tl ? tv0 : v[u].x, tl ? tv1 : v[u].y, tl ? tv2 : v[u].z, v[u].w};
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const uint32_t w = LDSB ? sbits[src[k] >> 5] : gb[src[k] >> 5];
-                c += (int)((w >> (src[k] & 31)) & (uint32_t)(a + k >= e0) & (uint32_t)(a + k < e1));
+                const bool in = a + k >= e0 && a + k < e1;
+                // (in global memory an edge outside costs a transaction: not read)
+                const uint32_t w = LDSB ? sbits[src[k] >> 5] : in ? gb[src[k] >> 5] : 0u;
+                c += (int)((w >> (src[k] & 31)) & (uint32_t)in);
             }
         }
         return c;
@@ -487,14 +489,13 @@ __global__ __launch_bounds__(1024) void k_pull_count(int64_t n, int64_t nnz, con
 }
 
 // The same counts for larger networks: a wavefront streams the in-edge slab
-// of tg consecutive targets (lane j holds target j's end) in chunks of 256
+// of 64 consecutive targets (lane j holds target j's end) in chunks of 256
 // in-edges, three chunks of sources in flight at clamped addresses as in
 // k_pull_lds, and a chunk's four ballots give every target's lane the number
 // of spiking in-edges before its end; a target's count is the difference to
 // its predecessor's.
 template <class T>
-__global__ __launch_bounds__(1024) void k_pull_count_slab(int64_t n, int64_t nnz, int tg,
-                                                          const int32_t* __restrict__ in_off,
+__global__ __launch_bounds__(1024) void k_pull_count_slab(int64_t n, int64_t nnz, const int32_t* __restrict__ in_off,
                                                           const int32_t* __restrict__ in_src,
                                                           const uint64_t* __restrict__ bits, T* __restrict__ g) {
     extern __shared__ uint32_t sbits[];
@@ -510,14 +511,18 @@ __global__ __launch_bounds__(1024) void k_pull_count_slab(int64_t n, int64_t nnz
     __syncthreads();
     const int lane = threadIdx.x & 63;
     const int64_t nwaves = (int64_t)gridDim.x * 16;
-    for (int64_t t0 = (blockIdx.x * 16ll + (threadIdx.x >> 6)) * tg; t0 < n; t0 += nwaves * tg) {
-        const int cnt = (int)(n - t0 < tg ? n - t0 : tg);
+    for (int64_t t0 = (blockIdx.x * 16ll + (threadIdx.x >> 6)) * 64; t0 < n; t0 += nwaves * 64) {
+        const int cnt = (int)(n - t0 < 64 ? n - t0 : 64);
         const int32_t E0 = in_off[t0], S = E0 & ~3;
         const int32_t o1 = lane < cnt ? in_off[t0 + lane + 1] : E0, E1 = rdl(o1, cnt - 1);
         const int32_t nch = E1 > S ? (E1 - S + 255) >> 8 : 0;
+        // (clamped to the slab's last group: the chunks past it fetch nothing new)
+        int32_t qlim = (E1 - 1) & ~3;
+        qlim = qlim < qmax ? qlim : qmax;
+        qlim = qlim > 0 ? qlim : 0;
         auto load = [&](int32_t c) {
             const int32_t q = S + c * 256 + 4 * lane;
-            return *reinterpret_cast<const int4*>(in_src + (q < qmax ? q : qmax));
+            return *reinterpret_cast<const int4*>(in_src + (q < qlim ? q : qlim));
         };
         int4 ring[4];
 #pragma unroll
@@ -568,21 +573,26 @@ static void pull_count_launch(nnx_ctx* c, const nnx_graph* g, const uint64_t* bi
 }
 
 // More than half the LDS bitmap's network: slabs (a lane-per-target split has
-// too little in flight with one workgroup per CU: 1,048,576 x 50 39.5 against
-// 45.4 us, x 200 154 against 175), 64 targets a wavefront, 32 where 64 would
-// be a few chunks only (x 50: 39.5 against 46.7).  Below, S lanes a target,
-// about two rounds of them: 400,000 x 50 19.5 us (4 lanes, 2 in flight)
-// against 22.5 by slabs, 100,003 x 100 10.1 (8 lanes, 4 in flight) against
-// 11.0-20.7.
+// too little in flight with one workgroup per CU: 1,048,576 x 50 45 us, x 200
+// 175; by slabs 38 and 151 at 0.1% firing, 45 and 157 at 5%, where summing
+// ones took 40 and 151, 113 and 361.  Slabs of 32 targets are 16 us against 17
+// at 600,000 x 20, 27 against 29 at x 60, but 19 against 13 at 800,000 x 8 and 28
+// against 24 at 700,000 x 40, where the last round of wavefronts is nearly
+// empty).  Below, S lanes a target, about two rounds of them: 400,000 x 50 19.5
+// us (4 lanes, 2 in flight) against 22.5 by slabs, 100,003 x 100 10.1 (8 lanes, 4
+// in flight) against 11.0-20.7.  Above the LDS bitmap S lanes too, the bits of
+// the in-edges alone read from global memory (random 8-byte reads, the bound):
+// 1,048,640 x 8, 50 and 200 at 0.1% firing 36, 184 and 802 us, 4,194,304 x 50 924,
+// 3,145,728 x 150 2,046 at any rate; a wavefront a target (k_pull) 249, 269, 871,
+// 1,381 and 2,256, more at higher rates.
 template <class T>
 static void pull_count(nnx_ctx* c, const nnx_graph* g, const uint64_t* bits, T* out) {
     const int64_t n = g->n, deg = g->nnz / n;
     if (n > kLdsBitsMax / 2 && n <= kLdsBitsMax) {
-        const int tg = deg >= 64 ? 64 : 32;
         const size_t lds = (size_t)ceil_div(n, 64) * 8;
         const int64_t cap = lds <= (64 << 10) ? 512 : 256;
-        k_pull_count_slab<T><<<(unsigned)std::min(ceil_div(n, 16 * tg), cap), 1024, lds, c->stream>>>(
-            n, g->nnz, tg, g->in_offsets, g->in_sources, bits, out);
+        k_pull_count_slab<T><<<(unsigned)std::min(ceil_div(n, 16 * 64), cap), 1024, lds, c->stream>>>(
+            n, g->nnz, g->in_offsets, g->in_sources, bits, out);
         return;
     }
     if (deg <= 64) pull_count_launch<T, 4, 2>(c, g, bits, out);

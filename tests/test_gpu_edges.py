@@ -25,6 +25,19 @@ def free_bytes(ctx):
     return free.value
 
 
+def _time(ctx, call, reps=4):
+    """Shortest of a few calls after one to warm up, in seconds."""
+    import time
+    ts = []
+    for _ in range(reps + 1):
+        ctx.synchronize()
+        t = time.perf_counter()
+        call()
+        ctx.synchronize()
+        ts.append(time.perf_counter() - t)
+    return min(ts[1:])
+
+
 def _csc(n, nnz, seed):
     """Random in-edges, sorted per target, with empty targets and one hub."""
     rng = np.random.default_rng(seed)
@@ -36,7 +49,7 @@ def _csc(n, nnz, seed):
     return off, rng.integers(0, n, nnz, dtype=np.int32)
 
 
-# lanes per target (few and many in-edges), slabs of 32 and 64 targets, and
+# lanes per target (few and many in-edges), slabs of 64 targets, and
 # the bitmap in global memory; every residue of the CSC length mod 4
 @pytest.mark.parametrize("n,nnz", [(130, 4), (1500, 45_001), (1500, 150_001), (1500, 150_002), (1500, 150_003),
                                    ((1 << 19) + 65, 2_000_002), ((1 << 19) + 1, 34_000_001),
@@ -56,6 +69,27 @@ def test_count_coupling_splits(ctx, n, nnz):
             bits, out = DA.from_numpy(ctx, words), DA.from_numpy(ctx, np.full(n, np.nan, T))
             ctx.call("nnx_couple", C.byref(g), _lib.COUPLE_COUNT, DT[T], bits.ptr, None, None, None, out.ptr)
             assert np.array_equal(out.numpy(), (cum[off[1:]] - cum[off[:-1]]).astype(T))
+
+
+def test_count_coupling_above_the_lds_bitmap(ctx):
+    """Counting is no slower than the general kernel (which takes a source
+    array off the 16-byte grid) where the spike bits are read from global
+    memory and few neurons fire: 0.9 of its time; 1.07 when the bits of in-edges
+    outside a target's range were read as well."""
+    n, deg = (1 << 20) + 64, 200
+    src = np.random.default_rng(1).integers(0, n, n * deg + 4, dtype=np.int32)
+    d_src = DA.from_numpy(ctx, src)
+    d_off = DA.from_numpy(ctx, np.arange(n + 1, dtype=np.int32) * deg)
+    fire = np.random.default_rng(2).random(n) < 0.001
+    bits, out = DA.from_numpy(ctx, np.packbits(fire, bitorder="little").view(np.uint64)), DA.zeros(ctx, n, np.float32)
+    t = []
+    for shift in (0, 1):
+        g = _lib.Graph(n=n, nnz=n * deg, in_offsets=d_off.ptr, in_sources=d_src.ptr + 4 * shift)
+        t.append(_time(ctx, lambda: ctx.call("nnx_couple", C.byref(g), _lib.COUPLE_COUNT, _lib.F32, bits.ptr, None,
+                                             None, None, out.ptr)))
+        assert np.array_equal(out.numpy(), fire[src[shift:shift + n * deg]].reshape(n, deg).sum(1).astype(np.float32))
+    say("count above the LDS bitmap", t)
+    assert t[0] <= t[1]
 
 
 def _operator(ctx, nx, ny, nz, var, seed=6):
@@ -156,19 +190,6 @@ def test_capturable_solve_allocates_once(var):
         ctx.synchronize()
         free.append(free_bytes(ctx))
     assert free[1] == free[0]
-
-
-def _time(ctx, call, reps=4):
-    """Shortest of a few calls after one to warm up, in seconds."""
-    import time
-    ts = []
-    for _ in range(reps + 1):
-        ctx.synchronize()
-        t = time.perf_counter()
-        call()
-        ctx.synchronize()
-        ts.append(time.perf_counter() - t)
-    return min(ts[1:])
 
 
 @pytest.mark.parametrize("var", [False, True])
