@@ -1332,9 +1332,14 @@ CgMem cg_mem_carve(void* base, const nnx_grid* g, int precond, const float* x) {
     return m;
 }
 
-// the working set from the context's named scratch buffers `prefix`_*
+// The working set from the context's named scratch buffers `prefix`_*.  The
+// padded iterate's own vector (variable coefficients) is taken where the solve
+// needs it, for the capturable solve (kXpAnyX) also on rows of whole groups
+// into an x that needs none, so that a captured solve of the same grid into an
+// unaligned one finds it; kXpNone: only the partials are used.
+enum { kXpNone, kXpPadded, kXpAnyX };
 static nnx_status cg_mem_scratch(nnx_ctx* c, const char* prefix, const GridK& gk, int precond, const float* x,
-                                 CgMem* m) {
+                                 CgMem* m, int xp = kXpPadded) {
     bool pad;
     cg_fast(gk, precond, x, &pad);
     const GridK gp = pad ? padded_grid(gk) : gk;
@@ -1358,9 +1363,7 @@ static nnx_status cg_mem_scratch(nnx_ctx* c, const char* prefix, const GridK& gk
     m->r = (float*)p[0], m->pa = (float*)p[1], m->pb = (float*)p[2], m->q = (float*)p[3];
     m->sc = (double*)p[4], m->fl = (int32_t*)p[5], m->part = (double*)p[6];
     m->xp = pad ? m->q : nullptr;
-    // (rows of whole groups: also where this x needs none, so that a captured
-    // solve of the same grid into an unaligned one finds it)
-    if (gk.kind == 1 && (pad || (gk.nx % 4 == 0 && gk.nx >= 12 && !gk.block))) {
+    if (gk.kind == 1 && ((pad && xp != kXpNone) || (xp == kXpAnyX && gk.nx % 4 == 0 && gk.nx >= 12))) {
         std::snprintf(nm, sizeof nm, "%s_xp", prefix);
         void* xpp;
         NNX_TRY(scratch(c, nm, n * 4, false, &xpp));
@@ -1411,9 +1414,10 @@ static nnx_status cg_bind(nnx_ctx* c, const GridK& gk, int precond, const float*
     return NNX_OK;
 }
 
-static nnx_status cg_buffers(nnx_ctx* c, const GridK& gk, int precond, const float* x, CgHost* h) {
+static nnx_status cg_buffers(nnx_ctx* c, const GridK& gk, int precond, const float* x, CgHost* h,
+                             int xp = kXpPadded) {
     CgMem m;
-    NNX_TRY(cg_mem_scratch(c, "cg", gk, precond, x, &m));
+    NNX_TRY(cg_mem_scratch(c, "cg", gk, precond, x, &m, xp));
     return cg_bind(c, gk, precond, x, m, h);
 }
 
@@ -2051,12 +2055,12 @@ nnx_status nnx_cg_solve_refine(nnx_ctx* c, const nnx_grid* g, const double* b, d
     const GridK gk = make_grid(g);
     const int64_t n = (int64_t)gk.nx * gk.ny * gk.nz;
     auto t0 = std::chrono::steady_clock::now();
-    void *r64, *rhs, *d;
+    void *r64, *rhs = nullptr, *d;
     NNX_TRY(scratch(c, "ir_r64", n * 8, false, &r64));
-    NNX_TRY(scratch(c, "ir_rhs", n * 4, false, &rhs));
     NNX_TRY(scratch(c, "ir_d", n * 4, false, &d));
     CgHost h;
     NNX_TRY(cg_buffers(c, gk, o->precond, (const float*)d, &h));
+    if (!h.fast) NNX_TRY(scratch(c, "ir_rhs", n * 4, false, &rhs));
     if (!o->use_x0) NNX_HIP(c, hipMemsetAsync(x, 0, n * 8, c->stream));
     nnx_cg_result out{};
     int outer = 0, inner_total = 0;
@@ -2249,7 +2253,7 @@ extern "C" nnx_status nnx_cg_solve_async(nnx_ctx* c, const nnx_grid* g, const fl
     NNX_TRY(cg_async_check(c, g, b, x, o, d_result));
     const GridK gk = make_grid(g);
     CgMem m;
-    NNX_TRY(cg_mem_scratch(c, "cga", gk, o->precond, x, &m));
+    NNX_TRY(cg_mem_scratch(c, "cga", gk, o->precond, x, &m, kXpAnyX));
     return cg_async_launch(c, g, b, x, o, d_result, m);
 }
 
@@ -2420,7 +2424,7 @@ nnx_status nnx_fcg_solve(nnx_ctx* c, const nnx_grid* g, nnx_unet* net, const flo
                     o->smooth, &r));
     auto t1 = std::chrono::steady_clock::now();
     CgHost h;
-    NNX_TRY(cg_buffers(c, gk, NNX_PRECOND_NONE, nullptr, &h));
+    NNX_TRY(cg_buffers(c, gk, NNX_PRECOND_NONE, nullptr, &h, kXpNone));
     NNX_TRY((true_residual<float, float>(c, gk, h, x, b, &r.true_relres, nullptr, nullptr)));
     r.ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
     if (res) *res = r;
@@ -2438,7 +2442,7 @@ nnx_status nnx_fcg_solve_refine(nnx_ctx* c, const nnx_grid* g, nnx_unet* net, co
     const int64_t n = (int64_t)gk.nx * gk.ny * gk.nz;
     auto t0 = std::chrono::steady_clock::now();
     CgHost h;
-    NNX_TRY(cg_buffers(c, gk, NNX_PRECOND_NONE, nullptr, &h));
+    NNX_TRY(cg_buffers(c, gk, NNX_PRECOND_NONE, nullptr, &h, kXpNone));
     void *r64, *rhs, *d;
     NNX_TRY(scratch(c, "ir_r64", n * 8, false, &r64));
     NNX_TRY(scratch(c, "ir_rhs", n * 4, false, &rhs));

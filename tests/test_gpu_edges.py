@@ -219,6 +219,36 @@ def test_solves_on_one_long_row(ctx, var, refine):
     assert t[1] <= 10 * t[0]
 
 
+@pytest.mark.parametrize("call,vectors", [("solve", 5), ("refine", 8), ("fcg", 11), ("capturable", 6)])
+def test_working_memory(call, vectors):
+    """The device memory a new context's first solve on 128^3 with variable
+    coefficients takes, in fp32 vectors of the grid (8 MiB): r, two directions,
+    q and the inverse diagonal; a refinement's FP64 residual (two) and
+    correction; flexible CG's seven and the residual's four; the capturable
+    solve's vector for an unaligned x.  Reductions and state: under 4 MiB."""
+    ctx = _lib.Context(0)
+    n = 128 ** 3
+    g, og, keep = _operator(ctx, 128, 128, 128, True)
+    T = np.float64 if call == "refine" else np.float32
+    db, dx = DA.from_numpy(ctx, np.ones(n, T)), DA.zeros(ctx, n + 4, T)
+    res = DA.zeros(ctx, 4, np.float64)
+    o = _lib.CgOpts(rtol=1e-2, maxit=200, precond=_lib.PRECOND_JACOBI, check_every=4)
+    ctx.synchronize()
+    before = free_bytes(ctx)
+    if call == "solve":
+        ctx.call("nnx_cg_solve", C.byref(g), db.ptr, dx.ptr, C.byref(o), None)
+    elif call == "refine":
+        ctx.call("nnx_cg_solve_refine", C.byref(g), db.ptr, dx.ptr, C.byref(o), 1e-2, 5, None)
+    elif call == "fcg":
+        ctx.call("nnx_fcg_solve", C.byref(g), None, None, db.ptr, dx.ptr, C.byref(o), None)
+    else:
+        ctx.call("nnx_cg_solve_async", C.byref(g), db.ptr, dx.ptr, C.byref(o), res.ptr)
+    ctx.synchronize()
+    used = (before - free_bytes(ctx)) / 4.0 / n
+    say("working memory", call, used, "vectors")
+    assert vectors <= used <= vectors + 0.5
+
+
 @pytest.mark.parametrize("dims,var", [((32, 32, 32), False), ((33, 20, 31), True)])
 def test_converged_guess_enqueues_nothing(ctx, dims, var):
     """A solve whose start meets the tolerance (its own solution as the guess;
