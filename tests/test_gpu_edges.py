@@ -315,6 +315,69 @@ def test_paracrine_step_on_ragged_grids(ctx, dims):
     assert sim.paracrine_stats()["unconverged"] == 0
 
 
+# variable coefficients: rows of whole groups, with ky and kz off the 16-byte
+# grid too (padded working rows), of each other residue, the shortest padded
+# row, shorter ones (the generic kernels); and a constant field off 16 bytes
+@pytest.mark.parametrize("dims,var,foff,coff", [((36, 33, 34), True, 0, 0), ((36, 33, 34), True, 1, 0),
+                                                ((33, 35, 37), True, 0, 0), ((34, 33, 30), True, 0, 1),
+                                                ((35, 34, 33), True, 3, 0), ((13, 40, 41), True, 0, 0),
+                                                ((11, 40, 41), True, 0, 0), ((36, 33, 34), False, 0, 1),
+                                                ((35, 33, 34), False, 0, 1)])
+@pytest.mark.parametrize("graph", [False, True])
+def test_paracrine_step_with_face_coefficients(ctx, dims, var, foff, coff, graph):
+    """In-step solves, the first on a zero field without releases, the later
+    ones from the field before, and between them one of another simulation on
+    another grid in the same context (the inverse diagonal is kept per grid):
+    each field by its FP64 residual with the oracle's operator on what it
+    consumed, no neighbour of the field written, and a field that already meets
+    the tolerance left as it is."""
+    import oracle
+    from neuronephys_clean_amd import configs
+    from neuronephys_clean_amd.sim import Simulation
+    nx, ny, nz = dims
+    n = nx * ny * nz
+
+    def start(dims, seed, foff, var=True):
+        nx, ny, nz = dims
+        k = [np.random.default_rng(seed + q).uniform(0.1, 2, sh).astype(np.float32)
+             for q, sh in enumerate(((nz, ny, nx + 1), (nz, ny + 1, nx), (nz + 1, ny, nx)))]
+        if not var:
+            k = []
+        d = [DA.from_numpy(ctx, np.concatenate([np.zeros(foff, np.float32), a.ravel()])) for a in k]
+        f = [a.ptr + 4 * foff for a in d] if var else [None] * 3
+        net = configs.c1(seed=0)
+        net.grid, net.voxel = dims, None
+        sim = Simulation(net, np.float32, couple="event", record_cap=1 << 16, deposit=True, ctx=ctx)
+        sim.set_paracrine(20, max_inner=40, max_outer=3, grid=_lib.Grid(nx, ny, nz, 7, 0.0 if var else 1.3, 0.0, *f))
+        sim.keep = d
+        return sim, oracle.grid(nx, ny, nz, 7, 0.0 if var else 1.3, 0.0, *(k or [None] * 3))
+    sim, og = start(dims, 1, foff, var)
+    other, _ = start((nx + 4, ny, nz), 5, 0)
+    field = DA.from_numpy(ctx, np.concatenate([np.full(coff, 7.0), np.zeros(n), [7.0]]))
+    sim.plan.paracrine.conc = field.ptr + 8 * coff
+    say("in-step faces", dims, var, foff, coff, graph)
+    for w in range(5):
+        before = field.numpy()[coff:coff + n]
+        counts = np.random.default_rng(w).poisson(0.05 if 0 < w < 4 else 0.0, n).astype(np.int32)
+        sim.a["voxel_counts"].upload(counts)
+        if w == 4:  # nothing released, and any field will do
+            sim.plan.paracrine.rtol = 1e9
+        sim.run(20, use_graph=graph, chunk=20)
+        after = field.numpy()
+        assert (after[:coff] == 7.0).all() and after[coff + n] == 7.0
+        after = after[coff:coff + n]
+        st = sim.paracrine_stats()
+        if w == 0 or w == 4:
+            assert np.array_equal(after, before) and st["last_inner_iters"] == 0
+            continue
+        b = before + sim.net.amount * counts.astype(np.float64)
+        rel = np.linalg.norm(b - oracle.apply(og, after)) / np.linalg.norm(b)
+        say("  solve", w, int(counts.sum()), rel, st["last_inner_iters"], st["last_outer_steps"])
+        assert rel <= 1e-8 and st["unconverged"] == 0 and st["last_outer_steps"] >= 2
+        if w == 2:
+            other.run(20, use_graph=graph, chunk=20)
+
+
 @pytest.mark.parametrize("dims,block,off", [((64, 33, 20), 0, 1), ((50, 33, 20), 0, 1), ((32, 32, 16), 16, 1),
                                             ((32, 32, 16), 16, 0), ((256, 256, 208), 0, 0), ((8, 9, 10), 0, 1)])
 def test_refinement_on_unaligned_fields(ctx, dims, block, off):
