@@ -231,8 +231,9 @@ __global__ __launch_bounds__(256) void k_cg_status(CgDev d) {
 // marches kZ4 planes in z (DYN: zdyn of them); thread (lx, ly) holds x = 4lx ..
 // 4lx+3 of row ly as a float4.  tile_shape has the choice.  Each plane (plus
 // its one-voxel halo in x and y) goes into a double-buffered LDS tile; the
-// column's z neighbours stay in registers; the next plane's loads are issued before the plane's barrier (a barrier drains outstanding loads,
-// so 16-byte loads per thread are what keeps enough bytes in flight).
+// column's z neighbours stay in registers; the next plane's loads are issued
+// before the plane's barrier (a barrier drains outstanding loads, so 16-byte
+// loads per thread are what keeps enough bytes in flight).
 // Requires nx % 4 == 0 (16-byte aligned rows).
 //   MODE 0: y = A src (summation order of the CPU restatement); dst = y.
 //   MODE 2: CG iteration k, first half - p_new = dinv r + beta p_old at
@@ -247,21 +248,19 @@ __global__ __launch_bounds__(256) void k_cg_status(CgDev d) {
 //           partials of r . dinv r and r . r.  12 B per voxel.
 // The last iteration's x += alpha p is left to k_cg_finish.  Together the
 // two halves move 32 B per voxel where storing q would take 40.
-// PF: planes loaded ahead of the one being computed.  With 1, plane k+1's
-// loads are issued at the start of plane k and its z+1 neighbours wait for
-// them; with 2 they were issued one plane earlier, which hides a memory
-// latency per plane (a workgroup marches its tile alone on its CU) - but the
-// direction is formed from the values as they are loaded, so every load is
-// still waited for in the step that issues it.  3, the deferred form: the
-// raw values are loaded two planes ahead at clamped addresses, with no
-// arithmetic and no condition at the load, and finished one step later.
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // 16 bytes at a 4-byte address
+// PF: planes loaded ahead of the one being computed.  With 2, plane k+1's
+// loads were issued before plane k's step, which hides a memory latency per
+// plane (a workgroup marches its tile alone on its CU) - but the direction is
+// formed from the values as they are loaded, so every load is still waited
+// for in the step that issues it.  3, the deferred form: the raw values are
+// loaded two planes ahead at clamped addresses, with no arithmetic and no
+// condition at the load, and finished one step later.
 constexpr int kTX4 = 256, kTY4 = 16, kZ4 = 16, kT4 = 64 * kTY4;
 // prefetch forms and tile heights the solver launches (measured at 256^3):
 // the apply and the variable-coefficient first half take the deferred form;
-// the constant-coefficient iteration on 1024-thread tiles stays at PF 2 (the deferred form for
-// its second half or for both halves: 98.1-98.5 us per iteration against
-// 96.3-96.6), its first half on 16-row tiles and its second half on 4-row
+// the constant-coefficient iteration on 1024-thread tiles stays at PF 2 (the
+// deferred form for its second half or for both halves: 98.1-98.5 us per
+// iteration against 96.3-96.6), its first half on 16-row tiles and its second half on 4-row
 // tiles, four 256-thread workgroups per CU (94.4-94.5 us per iteration
 // against 97.7-97.9 with 16 rows and 96.2 with 8; the first half on 8 or
 // 4 rows: 95.2 and 95.6); the apply on 8-row tiles (21.8 us at 256^3
@@ -287,8 +286,9 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
     const int kZs = DYN ? zdyn : kZ4;          // planes it marches (DYN: even)
     static_assert(!DYN || PF == 3, "the deferred form for a march of any length");
     static_assert(MODE == 0 || MODE == 2 || MODE == 3, "mode");
-    static_assert(PF == 1 || PF == 2 || PF == 3, "prefetch form");
-    static_assert(!VAR || MODE == 2, "variable coefficients: the first half only (k_cg_rupd is the second)");
+    static_assert(PF == 2 || PF == 3, "prefetch form");
+    static_assert(!VAR || (MODE == 2 && PF == 3),
+                  "variable coefficients: the first half only (k_cg_rupd is the second), deferred");
     __shared__ float t[2][R + 2][kRowS];
     float beta = 0.0f, di = 1.0f, alpha = 0.0f;
     // the scalars in one round of loads: the done flag, r.z and alpha of
@@ -396,17 +396,14 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
             return use_pold ? d.r[e] * de + beta * pold[e] : d.r[e] * de;
         };
         // the own column: the tile value, and p_old and x (MODE 2) or r
-        // (MODE 3) of the same point.  MODE 2 with PF >= 2 reads x only in
-        // its own plane's step (it is not a neighbour value: registers).
-        constexpr bool late_x = MODE == 2 && PF >= 2;
+        // (MODE 3) of the same point.  MODE 2 reads x only in its own plane's
+        // step (it is not a neighbour value: registers).
+        constexpr bool late_x = MODE == 2;
         auto own4 = [&](bool ok, int64_t e, float4& po, float4& xr) -> float4 {
             po = z4;
             xr = z4;
             if (!ok) return z4;
-            if (MODE == 2) {
-                if (use_pold && read_x && !late_x) xr = *reinterpret_cast<const float4*>(dst + e);
-                return dir4(e, po);
-            }
+            if (MODE == 2) return dir4(e, po);
             if (MODE == 3) xr = *reinterpret_cast<const float4*>(d.r + e);
             return *reinterpret_cast<const float4*>(src + e);
         };
@@ -472,7 +469,7 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
         RawR rwr;
         RawC rwc;
         bool rok_o = false, rok_r = false, rok_c = false;
-        // VAR with PF == 3: the next plane's face coefficients of the own
+        // VAR: the next plane's face coefficients of the own
         // voxels, loaded a plane ahead (element 0 for a plane past the grid);
         // the z face below a plane is the one above the plane before it
         float nkx[5] = {0, 0, 0, 0, 0};
@@ -483,7 +480,7 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
         // entries and shifted
         auto ldu = [&](const float* f, int64_t e, int64_t tot) -> float4 {
             const int64_t ec = e < tot - 4 ? e : tot - 4;
-            const f4u v = *reinterpret_cast<const f4u*>(f + ec);
+            const f4u_t v = *reinterpret_cast<const f4u_t*>(f + ec);
             const int sh = (int)(e - ec);
             return make_float4(sh == 0 ? v.x : sh == 1 ? v.y : sh == 2 ? v.z : v.w,
                                sh == 0 ? v.y : sh == 1 ? v.z : v.w, sh == 0 ? v.z : v.w, v.w);
@@ -544,12 +541,7 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
             const int b = (kz - k0) & 1;
             float4 pp, pop, xrp, hr;
             float hc;
-            if (PF == 1) {
-                const bool nxt = kz + 1 < nz;
-                pp = own4(own && nxt, ocol + sxy * (kz + 1), pop, xrp);
-                hr = val4(hr_ok && nxt, rcol + sxy * (kz + 1));
-                hc = val1(hc_ok && nxt, ccol + sxy * (kz + 1));
-            } else if (PF == 2) {
+            if (PF == 2) {
                 pp = pp1, pop = pop1, xrp = xrp1, hr = hr1, hc = hc1;
                 const bool n2 = kz + 2 < nz && kz + 2 <= kend;
                 pp1 = own4(own && n2, ocol + sxy * (kz + 2), pop1, xrp1);
@@ -573,7 +565,7 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
             // the row; ky: rows j and j+1; kz: planes kz and kz+1)
             float kxf[5] = {0, 0, 0, 0, 0};
             float4 kym = z4, kyp = z4, kzm = z4, kzp = z4;
-            if (VAR && PF == 3) {
+            if (VAR) {
 #pragma unroll
                 for (int q = 0; q < 5; ++q) kxf[q] = nkx[q];
                 kym = nkym, kyp = nkyp, kzm = ckzm, kzp = nkzp;
@@ -581,16 +573,6 @@ __global__ __launch_bounds__(64 * TY) void k_stencil7x4(GridK g, CgDev d, int k,
                 ld_faces(kz + 1);
             }
             if (PF == 2 && late_x && own && read_x) xrc = *reinterpret_cast<const float4*>(dst + ocol + sxy * kz);
-            if (VAR && PF != 3 && own) {
-                const float* kxr = g.kx + xo + (int64_t)(nx + 1) * (j + (int64_t)ny * kz);
-#pragma unroll
-                for (int q = 0; q < 5; ++q) kxf[q] = kxr[q];
-                const int64_t fy = xo + (int64_t)nx * (j + (int64_t)(ny + 1) * kz);
-                kym = *reinterpret_cast<const float4*>(g.ky + fy);
-                kyp = *reinterpret_cast<const float4*>(g.ky + fy + nx);
-                kzm = *reinterpret_cast<const float4*>(g.kz + ocol + sxy * kz);
-                kzp = *reinterpret_cast<const float4*>(g.kz + ocol + sxy * (kz + 1));
-            }
             __syncthreads();
             if (own) {
                 const float left = t[b][ly + 1][3 + 4 * lx], right = t[b][ly + 1][8 + 4 * lx];

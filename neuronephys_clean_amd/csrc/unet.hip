@@ -32,6 +32,7 @@
 #include <cstring>
 #include <vector>
 
+#include "grid_dev.h"
 #include "internal.h"
 
 namespace nnx {
@@ -839,6 +840,9 @@ __global__ void k_prep_w(PrepJobs jobs) {
     }
     a.out[i] = (uint16_t)f2bf(v);
 }
+
+// per-block FP64 partial sums of x^2 over batch member blockIdx.y (nper a
+// multiple of 4: the network's grids are)
 __global__ __launch_bounds__(256) void k_sumsq(const float* __restrict__ x, int64_t nper, double* __restrict__ part) {
     __shared__ double sh[4];
     const int b = blockIdx.y;
@@ -1113,9 +1117,6 @@ constexpr float kSmoothWTrain = 2.0f / 3.0f;
 // takes a contiguous eighth of the batch, so the rows above and below are in
 // its own L2.  Bound by memory (faces, field and result once): 8 x 64^3 16 us
 // by single voxels, 8 so (the division alone 6.3).
-typedef float f4_t __attribute__((ext_vector_type(4)));
-typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ f4_t ld4(const float* __restrict__ p) { return *reinterpret_cast<const f4u_t*>(p); }
 template <int MODE>
 __global__ __launch_bounds__(256) void k_sample_op(int nx, int ny, int nz, int batch, const float* __restrict__ x,
                                                     const float* __restrict__ x2, const float* __restrict__ kx,
@@ -1167,7 +1168,7 @@ __global__ __launch_bounds__(256) void k_sample_op(int nx, int ny, int nz, int b
             o[e] = MODE == 0 ? ax : MODE == 1 ? xc[e] - kSmoothWTrain * ax / dg : o2[e] - kSmoothWTrain * ax;
         }
     }
-    if (mine < n4) *reinterpret_cast<f4u_t*>(out + g) = o;
+    if (mine < n4) st4(out + g, o);
 }
 void sample_op(nnx_ctx* c, int nx, int ny, int nz, int batch, int mode, const float* x, const float* x2,
                const float* kx, const float* ky, const float* kz, float* out) {
