@@ -257,15 +257,15 @@ __global__ __launch_bounds__(256) void k_cg_status(CgDev d) {
 // condition at the load, and finished one step later.
 constexpr int kTX4 = 256, kTY4 = 16, kZ4 = 16, kT4 = 64 * kTY4;
 // prefetch forms and tile heights the solver launches (measured at 256^3):
-// the apply and the variable-coefficient first half take the deferred form;
-// the constant-coefficient iteration on 1024-thread tiles stays at PF 2 (the
+// the apply and every march of any length take the deferred form; the
+// constant-coefficient iteration on 1024-thread tiles stays at PF 2 (the
 // deferred form for its second half or for both halves: 98.1-98.5 us per
-// iteration against 96.3-96.6), its first half on 16-row tiles and its second half on 4-row
-// tiles, four 256-thread workgroups per CU (94.4-94.5 us per iteration
-// against 97.7-97.9 with 16 rows and 96.2 with 8; the first half on 8 or
-// 4 rows: 95.2 and 95.6); the apply on 8-row tiles (21.8 us at 256^3
+// iteration against 96.3-96.6), its first half on 16-row tiles and its second
+// half on 4-row tiles, four 256-thread workgroups per CU (94.4-94.5 us per
+// iteration against 97.7-97.9 with 16 rows and 96.2 with 8; the first half on
+// 8 or 4 rows: 95.2 and 95.6); the apply on 8-row tiles (21.8 us at 256^3
 // against 22.2 with 16 rows and 22.3 with 4)
-constexpr int kPFa = 3, kPFv = 3, kPFc = 2, kTYc = kTY4, kTYc3 = 4, kTYa = 8;
+constexpr int kPFa = 3, kPFc = 2, kTYc = kTY4, kTYc3 = 4, kTYa = 8;
 
 // Tile of workgroup b in round `round` of a tiled launch of nb workgroups.
 // Workgroups are dealt to the 8 XCDs round-robin (b % 8), each XCD with its
@@ -955,9 +955,6 @@ __global__ __launch_bounds__(64 * TY) void k_res64x4(GridK g, const double* __re
         }
 }
 
-// rows per tile of the variable-coefficient iteration (512 threads: room for
-// the face coefficients' registers)
-constexpr int kTYv = 8;
 enum { kFastConst = 1, kFastVar = 2 };
 
 static int stencil4_blocks(const GridK& g, int ty = kTY4) {
@@ -1169,8 +1166,8 @@ static nnx_status check_grid(nnx_ctx* c, const nnx_grid* g) {
     return NNX_OK;
 }
 
-// Shape of the tiled iteration: lx = 0, the 256-wide tiles of 16 planes;
-// otherwise 256-thread tiles of 4 lx voxels by 256 / lx rows by zd planes.
+// Shape of the tiled iteration: lx = 0, the 256-wide tiles of 16 planes
+// (constant coefficients); otherwise 256-thread tiles of 4 lx voxels by 256 / lx rows by zd planes.
 struct CgShape {
     int lx, zd;
 };
@@ -1208,10 +1205,12 @@ struct CgHost {
 // 35.3; 200^3: -, 67.0, 57.1).  The 16-row tiles of 1024 threads (lx = 0) where
 // they are one workgroup on (nearly) every CU (256^3: 93.5 against 100 us; but
 // 256 x 256 x 192 71.3 against 67.3, 512 x 512 x 128 218 against 208, and 39-60
-// us on the grids up to 128^3 above).  Variable coefficients: 2 planes up to
-// 128 tiles, 4 up to 640, 8 up to 2560 (64^3: 13.5, 15.8, 20.9 us; 128^3: 28.9,
-// 26.7, 26.8; 200^3 with 8, 16: 99.8, 108), then 16 where a row has idle lanes
-// in 64 (288 x 288 x 200: 204 against 246 us) and the 8-row tiles elsewhere.
+// us on the grids up to 128^3 above).  Variable coefficients, whose registers
+// let two workgroups on a CU: the planes (2, 4, 8 or 16) for which rounds of
+// 512 tiles x (planes + 3 of start-up) is least (64^3 13.8 us with 2, 15.9 with 4;
+// 128^3 27.0 with 4, 27.1 with 8, 34.8 with 16; 160^3 55, 50.7 and 45.9; 200^3 103,
+// 97, 107; 400 x 100 x 100 50, 52, 48); 256-wide tiles of 8 rows and 16 planes,
+// 512 threads: 34.0, 39.3, 46.0, 107, 50.7 us.
 static CgShape tile_shape(const GridK& g, bool var) {
     CgShape sh{64, 16};
     const int64_t nx4 = ceil_div(g.nx, 4);
@@ -1220,10 +1219,13 @@ static CgShape tile_shape(const GridK& g, bool var) {
         const int64_t cost = ceil_div(nx4, lx) * (lx + 12);
         if (cost < best) best = cost, sh.lx = lx;
     }
-    const int64_t t4 = ceil_div(nx4, sh.lx) * ceil_div(g.ny, 256 / sh.lx) * ceil_div(g.nz, 4);
+    const int64_t cols = ceil_div(nx4, sh.lx) * ceil_div(g.ny, 256 / sh.lx), t4 = cols * ceil_div(g.nz, 4);
     if (var) {
-        sh.zd = t4 <= 128 ? 2 : t4 <= 640 ? 4 : t4 <= 2560 ? 8 : 16;
-        if (sh.lx == 64 && t4 > 2560) sh.lx = 0;
+        best = INT64_MAX;
+        for (int zd = 16; zd >= 2; zd /= 2) {
+            const int64_t cost = ceil_div(cols * ceil_div(g.nz, zd), 512) * (zd + 3);
+            if (cost < best) best = cost, sh.zd = zd;
+        }
         return sh;
     }
     sh.zd = t4 <= 400 ? 2 : t4 <= 1024 ? 4 : 16;
@@ -1235,11 +1237,21 @@ static CgShape tile_shape(const GridK& g, bool var) {
 static CgShape cg_shape(const GridK& gk, int fast) {
     return fast && !gk.block ? tile_shape(gk, fast == kFastVar) : CgShape{0, 0};
 }
-// blocks of the first-half launch of a tiled iteration
-static int fast_blocks(const GridK& g, int fast, const CgShape& sh) {
-    if (!sh.lx) return stencil4_blocks(g, fast == kFastVar ? kTYv : kTYc);
+// Blocks of a tiled launch of the shape, at most cap (a multiple of 8): as many
+// rounds as needed, each block the same number of tiles or one fewer, and a
+// multiple of 8, so that xcd_tile gives every XCD its consecutive eighth.
+// (With cap blocks and the tiles beyond dealt from the first on, one or two
+// XCDs did all of the second round: 320^3 variable, 2,400 tiles, 504 us an
+// iteration, 426 so; 200^3, 1,250 tiles of the second half in 1,024 blocks, 57.9,
+// 53.2 so.)
+static int tiled_blocks(const GridK& g, const CgShape& sh, int cap) {
     const int64_t nt = ceil_div(g.nx, 4 * sh.lx) * ceil_div(g.ny, 256 / sh.lx) * ceil_div(g.nz, sh.zd);
-    return (int)std::min<int64_t>(nt, 2048);
+    const int64_t per_round = ceil_div(nt, ceil_div(nt, cap));
+    return (int)(ceil_div(per_round, 8) * 8);
+}
+// blocks of the first-half launch of a tiled iteration
+static int fast_blocks(const GridK& g, const CgShape& sh) {
+    return sh.lx ? tiled_blocks(g, sh, 2048) : stencil4_blocks(g, kTYc);
 }
 
 static_assert(kCgPartDoubles == (size_t)kRedBlocks * 16, "partials region");
@@ -1363,8 +1375,7 @@ static nnx_status cg_bind(nnx_ctx* c, const GridK& gk, int precond, const float*
     h->gp = h->pad ? padded_grid(gk) : gk;
     h->xp = m.xp;
     h->sh = cg_shape(h->gp, h->fast);
-    if (h->pad && h->fast == kFastVar && !h->sh.lx) h->sh = CgShape{64, 16};
-    h->nb4 = fast_blocks(h->gp, h->fast, h->sh);
+    h->nb4 = fast_blocks(h->gp, h->sh);
     double* P = m.part;
     h->d.npq = h->fast ? h->nb4 : kRedBlocks;
     h->d.r = m.r;
@@ -1430,9 +1441,6 @@ static void cg_iter_launch(nnx_ctx* c, CgHost& h, int k, float* x, int xzero = 0
         if (h.pad)
             NNX_BY_LX(sh.lx, k_stencil7x4<2, 3, true, 4, false, LX, true, true>
                       <<<nb4, 256, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, sh.zd));
-        else if (sh.lx == 0)
-            k_stencil7x4<2, kPFv, true, kTYv>
-                <<<nb4, 64 * kTYv, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, 0);
         else
             NNX_BY_LX(sh.lx, k_stencil7x4<2, 3, true, 4, false, LX, true>
                       <<<nb4, 256, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, sh.zd));
@@ -1451,8 +1459,8 @@ static void cg_iter_launch(nnx_ctx* c, CgHost& h, int k, float* x, int xzero = 0
         NNX_BY_LX(sh.lx, k_stencil7x4<2, 3, false, 4, false, LX, true>
                   <<<nb4, 256, 0, c->stream>>>(gk, h.d, k, nullptr, pold, pnew, x, xzero, sh.zd));
         NNX_BY_LX(sh.lx, k_stencil7x4<3, 3, false, 4, false, LX, true>
-                  <<<std::min(nb4, kRedBlocks), 256, 0, c->stream>>>(gk, h.d, k, pnew, nullptr, nullptr, nullptr, 0,
-                                                                     sh.zd));
+                  <<<tiled_blocks(gk, sh, kRedBlocks), 256, 0, c->stream>>>(gk, h.d, k, pnew, nullptr, nullptr, nullptr,
+                                                                            0, sh.zd));
         return;
     }
     if (fast) {
@@ -1493,7 +1501,7 @@ static void res64_launch(nnx_ctx* c, const CgHost& h, const double* x, const dou
         return;
     }
     const CgShape sh = h.sh.lx ? h.sh : CgShape{64, 16};
-    const int nb = std::min(fast_blocks(gp, kFastConst, sh), kRedBlocks);
+    const int nb = tiled_blocks(gp, sh, kRedBlocks);
     if (gp.nx != gp.nxr || ((uintptr_t)x | (uintptr_t)b | (uintptr_t)r64) % 16 != 0)
         NNX_BY_LX(sh.lx, k_res64x4<OUT, false, 4, LX, true, true>
                   <<<nb, 256, 0, c->stream>>>(gp, x, b, h.d, prr, pfl, r64, sh.zd));
@@ -1993,8 +2001,8 @@ nnx_status nnx_stencil_apply(nnx_ctx* c, const nnx_grid* g, const float* x, floa
                 <<<stencil4_blocks(gk, kTYa), 64 * kTYa, 0, c->stream>>>(gk, none, 0, x, nullptr, nullptr, y, 0, 0);
         else if (const CgShape sh = tile_shape(gk, false); sh.lx && sh.zd <= 4)
             NNX_BY_LX(sh.lx, k_stencil7x4<0, 3, false, 4, false, LX, true>
-                      <<<fast_blocks(gk, kFastConst, sh), 256, 0, c->stream>>>(gk, none, 0, x, nullptr, nullptr, y, 0,
-                                                                                sh.zd));
+                      <<<tiled_blocks(gk, sh, 2048), 256, 0, c->stream>>>(gk, none, 0, x, nullptr, nullptr, y, 0,
+                                                                           sh.zd));
         else
             k_stencil7x4<0, kPFa, false, kTYa>
                 <<<stencil4_blocks(gk, kTYa), 64 * kTYa, 0, c->stream>>>(gk, none, 0, x, nullptr, nullptr, y, 0, 0);

@@ -108,6 +108,9 @@ def _operator(ctx, nx, ny, nz, var, seed=6):
 # rows of 8, 16, 32 and 64 lanes with remainders in x, y and z; 2, 4 and 16
 # planes a tile (variable coefficients: 2, 4, 8 and 16)
 SHAPES = [(4, 3, 2), (20, 33, 7), (60, 50, 41), (100, 131, 22), (128, 130, 66), (152, 90, 97), (200, 120, 151)]
+# more tiles than blocks: the first half's 2048 (variable coefficients), the
+# second half's and the residual's 1024 (constant), in place and in padded rows
+SHAPES += [(4, 1000, 600), (13, 1000, 600)]
 # rows of every residue mod 4 (padded working rows), from the shortest padded
 # row and one below it on, in every tile width
 SHAPES += [(11, 9, 7), (12, 9, 5), (13, 9, 5), (31, 33, 8), (67, 40, 33), (102, 64, 21), (150, 131, 30), (201, 120, 150)]
