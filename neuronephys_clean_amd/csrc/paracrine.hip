@@ -1281,7 +1281,10 @@ static size_t cg_bytes(const GridK& gk, int precond, bool pad) {
 // the 4-voxel groups: the generic kernels (150 x 131 x 97: 45 us per
 // iteration against 25 in padded rows).  A grid that only fits
 // nnx_cg_solve_async_noalloc's array unpadded stays generic in every solver,
-// so that the solvers' results agree.
+// so that the solvers' results agree: with variable coefficients and Jacobi the
+// ragged cubes from 129^3 to 135^3 (and 128^3 and 132^3 off the 16-byte grid),
+// with constant ones 146^3 (130^3 variable 56 us per iteration, 28 at 127^3 and
+// 47 at 137^3; 146^3 constant 65, 41 at 145^3 and 147^3).
 static int cg_fast(const GridK& gk, int precond, const float* x, bool* pad) {
     *pad = false;
     if (gk.kind == 2 || gk.block % 4 != 0) return 0;

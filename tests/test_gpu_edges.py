@@ -144,11 +144,13 @@ def test_tiled_solve_shapes(ctx, dims, var):
 
 
 @pytest.mark.parametrize("dims,var,shift", [((33, 21, 14), False, 0), ((33, 21, 14), True, 0), ((34, 21, 14), True, 0),
-                                            ((35, 20, 9), False, 1), ((36, 20, 9), False, 1), ((36, 20, 9), True, 1)])
+                                            ((35, 20, 9), False, 1), ((36, 20, 9), False, 1), ((36, 20, 9), True, 1),
+                                            ((130, 131, 130), True, 0), ((147, 146, 146), False, 0)])
 def test_padded_solvers_agree(ctx, dims, var, shift):
     """nnx_cg_solve, nnx_cg_solve_async and its allocation-free form on rows
     that are no multiple of 4 voxels, and on vectors off the 16-byte grid
-    (shift): the same bits, from zero and from a guess, and nothing written
+    (shift), the last two grids of the sizes that the allocation-free form's
+    array holds unpadded only (generic kernels in all three): the same bits, from zero and from a guess, and nothing written
     beside x."""
     nx, ny, nz = dims
     say("padded", dims, var, shift)
