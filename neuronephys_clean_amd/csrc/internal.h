@@ -166,8 +166,8 @@ nnx_status check_hebbian_plan(nnx_ctx* c, const nnx_step_plan* p);
 
 // Device memory of one CG working set (paracrine.hip): four n-vectors (r,
 // p ping-pong, q), the Jacobi inverse diagonal (n floats, variable
-// coefficients with Jacobi only), 64 scalars, 64 flags and the reduction
-// partials (kCgPartDoubles).
+// coefficients with Jacobi only), 32 scalars with 64 flags behind them and the
+// reduction partials (kCgPartDoubles).
 struct CgMem {
     float *r, *pa, *pb, *q, *dinv;
     float* xp;  // the iterate in padded rows (null: the caller's x is used)
@@ -176,6 +176,7 @@ struct CgMem {
     double* part;
 };
 constexpr size_t kCgPartDoubles = (size_t)1024 * 16;
+constexpr int kCgFlagsAt = 32;  // doubles from sc to fl
 // bytes of a working set for a solve of g into x (256-byte aligned pieces)
 // and its layout inside `base` (256-byte aligned, cg_mem_bytes long)
 size_t cg_mem_bytes(const nnx_grid* g, int precond, const float* x);

@@ -1315,9 +1315,8 @@ CgMem cg_mem_carve(void* base, const nnx_grid* g, int precond, const float* x) {
     m.part = (double*)p;
     p += align256(kCgPartDoubles * 8);
     m.sc = (double*)p;
-    p += 512;
-    m.fl = (int32_t*)p;
-    p += 512;
+    m.fl = (int32_t*)(m.sc + kCgFlagsAt);
+    p += 1024;
     m.r = (float*)p, p += vec;
     m.pa = (float*)p, p += vec;
     m.pb = (float*)p, p += vec;
@@ -1342,13 +1341,12 @@ static nnx_status cg_mem_scratch(nnx_ctx* c, const char* prefix, const GridK& gk
     const GridK gp = pad ? padded_grid(gk) : gk;
     const int64_t n = (int64_t)gp.nx * gp.ny * gp.nz;
     char nm[64];
-    void* p[8] = {};
-    const char* names[] = {"r", "pa", "pb", "q", "sc", "fl", "part"};
-    const size_t bytes[] = {(size_t)n * 4, (size_t)n * 4, (size_t)n * 4, (size_t)n * 4, 64 * 8, 64 * 4,
-                            kCgPartDoubles * 8};
-    for (int i = 0; i < 7; ++i) {
+    void* p[6] = {};
+    const char* names[] = {"r", "pa", "pb", "q", "sc", "part"};
+    const size_t bytes[] = {(size_t)n * 4, (size_t)n * 4, (size_t)n * 4, (size_t)n * 4, 64 * 8, kCgPartDoubles * 8};
+    for (int i = 0; i < 6; ++i) {
         std::snprintf(nm, sizeof nm, "%s_%s", prefix, names[i]);
-        NNX_TRY(scratch(c, nm, bytes[i], i == 4 || i == 5, &p[i]));
+        NNX_TRY(scratch(c, nm, bytes[i], i == 4, &p[i]));
     }
     m->dinv = nullptr;
     if (cg_needs_dinv(gk, precond)) {
@@ -1358,7 +1356,7 @@ static nnx_status cg_mem_scratch(nnx_ctx* c, const char* prefix, const GridK& gk
         m->dinv = (float*)dvp;
     }
     m->r = (float*)p[0], m->pa = (float*)p[1], m->pb = (float*)p[2], m->q = (float*)p[3];
-    m->sc = (double*)p[4], m->fl = (int32_t*)p[5], m->part = (double*)p[6];
+    m->sc = (double*)p[4], m->fl = (int32_t*)(m->sc + kCgFlagsAt), m->part = (double*)p[5];
     m->xp = pad ? m->q : nullptr;
     if (gk.kind == 1 && ((pad && xp != kXpNone) || (xp == kXpAnyX && gk.nx % 4 == 0 && gk.nx >= 12))) {
         std::snprintf(nm, sizeof nm, "%s_xp", prefix);
@@ -1417,12 +1415,13 @@ static nnx_status cg_buffers(nnx_ctx* c, const GridK& gk, int precond, const flo
     return cg_bind(c, gk, precond, x, m, h);
 }
 
+// (the flags lie behind the scalars: one copy)
 static nnx_status cg_readback(nnx_ctx* c, CgHost& h, int32_t* fl, double* sc) {
-    NNX_HIP(c, hipMemcpyAsync(c->pinned, h.d.fl, 4 * FL_N, hipMemcpyDeviceToHost, c->stream));
-    NNX_HIP(c, hipMemcpyAsync((char*)c->pinned + 64, h.d.sc, 8 * SC_N, hipMemcpyDeviceToHost, c->stream));
+    const size_t off = (const char*)h.d.fl - (const char*)h.d.sc;
+    NNX_HIP(c, hipMemcpyAsync(c->pinned, h.d.sc, off + 4 * FL_N, hipMemcpyDeviceToHost, c->stream));
     NNX_HIP(c, hipStreamSynchronize(c->stream));
-    std::memcpy(fl, c->pinned, 4 * FL_N);
-    std::memcpy(sc, (char*)c->pinned + 64, 8 * SC_N);
+    std::memcpy(sc, c->pinned, 8 * SC_N);
+    std::memcpy(fl, (const char*)c->pinned + off, 4 * FL_N);
     return NNX_OK;
 }
 
