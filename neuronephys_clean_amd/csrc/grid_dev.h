@@ -134,8 +134,9 @@ template <class F> __device__ __forceinline__ void for_rows(int nx, int ny, int 
 
 // The same flat over the grid, for any shape: for_rows leaves lanes idle on
 // rows shorter than a wavefront and wavefronts idle on grids of few long rows
-// (a pass of 1,000,000 x 1 x 1 in one wavefront: 1.1 ms; 3 us flat).  Two 32-bit
-// divisions a voxel (fewer than 2^32 of them, rows padded to four included).
+// (ten CG iterations and the FP64 residual on 1,000,000 x 1 x 1: 12.0 ms with the
+// residual in one wavefront, 0.44 flat).  Two 32-bit divisions a voxel (fewer
+// than 2^32 of them, rows padded to four included).
 template <class F> __device__ __forceinline__ void for_voxels(int nx, int ny, int nz, F&& f) {
     const int64_t n = (int64_t)nx * ny * nz, stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t id = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; id < n; id += stride) {
