@@ -1535,7 +1535,7 @@ static void cg_init_launch(nnx_ctx* c, const GridK& gk, CgHost& h, const float* 
 
 // The iterations after an init: check_every at a time, then one status
 // kernel and a read-back.  `started`: the start cannot meet the tolerance, so
-// the first batch goes out without a read-back (12 us) of the init; otherwise
+// the first batch goes out without a read-back (10 us) of the init; otherwise
 // the init is read first - check_every iterations past the end are two
 // launches each, 7.5 ms for 1000 of them.
 static nnx_status cg_loop(nnx_ctx* c, CgHost& h, float* x, int maxit, int check_every, int xzero, bool started,

@@ -231,6 +231,8 @@ def test_working_memory(call, vectors):
     q and the inverse diagonal; a refinement's FP64 residual (two) and
     correction; flexible CG's seven and the residual's four; the capturable
     solve's vector for an unaligned x.  Reductions and state: under 4 MiB."""
+    import gc
+    gc.collect()  # (nothing of an earlier test is freed in between)
     ctx = _lib.Context(0)
     n = 128 ** 3
     g, og, keep = _operator(ctx, 128, 128, 128, True)
