@@ -1081,14 +1081,14 @@ __global__ __launch_bounds__(256) void k_cg_init_pad(GridK g, int px, CgDev d, c
     put_partial<2>(vu, d.pu0);
 }
 // x = xp + the deferred alpha_k p_k of the last executed iteration (without
-// one: x = xp); acc: acc += scale times that instead (nothing without one);
-// xzero as in k_cg_finish
+// one: x = xp, nothing to do where x is the guess xp was copied from); acc: acc
+// += scale times that instead (nothing without one); xzero as in k_cg_finish
 __global__ __launch_bounds__(256) void k_cg_finish_pad(GridK g, CgDev d, const float* __restrict__ pa,
                                                        const float* __restrict__ pb, const float* __restrict__ xp,
                                                        float* __restrict__ x, int xzero, double* __restrict__ acc,
-                                                       double scale) {
+                                                       double scale, int guess) {
     const bool pend = d.fl[FL_XPEND] != 0;
-    if (!pend && acc) return;
+    if (!pend && (acc || guess)) return;
     const int k = d.fl[FL_ITERS] - 1;
     const bool read_x = !(xzero && k == 0);
     const float alpha = pend ? (float)d.sc[SC_ALK + (k & 1)] : 0.0f;
@@ -1488,11 +1488,12 @@ static void cg_iter_launch(nnx_ctx* c, CgHost& h, int k, float* x, int xzero = 0
 }
 
 // the pending x update of the fast path (nothing otherwise; padded rows: the
-// iterate into x); acc: the iterate times scale added to acc instead
+// iterate into x, which holds the solve's guess if `guess`); acc: the iterate
+// times scale added to acc instead
 static void cg_finish_launch(nnx_ctx* c, CgHost& h, float* x, int xzero = 0, double* acc = nullptr,
-                             double scale = 1.0) {
+                             double scale = 1.0, int guess = 0) {
     if (h.pad)
-        k_cg_finish_pad<<<kRedBlocks, 256, 0, c->stream>>>(h.gp, h.d, h.pa, h.pb, h.xp, x, xzero, acc, scale);
+        k_cg_finish_pad<<<kRedBlocks, 256, 0, c->stream>>>(h.gp, h.d, h.pa, h.pb, h.xp, x, xzero, acc, scale, guess);
     else
         k_cg_finish<<<flat_blocks(h.n() / 4), 256, 0, c->stream>>>(h.n(), h.d, h.pa, h.pb, x, xzero, acc, scale);
 }
@@ -1565,7 +1566,7 @@ static nnx_status cg_run(nnx_ctx* c, const GridK& gk, CgHost& h, const float* b,
     double sc[SC_N];
     NNX_TRY(cg_loop(c, h, x, maxit, check_every, 0, false, fl, sc));
     if (initdone) *initdone = fl[FL_INITDONE];
-    cg_finish_launch(c, h, x);
+    cg_finish_launch(c, h, x, 0, nullptr, 1.0, use_x0);
     NNX_LAUNCHED(c);
     if (res) {
         res->iters = fl[FL_ITERS];
@@ -1623,7 +1624,7 @@ static void cg_enqueue_fixed(nnx_ctx* c, const GridK& gk, CgHost& h, const float
                              double tol, int maxit) {
     cg_init_launch(c, gk, h, b, x, use_x0, tol, 0, maxit);
     for (int k = 0; k < maxit; ++k) cg_iter_launch(c, h, k, x);
-    cg_finish_launch(c, h, x);
+    cg_finish_launch(c, h, x, 0, nullptr, 1.0, use_x0);
 }
 
 // The paracrine solve of a timestep (nnx_paracrine): rhs, then max_outer
