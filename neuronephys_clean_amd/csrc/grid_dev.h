@@ -13,8 +13,8 @@ namespace nnx {
 struct GridK {
     int32_t nx, ny, nz, kind;  // kind: 0 const 7-pt, 1 variable 7-pt, 2 27-pt
     int32_t block;             // kind 0: Dirichlet faces every `block` voxels (0: none)
-    int32_t nxr;               // voxels of a row that belong to the grid (< nx: padded rows)
     float c, diag, a0, w;      // fp32 constants (cast once on the host)
+    int32_t nxr;               // voxels of a row that belong to the grid (< nx: padded rows)
     double cd, diagd, a0d, wd; // fp64 constants
     const float *kx, *ky, *kz;
 };
